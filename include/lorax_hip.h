@@ -342,6 +342,30 @@ int lorax_sgmv_expand_planned(void* y, const void* v, const int64_t* w_ptrs, con
                               int32_t h_out, int64_t y_offset, int64_t y_stride, int64_t layer_idx,
                               int32_t accumulate, const lorax_sgmv_tiles_t* tiles, int32_t dtype, void* stream);
 
+/*
+ * lorax_sgmv_expand_planned for up to 16 problems in ONE launch: the projections of a layer that share their input
+ * (q/k/v, gate/up), for every LoRA rank of the batch.  The reference launches one expand per projection and rank
+ * (lorax_server/utils/layers.py:134-143).  Problems share num_tokens (the rows of every v and y), layer_idx and dtype;
+ * the elements of y they update must be disjoint.  A problem without segments, or with a plan without tiles, is
+ * skipped.  Every problem's result equals lorax_sgmv_expand's, bit for bit.
+ */
+typedef struct lorax_sgmv_expand_problem {
+  void* y;                /* [num_tokens, y_stride]                                  */
+  const void* v;          /* [num_tokens, r]                                         */
+  const int64_t* w_ptrs;  /* [num_segments] device addresses of [L, h_out, r] stacks */
+  const int32_t* s_start; /* [num_segments]                                          */
+  const int32_t* s_end;
+  int32_t num_segments;
+  int32_t r;
+  int32_t h_out;
+  int64_t y_offset;
+  int64_t y_stride;
+  const lorax_sgmv_tiles_t* tiles; /* row-tile plan (LORAX_TILES_EXPAND) or NULL; host struct, read during the call */
+} lorax_sgmv_expand_problem_t;
+
+int lorax_sgmv_expand_multi(const lorax_sgmv_expand_problem_t* problems, int32_t num_problems, int64_t num_tokens,
+                            int64_t layer_idx, int32_t accumulate, int32_t dtype, void* stream);
+
 /* Bytes of grouped-GEMM argument scratch for `num_problems` segments.  Replaces
  * sgmv_tmp_size (sgmv/sgmv_cutlass.cuh:54-58): 3 pointers + 3 int64 + one
  * 3 x int32 problem size per segment = 60 * num_problems. */

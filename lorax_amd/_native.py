@@ -83,6 +83,14 @@ class SgmvTiles(ctypes.Structure):
     _fields_ = [("tiles", _c.c_void_p), ("num_tiles", _c.c_int32), ("tile_rows", _c.c_int32)]
 
 
+class SgmvExpandProblem(ctypes.Structure):
+    """lorax_sgmv_expand_problem_t of include/lorax_hip.h."""
+
+    _fields_ = [("y", _c.c_void_p), ("v", _c.c_void_p), ("w_ptrs", _c.c_void_p), ("s_start", _c.c_void_p),
+                ("s_end", _c.c_void_p), ("num_segments", _c.c_int32), ("r", _c.c_int32), ("h_out", _c.c_int32),
+                ("y_offset", _c.c_int64), ("y_stride", _c.c_int64), ("tiles", _c.POINTER(SgmvTiles))]
+
+
 TILES_SHRINK, TILES_EXPAND = 0, 1
 
 
@@ -148,6 +156,10 @@ _SIGNATURES = {
         _c.c_int,
         [_c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32,
          _c.c_int32, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int32, _c.POINTER(SgmvTiles), _c.c_int32, _c.c_void_p],
+    ),
+    "lorax_sgmv_expand_multi": (
+        _c.c_int,
+        [_c.POINTER(SgmvExpandProblem), _c.c_int32, _c.c_int64, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_void_p],
     ),
     "lorax_sgmv_plan_tiles": (
         _c.c_int,
@@ -477,6 +489,36 @@ def sgmv_expand(y, x, w_ptr, s_start, s_end, tmp, layer_idx, y_offset=0, y_slice
             1 if accumulate else 0, tmp.data_ptr(),
             tmp.numel() * tmp.element_size(), _dtype_code(x), _stream(x),
         )
+    if rc != 0:
+        _raise_last(rc)
+
+
+MAX_SGMV_EXPAND_PROBLEMS = 16
+
+
+def sgmv_expand_multi(problems, layer_idx, accumulate: bool = True) -> None:
+    """lorax_sgmv_expand_multi: up to 16 expands over transposed stacks in one launch.  `problems` is a list of tuples
+    (y, v, w_ptr, s_start, s_end, y_offset, y_slice_size, tiles) of one row count, dtype and device whose elements of y
+    are disjoint; ranks (v's width) may differ, tiles is a row-tile plan or None."""
+    if not 1 <= len(problems) <= MAX_SGMV_EXPAND_PROBLEMS:
+        raise RuntimeError(f"between 1 and {MAX_SGMV_EXPAND_PROBLEMS} problems per launch, got {len(problems)}")
+    arr = (SgmvExpandProblem * len(problems))()
+    v0 = problems[0][1]
+    plans = []  # keeps the host structs alive until the call has read them
+    for i, (y, v, w_ptr, s_start, s_end, y_offset, y_slice_size, tiles) in enumerate(problems):
+        _check_sgmv(y, v, w_ptr, s_start, s_end, s_start)
+        if v.size(0) != v0.size(0) or v.dtype != v0.dtype or v.device != v0.device:
+            raise RuntimeError("all problems of one launch must have inputs of one row count, dtype and device")
+        plan = None
+        if tiles is not None:
+            plans.append(tiles.c_struct(v.device))
+            plan = ctypes.pointer(plans[-1])
+        h_out = y.size(1) if y_slice_size is None else int(y_slice_size)
+        arr[i] = SgmvExpandProblem(y.data_ptr(), v.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(),
+                                   s_start.size(0), v.size(1), h_out, int(y_offset), y.size(1), plan)
+    with torch.cuda.device(v0.device):
+        rc = lib().lorax_sgmv_expand_multi(arr, len(problems), v0.size(0), int(layer_idx), 1 if accumulate else 0,
+                                           _dtype_code(v0), _stream(v0))
     if rc != 0:
         _raise_last(rc)
 

@@ -86,7 +86,7 @@ const Tuning& tuning() {
   static const Tuning t = {};
 #else
   static const Tuning t = {env_int("LORAX_BGMV_LORA_BLOCKS"), env_int("LORAX_BGMV_SHRINK_ROWS"), env_int("LORAX_SHRINK_KSPLIT"),
-                           env_int("LORAX_SHRINK_MB"), env_int("LORAX_SHRINK_WAVES"), env_int("LORAX_EXPAND_ROWS"),
+                           env_int("LORAX_SHRINK_MB"), env_int("LORAX_SHRINK_WAVES"), env_int("LORAX_EXPAND_ROWS"), env_int("LORAX_EXPAND_SUB"),
                            env_int("LORAX_SHRINK_NO_ROTATE"), env_int("LORAX_SHRINK_LDS"), env_int("LORAX_SHRINK_LDS_KB"), env_int("LORAX_BGMV_EXPAND_COLS"), env_int("LORAX_EXPAND_PANELS"), env_int("LORAX_BGMV_NO_RUNS"), env_int("LORAX_BGMV_NO_BALANCE"), env_int("LORAX_SHRINK_ROWS_MAX"), env_int("LORAX_SHRINK_ROWS"), env_int("LORAX_BGMV_SCALAR_Y")};
 #endif
   return t;
@@ -248,22 +248,12 @@ int sgmv_shrink_checked(void* v, const void* x, const int64_t* w_ptrs, const int
   return LORAX_OK;
 }
 
-// Shape checks and launch shared by lorax_sgmv_expand and lorax_sgmv_expand_planned.
-int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start, const int32_t* s_end,
-                        int32_t num_segments, int64_t num_tokens, int32_t r, int32_t h_out, int32_t b_layout,
-                        int64_t y_offset, int64_t y_stride, int64_t layer_idx, int32_t accumulate,
-                        const lorax_sgmv_tiles_t* tiles, int32_t dtype, void* stream) {
-  if (accumulate != 0 && accumulate != 1)
-    return fail(LORAX_EINVAL, "accumulate=%d (0 = overwrite, 1 = add)", accumulate);
-  if (b_layout != LORAX_B_RH && b_layout != LORAX_B_HR) return fail(LORAX_EINVAL, "b_layout=%d", b_layout);
-  if (num_segments < 0 || num_tokens < 0)
-    return fail(LORAX_EINVAL, "negative size (num_segments=%d num_tokens=%lld)", num_segments,
-                (long long)num_tokens);
-  if (num_segments == 0 || num_tokens == 0) return LORAX_OK;
+// Shape checks of one expand problem (both B layouts).
+int check_expand(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start, const int32_t* s_end, int64_t num_tokens,
+                 int32_t r, int32_t h_out, int64_t y_offset, int64_t y_stride, int32_t dtype) {
   if (int rc = check_common(y, v, w_ptrs, dtype)) return rc;
   if (s_start == nullptr || s_end == nullptr)
     return fail(LORAX_EINVAL, "null pointer argument (s_start=%p s_end=%p)", s_start, s_end);
-  if (layer_idx < 0) return fail(LORAX_EINVAL, "layer_idx=%lld is negative", (long long)layer_idx);
   if (r < 8 || r > kMaxRank || r % 8 != 0 || h_out <= 0 || h_out % 8 != 0 ||
       num_tokens > INT32_MAX / 2)
     return fail(LORAX_ENOKERNEL, "No suitable kernel. dtype=%d d_in=%d d_out=%d", dtype, r, h_out);
@@ -272,6 +262,61 @@ int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int
                 (long long)y_offset, (long long)y_stride, h_out);
   if (y_stride >= (1ll << 24))
     return fail(LORAX_EINVAL, "y_stride=%lld: rows of y hold fewer than 2^24 elements", (long long)y_stride);
+  return LORAX_OK;
+}
+
+// Expand problems over the transposed stacks in one launch.
+int expand_batch(const lorax_sgmv_expand_problem_t* problems, int32_t count, int64_t num_tokens, int64_t layer_idx,
+                 int32_t accumulate, int32_t dtype, void* stream) {
+  if (accumulate != 0 && accumulate != 1)
+    return fail(LORAX_EINVAL, "accumulate=%d (0 = overwrite, 1 = add)", accumulate);
+  if (count < 0 || count > kMaxExpandProblems)
+    return fail(LORAX_EINVAL, "num_problems=%d (at most %d per launch)", count, kMaxExpandProblems);
+  if (num_tokens < 0) return fail(LORAX_EINVAL, "num_tokens=%lld is negative", (long long)num_tokens);
+  if (count == 0 || num_tokens == 0) return LORAX_OK;
+  if (problems == nullptr) return fail(LORAX_EINVAL, "null pointer argument (problems)");
+  ExpandArgs a{};
+  for (int i = 0; i < count; ++i) {
+    const lorax_sgmv_expand_problem_t& q = problems[i];
+    if (q.num_segments < 0) return fail(LORAX_EINVAL, "negative size (num_segments=%d)", q.num_segments);
+    if (q.num_segments == 0) continue;
+    if (int rc = check_expand(q.y, q.v, q.w_ptrs, q.s_start, q.s_end, num_tokens, q.r, q.h_out, q.y_offset, q.y_stride, dtype))
+      return rc;
+    if (layer_idx < 0) return fail(LORAX_EINVAL, "layer_idx=%lld is negative", (long long)layer_idx);
+    SgmvArgs t{};
+    if (int rc = take_tiles(q.tiles, t)) return rc;
+    if (t.tiles != nullptr && t.num_tiles == 0) continue;  // a plan without tiles: no segment has rows
+    a.p[a.count++] = ExpandProblem{q.y, q.v, q.w_ptrs, q.s_start, q.s_end, q.num_segments, q.r, q.h_out, q.y_offset, q.y_stride,
+                                   t.tiles, t.num_tiles, t.tile_rows};
+  }
+  if (a.count == 0) return LORAX_OK;
+  a.num_tokens = num_tokens;
+  a.layer_idx = layer_idx;
+  a.accumulate = accumulate;
+  a.dtype = dtype;
+  const hipError_t e = launch_sgmv_expand_t(a, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_expand launch failed: %s", hipGetErrorString(e));
+  return LORAX_OK;
+}
+
+// Shape checks and launch shared by lorax_sgmv_expand and lorax_sgmv_expand_planned.
+int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start, const int32_t* s_end,
+                        int32_t num_segments, int64_t num_tokens, int32_t r, int32_t h_out, int32_t b_layout,
+                        int64_t y_offset, int64_t y_stride, int64_t layer_idx, int32_t accumulate,
+                        const lorax_sgmv_tiles_t* tiles, int32_t dtype, void* stream) {
+  if (b_layout == LORAX_B_HR) {
+    const lorax_sgmv_expand_problem_t one{y, v, w_ptrs, s_start, s_end, num_segments, r, h_out, y_offset, y_stride, tiles};
+    return expand_batch(&one, 1, num_tokens, layer_idx, accumulate, dtype, stream);
+  }
+  if (accumulate != 0 && accumulate != 1)
+    return fail(LORAX_EINVAL, "accumulate=%d (0 = overwrite, 1 = add)", accumulate);
+  if (b_layout != LORAX_B_RH) return fail(LORAX_EINVAL, "b_layout=%d", b_layout);
+  if (num_segments < 0 || num_tokens < 0)
+    return fail(LORAX_EINVAL, "negative size (num_segments=%d num_tokens=%lld)", num_segments,
+                (long long)num_tokens);
+  if (num_segments == 0 || num_tokens == 0) return LORAX_OK;
+  if (int rc = check_expand(y, v, w_ptrs, s_start, s_end, num_tokens, r, h_out, y_offset, y_stride, dtype)) return rc;
+  if (layer_idx < 0) return fail(LORAX_EINVAL, "layer_idx=%lld is negative", (long long)layer_idx);
   SgmvArgs a{};
   a.y = y;
   a.x = v;
@@ -288,10 +333,7 @@ int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int
   a.dtype = dtype;
   a.a_layout = b_layout;
   a.accumulate = accumulate;
-  if (int rc = take_tiles(tiles, a)) return rc;
-  if (a.tiles != nullptr && a.num_tiles == 0) return LORAX_OK;  // a plan without tiles: no segment has rows
-  const hipError_t e = b_layout == LORAX_B_HR ? launch_sgmv_expand_t(a, static_cast<hipStream_t>(stream))
-                                              : launch_sgmv_expand(a, static_cast<hipStream_t>(stream));
+  const hipError_t e = launch_sgmv_expand(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_expand launch failed: %s", hipGetErrorString(e));
   return LORAX_OK;
 }
@@ -458,6 +500,11 @@ int lorax_sgmv_expand_planned(void* y, const void* v, const int64_t* w_ptrs, con
                               int32_t accumulate, const lorax_sgmv_tiles_t* tiles, int32_t dtype, void* stream) {
   return sgmv_expand_checked(y, v, w_ptrs, s_start, s_end, num_segments, num_tokens, r, h_out, LORAX_B_HR, y_offset,
                              y_stride, layer_idx, accumulate, tiles, dtype, stream);
+}
+
+int lorax_sgmv_expand_multi(const lorax_sgmv_expand_problem_t* problems, int32_t num_problems, int64_t num_tokens,
+                            int64_t layer_idx, int32_t accumulate, int32_t dtype, void* stream) {
+  return expand_batch(problems, num_problems, num_tokens, layer_idx, accumulate, dtype, stream);
 }
 
 int lorax_bgmv_lora_multi(const lorax_bgmv_problem_t* problems, int32_t num_problems, int64_t num_tokens,

@@ -131,6 +131,33 @@ struct SgmvLoraArgs {
 };
 hipError_t launch_sgmv_lora_rows(const SgmvLoraArgs& a, hipStream_t stream);
 
+// Expand over the transposed stacks ([L, h_out, r]): up to 16 problems per launch - projections and rank groups of one
+// layer - each with its own segments, rank and column window of y.  Their elements of y must be disjoint.
+constexpr int kMaxExpandProblems = 16;
+struct ExpandProblem {
+  void* y;
+  const void* v;          // [num_tokens, r]
+  const int64_t* w_ptrs;  // [num_segments]
+  const int32_t* s_start;
+  const int32_t* s_end;
+  int num_segments;
+  int r;
+  int h_out;
+  int64_t y_offset;
+  int64_t y_stride;
+  const int32_t* tiles;  // optional row-tile plan (lorax_sgmv_tiles_t)
+  int num_tiles;
+  int tile_rows;
+};
+struct ExpandArgs {
+  ExpandProblem p[kMaxExpandProblems];
+  int count;
+  int64_t num_tokens;
+  int64_t layer_idx;
+  int accumulate;
+  int dtype;
+};
+
 // Launch parameters that can be overridden from the environment for tuning runs, read once per process;
 // 0 (unset) = the launcher's heuristic.
 struct Tuning {
@@ -140,11 +167,12 @@ struct Tuning {
   int shrink_mb;         // LORAX_SHRINK_MB: 16-row blocks per row tile of the SGMV shrink (1, 2, 4)
   int shrink_waves;      // LORAX_SHRINK_WAVES: waves per workgroup of the register-operand SGMV shrink
   int expand_rows;       // LORAX_EXPAND_ROWS: rows per tile of the SGMV expand
+  int expand_sub;        // LORAX_EXPAND_SUB: rows per workgroup of the transposed-B expand
   int shrink_no_rotate;  // LORAX_SHRINK_NO_ROTATE: SGMV shrinks whose tiles all walk the hidden dimension from k = 0
   int shrink_lds;  // LORAX_SHRINK_LDS: 1 = always take the LDS-staged shrink where it applies, -1 = never
   int shrink_lds_kb;  // LORAX_SHRINK_LDS_KB: LDS budget of the staged shrink's buffers
   int bgmv_expand_cols;  // LORAX_BGMV_EXPAND_COLS: columns per lane group of the BGMV expand (4, 8, 16)
-  int expand_panels;  // LORAX_EXPAND_PANELS: column panels per wave of the transposed-B expand
+  int expand_panels;  // LORAX_EXPAND_PANELS: column panels per wave of the reference-layout expand
   int bgmv_no_runs;   // LORAX_BGMV_NO_RUNS: number workgroups problem by problem
   int bgmv_no_balance;  // LORAX_BGMV_NO_BALANCE: plain workgroup numbering in the single-launch BGMV
   int shrink_rows_max;  // LORAX_SHRINK_ROWS_MAX: largest token count served by the streaming SGMV shrink (-1 = never)
@@ -160,7 +188,7 @@ hipError_t launch_bgmv(const BgmvArgs& a, hipStream_t stream);
 hipError_t launch_bgmv_lora(const BgmvArgs& a, hipStream_t stream);
 hipError_t launch_sgmv_shrink(const SgmvArgs& a, hipStream_t stream);
 hipError_t launch_sgmv_expand(const SgmvArgs& a, hipStream_t stream);
-hipError_t launch_sgmv_expand_t(const SgmvArgs& a, hipStream_t stream);  // B stacks stored as [L, h_out, r]
+hipError_t launch_sgmv_expand_t(const ExpandArgs& a, hipStream_t stream);  // B stacks stored as [L, h_out, r]
 // LDS-staged shrink (sgmv_shrink_lds.hip): [L, r, h_in] layout, h_in a multiple of 128.
 bool sgmv_shrink_lds_applies(const SgmvArgs& a);
 hipError_t launch_sgmv_shrink_lds(const SgmvArgs& a, hipStream_t stream);

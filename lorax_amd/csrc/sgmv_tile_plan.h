@@ -19,7 +19,6 @@ namespace lorax {
 
 constexpr int kShrinkTileRowsMax = 64;   // the LDS-staged shrink's buffers hold up to four 16-row blocks
 constexpr int kExpandTileRows = 256;     // nominal height of an expand tile
-constexpr int kExpandTileRowsMax = kExpandTileRows + kExpandTileRows / 8 + 16;  // with a merged remainder
 
 struct SegmentSpan {
   int32_t seg, start, end;  // clamped to [0, num_tokens], end > start
@@ -87,7 +86,9 @@ inline int plan_shrink_tiles(const std::vector<SegmentSpan>& segs, std::vector<l
 // Expand tiles: nominally 256 rows; a remainder of at most an eighth of the segment's full tiles is shared out
 // among them instead of becoming a tile of its own (a tile's prologue costs as much as a hundred rows), and the
 // segment's tiles get equal heights in 16-row blocks - the rule of the device-side search (merged_tile_count).
+// Returns the height of the tallest tile (the launcher sizes its grid by it).
 inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<lorax_sgmv_tile_t>& out) {
+  int tallest = 1;
   for (const SegmentSpan& s : segs) {
     const int len = s.end - s.start;
     const int full = len / kExpandTileRows;
@@ -101,9 +102,10 @@ inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<l
       t.row_end = std::min<int32_t>(s.end, s.start + 16 * static_cast<int32_t>(static_cast<int64_t>(i + 1) * blocks / nt));
       t.index = i;
       out.push_back(t);
+      tallest = std::max(tallest, t.row_end - t.row0);
     }
   }
-  return kExpandTileRowsMax;
+  return tallest;
 }
 
 }  // namespace lorax

@@ -88,7 +88,7 @@ class LoraLinear(nn.Module):
         tensor_parallel = self.process_group.size() > 1
         decode_jobs = defaultdict(list)  # (wave, rank) -> [(rank_segments, start, width)]
         stacked_jobs = []  # (lora_a_stack, lora_b_stack, start, width) of projections served by stacked weights
-        prefill_jobs = defaultdict(list)  # (rank, segment tables) -> [(rank_segments, start, width)]
+        prefill_jobs = defaultdict(list)  # (wave, rank, segment tables) -> [(rank_segments, start, width)]
         for name, start, end in slices:
             data = self._lora_data(adapter_data, name)
             if data is None:
@@ -121,7 +121,8 @@ class LoraLinear(nn.Module):
                 # does not take.
                 if rs.lora_a_t_ptr is not None and resident_shrink_applies(r, input.size(1), input.size(0)):
                     if rs.segments_key is not None and rs.lora_b_t_ptr is not None and not tensor_parallel:
-                        prefill_jobs[(r, rs.segments_key)].append((rs, start, end - start))
+                        wave = group_key[1] if isinstance(group_key, tuple) else 0
+                        prefill_jobs[(wave, r, rs.segments_key)].append((rs, start, end - start))
                         continue
                     whole = rs.num_long_segments == rs.segment_starts.numel()  # the plans cover the long segments
                     v = lora_a_sgmv_resident(
@@ -155,11 +156,38 @@ class LoraLinear(nn.Module):
                         result, v, rs.tmp_expand, rs.lora_b_ptr, rs.segment_starts, rs.segment_ends, self.layer_id
                     )
 
-        # Prefill: projections of one rank with the same segment tables (q/k/v, gate/up of adapters that target
-        # them all) shrink together, as many per launch as fit a summed rank of 128 - x is read once per
-        # launch; the reference issues one shrink per projection (utils/layers.py:121-133).
-        for (r, _), group in prefill_jobs.items():
-            if _native.sgmv_lora_fits(r, input.size(1), input.size(0), max(width for _, _, width in group)):
+        # (the rank chunks of an adapter of a rank above 128 update the same elements of the result, so each chunk number
+        # goes out on its own)
+        for wave in sorted({wave for wave, _, _ in prefill_jobs}):
+            self._prefill(result, input, [group for key, group in prefill_jobs.items() if key[0] == wave])
+
+        if stacked_jobs:  # the reference calls add_lora once per projection (utils/layers.py:92-104)
+            adapter_data.punica_wrapper.add_lora_slices(
+                result, input, stacked_jobs, 1.0, callback=self.collect_lora_a if tensor_parallel else None
+            )
+
+        # Decode.  When every job of the call has a small A slab (rank 8 or 16, moderate widths), shrink and
+        # expand run in one launch per rank and v never leaves the chip.  Otherwise all rank groups of all
+        # projections go out together: one shrink launch and one expand launch per 16 problems, whatever the
+        # mix of ranks (the reference issues a pair of launches per projection and rank, layers.py:146-164).
+        waves = sorted({wave for wave, _ in decode_jobs})
+        if len(waves) > 1:
+            for wave in waves:
+                self._decode(result, input, {k: v for k, v in decode_jobs.items() if k[0] == wave}, tensor_parallel)
+            return result
+        return self._decode(result, input, decode_jobs, tensor_parallel)
+
+    def _prefill(self, result, input, groups):
+        """The segment launches of forward_layer_types for jobs that touch disjoint elements of `result`: a group is
+        [(rank_segments, start, width)] of the projections of one rank with the same segment tables.  Those shrink
+        together, as many per launch as fit a summed rank of 128 - x is read once per launch; the expands of all
+        projections and ranks are one launch.  (The reference issues a shrink and an expand per projection and rank,
+        utils/layers.py:121-143.)"""
+        rows = input.size(0)
+        expands, short_shrinks, short_expands = [], [], []
+        for group in groups:
+            r = group[0][0].rank
+            if _native.sgmv_lora_fits(r, input.size(1), rows, max(width for _, _, width in group)):
                 # a short batch is bound by launches: shrink and expand of up to four projections in one
                 step = _native.MAX_FUSED_BGMV_PROBLEMS
                 for i in range(0, len(group), step):
@@ -177,57 +205,44 @@ class LoraLinear(nn.Module):
             plans = [rs.short_plan for rs, _, _ in group]
             # (the per-token kernels number rows and plan records with 16 bits; beyond that the segment kernels
             # take the whole tables, which still list every segment)
-            split = (all(p is not None for p in plans) and input.size(0) <= _native.MAX_BGMV_TOKENS
+            split = (all(p is not None for p in plans) and rows <= _native.MAX_BGMV_TOKENS
                      and all(p.size(0) <= _native.MAX_BGMV_TOKENS for p in plans))
             n_long = first.num_long_segments if split else first.segment_starts.numel()
             starts, ends = first.segment_starts[:n_long], first.segment_ends[:n_long]
             # the tables' row-tile plans cover their first num_long_segments entries
             planned = n_long == first.num_long_segments
-            shrink_tiles = first.shrink_tiles if planned else None
-            expand_tiles = first.expand_tiles if planned else None
             # v needs no zero-fill: the shrinks overwrite the rows of their segments and the expands read no others
-            flat = torch.empty((len(group), input.size(0), r), dtype=input.dtype, device=input.device)
-            vs = list(flat.unbind(0))
+            vs = list(torch.empty((len(group), rows, r), dtype=input.dtype, device=input.device).unbind(0))
             step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, MAX_RANK_CUSTOM // r))
             # (no long segment at all: the per-token launches do the whole update)
             for i in range(0, len(group) if n_long > 0 else 0, step):
                 _native.sgmv_shrink_multi(
                     vs[i : i + step], input, [rs.lora_a_t_ptr[:n_long] for rs, _, _ in group[i : i + step]],
-                    starts, ends, get_shrink_scratch(input.device), self.layer_id, 1.0, False, shrink_tiles,
+                    starts, ends, get_shrink_scratch(input.device), self.layer_id, 1.0, False,
+                    first.shrink_tiles if planned else None,
                 )
-            batch = _native.MAX_BGMV_PROBLEMS
-            if split:  # the short rows of every projection of the group in one launch
-                for i in range(0, len(group), batch):
-                    _native.bgmv_multi([(v, input, None, None, 0, None) for v in vs[i : i + batch]], self.layer_id,
-                                       1.0, accumulate=False, plans=plans[i : i + batch])
-            for v, (rs, start, width) in zip(vs, group) if n_long > 0 else ():
-                lora_b_sgmv_cutlass_slice(
-                    result, v, rs.tmp_expand[: get_tmp_expand_size(n_long)], rs.lora_b_t_ptr[:n_long], starts, ends,
-                    self.layer_id, start, width, transposed=True, tiles=expand_tiles,
-                )
-            if split:
-                for i in range(0, len(group), batch):
-                    _native.bgmv_multi(
-                        [(result, v, None, None, start, width)
-                         for v, (_, start, width) in zip(vs[i : i + batch], group[i : i + batch])],
-                        self.layer_id, 1.0, accumulate=True, plans=plans[i : i + batch],
-                    )
-
-        if stacked_jobs:  # the reference calls add_lora once per projection (utils/layers.py:92-104)
-            adapter_data.punica_wrapper.add_lora_slices(
-                result, input, stacked_jobs, 1.0, callback=self.collect_lora_a if tensor_parallel else None
-            )
-
-        # Decode.  When every job of the call has a small A slab (rank 8 or 16, moderate widths), shrink and
-        # expand run in one launch per rank and v never leaves the chip.  Otherwise all rank groups of all
-        # projections go out together: one shrink launch and one expand launch per 16 problems, whatever the
-        # mix of ranks (the reference issues a pair of launches per projection and rank, layers.py:146-164).
-        waves = sorted({wave for wave, _ in decode_jobs})
-        if len(waves) > 1:
-            for wave in waves:
-                self._decode(result, input, {k: v for k, v in decode_jobs.items() if k[0] == wave}, tensor_parallel)
-            return result
-        return self._decode(result, input, decode_jobs, tensor_parallel)
+            for v, plan, (rs, start, width) in zip(vs, plans, group):
+                if n_long > 0:
+                    expands.append((result, v, rs.lora_b_t_ptr[:n_long], starts, ends, start, width,
+                                    first.expand_tiles if planned else None))
+                    tmp_expand = rs.tmp_expand
+                if split:
+                    short_shrinks.append(((v, input, None, None, 0, None), plan))
+                    short_expands.append(((result, v, None, None, start, width), plan))
+        batch = _native.MAX_BGMV_PROBLEMS
+        for i in range(0, len(short_shrinks), batch):
+            chunk = short_shrinks[i : i + batch]
+            _native.bgmv_multi([p for p, _ in chunk], self.layer_id, 1.0, accumulate=False, plans=[p for _, p in chunk])
+        step = _native.MAX_SGMV_EXPAND_PROBLEMS
+        for i in range(0, len(expands) if len(expands) > 1 else 0, step):
+            _native.sgmv_expand_multi(expands[i : i + step], self.layer_id)
+        if len(expands) == 1:
+            y, v, table, starts, ends, start, width, tiles = expands[0]
+            lora_b_sgmv_cutlass_slice(y, v, tmp_expand[: get_tmp_expand_size(starts.numel())], table, starts, ends,
+                                      self.layer_id, start, width, transposed=True, tiles=tiles)
+        for i in range(0, len(short_expands), batch):
+            chunk = short_expands[i : i + batch]
+            _native.bgmv_multi([p for p, _ in chunk], self.layer_id, 1.0, accumulate=True, plans=[p for _, p in chunk])
 
     def _decode(self, result, input, decode_jobs, tensor_parallel):
         """The decode launches of forward_layer_types for jobs that touch disjoint elements of `result`:

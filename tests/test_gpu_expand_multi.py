@@ -1,0 +1,71 @@
+"""lorax_sgmv_expand_multi: several expands of different rank, width and segments in one launch, against one launch
+each (bit for bit: every element of the update is one dot product over r whatever the tiling) and against the oracle
+formula.  The batches are small enough for the launch to cut its row tiles into pieces of 128, 64 or 32 rows."""
+
+import pytest
+import torch
+
+from lorax_amd import _native, sgmv
+from tests.helpers import assert_close, ptr_table, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("parts", [
+    [(8, 8, [1]), (8, 1160, [31, 0, 33])],                          # one row, one short panel; pieces of 32 rows
+    [(64, 4096, [300]), (64, 1024, [300])],                         # a merged remainder: tiles higher than 256 rows
+    [(16, 512, [17, 1]), (24, 640, [65]), (128, 1024, [129, 3]), (72, 8, [5])],  # every body of the mixed launch
+    [(32, 4096, [700, 256, 511]), (16, 14336, [1000])],             # enough workgroups for higher pieces
+])
+def test_expands_of_one_launch_equal_single_launches(dtype, planned, parts):
+    print(f"case dtype={dtype} planned={planned} parts={parts}", flush=True)
+    gen = torch.Generator().manual_seed(sum(r + h for r, h, _ in parts))
+    layer, pos, spans = 1, 1, []
+    for _, _, lens in parts:  # every problem owns rows of its own
+        spans.append([])
+        for n in lens:
+            spans[-1].append((pos, pos + n))
+            pos += n + 1
+    T = pos + 2
+    width = sum(h for _, h, _ in parts) + 16
+    y0 = randn((T, width), 0.5, gen, dtype, DEV)
+    problems, weights, off = [], [], 8
+    for (r, h_out, lens), seg in zip(parts, spans):
+        bt = [randn((2, h_out, r), 0.05, gen, dtype, DEV) for _ in lens]
+        v = randn((T, r), 1.0, gen, dtype, DEV)
+        s, e = [a for a, _ in seg], [b for _, b in seg]
+        tiles = None
+        if planned:
+            records, rows = _native.plan_tiles(s, e, T, _native.TILES_EXPAND)
+            tiles = _native.TilePlan(torch.from_numpy(records.copy()).to(DEV), rows)
+        problems.append([None, v, ptr_table(bt, DEV), torch.tensor(s, dtype=torch.int32, device=DEV),
+                         torch.tensor(e, dtype=torch.int32, device=DEV), off, h_out, tiles])
+        weights.append(bt)
+        off += h_out
+    for accumulate in (True, False):
+        y_a, y_b = y0.clone(), y0.clone()
+        _native.sgmv_expand_multi([(y_a, *p[1:]) for p in problems], layer, accumulate)
+        for _, v, w, s, e, o, h, tiles in problems:
+            tmp = sgmv.get_tmp_tensor_for_size(s.numel(), torch.device(DEV))
+            _native.sgmv_expand(y_b, v, w, s, e, tmp, layer, o, h, True, accumulate, tiles)
+        torch.cuda.synchronize()
+        assert torch.equal(y_a, y_b), f"accumulate={accumulate}"
+    want = y0.cpu().clone()
+    for p, bt, seg in zip(problems, weights, spans):
+        for w, (s, e) in zip(bt, seg):
+            want[s:e, p[5]:p[5] + p[6]] = p[1].cpu()[s:e] @ w[layer].cpu().t()  # the last call overwrote
+    assert_close(y_a, want, "expands of one launch")
+
+
+def test_expand_multi_checks_its_problems():
+    y = torch.zeros((4, 64), dtype=torch.bfloat16, device=DEV)
+    v = torch.zeros((4, 16), dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(1, dtype=torch.int64, device=DEV)
+    s = torch.zeros(1, dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="y_offset=8"):
+        _native.sgmv_expand_multi([(y, v, w, s, s, 8, 64, None)], 0)
+    with pytest.raises(RuntimeError, match="between 1 and 16 problems"):
+        _native.sgmv_expand_multi([(y, v, w, s, s, 0, 64, None)] * 17, 0)
