@@ -36,6 +36,7 @@ extern "C" {
 #define LORAX_ELAUNCH 3    /* the HIP runtime refused the launch                            */
 #define LORAX_ETMPSIZE 4   /* tmp buffer size does not match the reference's contract       */
 #define LORAX_ESPACE 5     /* an output buffer of the caller is too small; sizes are reported */
+#define LORAX_EROUTE 6     /* lorax_layer_update: these tables need the single entry points       */
 
 #define LORAX_F16 0
 #define LORAX_BF16 1
@@ -426,6 +427,9 @@ typedef struct lorax_table_group {
   int32_t shrink_tile_rows;
   int32_t num_expand_tiles;
   int32_t expand_tile_rows;
+  int32_t segments_id;  /* use_sgmv = 1: equal for groups whose segment bounds hold the same values
+                           (their shrinks can share one pass over x); else -1                     */
+  int32_t reserved;
 } lorax_table_group_t;
 
 int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
@@ -434,6 +438,31 @@ int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
                              int64_t* segment_owners, int32_t* num_segments, void* packed,
                              int64_t packed_capacity, int64_t* packed_bytes, lorax_table_group_t* groups,
                              int32_t group_capacity, int32_t* num_groups);
+
+/*
+ * The whole LoRA update of the projections of one decoder layer that share their input (q/k/v, gate/up, one alone),
+ * from the tables of lorax_build_batch_tables: picks the launches - decode: one shrink+expand launch per rank, or one
+ * shrink and one expand launch per 16 projections and ranks; prefill: shared shrinks, one expand launch per 16
+ * projections and ranks, per-token launches for segments of a few rows - and issues them.  The reference spends one
+ * Python call per launch on this (lorax_server/utils/layers.py:107-167), which takes longer than the launch runs.
+ *   groups, num_groups  host: the builder's group records; tables: device copy of its packed buffer
+ *   slices              host: layer type (index into entry_counts), width and first column in y of each projection
+ *   v, v_bytes          device workspace, num_tokens * (sum of the ranks of the slices' groups) elements
+ *   tmp, tmp_bytes      device, LORAX_SHRINK_TMP_BYTES (read by prefill tables only)
+ *   device              the GPU the pointers live on; made current for the call
+ * Returns LORAX_EROUTE, before anything is launched, for tables that need a path of the caller's own (ranks that are
+ * no multiple of 8, shapes that only the reference's prefill layouts serve).
+ */
+typedef struct lorax_layer_slice {
+  int32_t layer_type;
+  int32_t width;
+  int64_t y_offset;
+} lorax_layer_slice_t;
+
+int lorax_layer_update(const lorax_table_group_t* groups, int32_t num_groups, const void* tables,
+                       const lorax_layer_slice_t* slices, int32_t num_slices, void* y, int64_t y_stride, const void* x,
+                       int64_t num_tokens, int32_t h_in, int64_t layer_idx, void* v, int64_t v_bytes, void* tmp,
+                       int64_t tmp_bytes, int32_t dtype, int32_t device, void* stream);
 
 /*
  * Per-device set-up: looks up the address of the static scratch of lorax_sgmv_shrink_static on `device`.

@@ -8,8 +8,10 @@ There is no other implementation behind them: if the shared library is missing e
 call raises.
 """
 
+import contextlib
 import ctypes
 import os
+import struct
 from pathlib import Path
 from typing import Optional
 
@@ -19,6 +21,7 @@ LIB_PATH = Path(__file__).resolve().parent / "liblorax_hip.so"
 
 F16, BF16 = 0, 1
 ESPACE = 5
+EROUTE = 6
 A_RH, A_HR = 0, 1
 B_RH, B_HR = 0, 1
 SHRINK_TMP_BYTES = 8 * 1024 * 1024
@@ -74,7 +77,14 @@ class TableGroup(ctypes.Structure):
                 ("ends_off", _c.c_int64), ("indices_off", _c.c_int64), ("plan_off", _c.c_int64),
                 ("shrink_tiles_off", _c.c_int64), ("expand_tiles_off", _c.c_int64),
                 ("num_shrink_tiles", _c.c_int32), ("shrink_tile_rows", _c.c_int32),
-                ("num_expand_tiles", _c.c_int32), ("expand_tile_rows", _c.c_int32)]
+                ("num_expand_tiles", _c.c_int32), ("expand_tile_rows", _c.c_int32),
+                ("segments_id", _c.c_int32), ("reserved", _c.c_int32)]
+
+
+class LayerSlice(ctypes.Structure):
+    """lorax_layer_slice_t of include/lorax_hip.h."""
+
+    _fields_ = [("layer_type", _c.c_int32), ("width", _c.c_int32), ("y_offset", _c.c_int64)]
 
 
 class SgmvTiles(ctypes.Structure):
@@ -127,7 +137,7 @@ _SIGNATURES = {
     ),
     "lorax_bgmv_multi": (
         _c.c_int,
-        [_c.POINTER(BgmvProblem), _c.c_int32, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_float, _c.c_int32,
+        [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_float, _c.c_int32,
          _c.c_int32, _c.c_void_p],
     ),
     "lorax_bgmv_lora_multi": (
@@ -184,6 +194,11 @@ _SIGNATURES = {
         [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int32, _c.c_void_p, _c.c_void_p,
          _c.POINTER(_c.c_int32), _c.c_void_p, _c.c_int64, _c.POINTER(_c.c_int64), _c.POINTER(TableGroup), _c.c_int32,
          _c.POINTER(_c.c_int32)],
+    ),
+    "lorax_layer_update": (
+        _c.c_int,
+        [_c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64,
+         _c.c_int32, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_void_p],
     ),
     "lorax_init": (_c.c_int, [_c.c_int32]),
     "lorax_workspace_bytes": (_c.c_size_t, []),
@@ -257,12 +272,17 @@ def init(device) -> None:
     _initialised_devices.add(index)
 
 
+def _ready(t: torch.Tensor) -> None:
+    """init() for t's device unless it has been done or the stream is capturing (the launches then do what is missing)."""
+    if t.get_device() not in _initialised_devices and not torch.cuda.is_current_stream_capturing():
+        init(t.device)
+
+
+_DTYPE_CODES = {torch.float16: F16, torch.bfloat16: BF16}
+
+
 def _dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float16:
-        return F16
-    if t.dtype == torch.bfloat16:
-        return BF16
-    return -1
+    return _DTYPE_CODES.get(t.dtype, -1)
 
 
 def _check_input(t: torch.Tensor, name: str, dim: int) -> None:
@@ -276,8 +296,23 @@ def _check_input(t: torch.Tensor, name: str, dim: int) -> None:
         raise RuntimeError(f"{name} must be a {dim}D tensor")
 
 
+# torch's own accessors build a Stream object and a guard object per call, 2 to 3 us each; these are the calls beneath.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+_unguarded = contextlib.nullcontext()
+
+
 def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _on_device(t: torch.Tensor):
+    """Context in which t's device is the current one."""
+    if _current_device is not None and _current_device() == t.get_device():
+        return _unguarded
+    return torch.cuda.device(t.device)
 
 
 def _check_same(y: torch.Tensor, x: torch.Tensor, *rest: torch.Tensor) -> None:
@@ -309,7 +344,7 @@ def bgmv(y, x, w_ptr, indicies, layer_idx, scale, y_offset=0, y_slice_size=None)
     if y.size(0) != x.size(0):
         raise RuntimeError(f"CHECK_EQ(y.size(0), x.size(0)) failed. {y.size(0)} vs {x.size(0)}")
     h_out = y.size(1) if y_slice_size is None else int(y_slice_size)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         rc = lib().lorax_bgmv(
             y.data_ptr(), x.data_ptr(), w_ptr.data_ptr(), indicies.data_ptr(), x.size(0), x.size(1), h_out,
             int(y_offset), y.size(1), int(layer_idx), float(scale), _dtype_code(x), _stream(x),
@@ -370,9 +405,54 @@ def bgmv_multi(problems, layer_idx, scale=1.0, accumulate=True, plans=None, stac
         arr[i] = BgmvProblem(y.data_ptr(), x.data_ptr(), None if planned_only else w_ptr.data_ptr(),
                              None if planned_only else indicies.data_ptr(), int(y_offset),
                              y.size(1), h_out, plan_ptr, num_groups, x.size(1), stack, stack)
-    with torch.cuda.device(x0.device):
+    with _on_device(x0):
         rc = lib().lorax_bgmv_multi(arr, len(problems), x0.size(0), x0.size(1), int(layer_idx), float(scale),
                                     1 if accumulate else 0, _dtype_code(x0), _stream(x0))
+    if rc != 0:
+        _raise_last(rc)
+
+
+# BgmvProblem for struct.pack: ctypes takes 1.5 us to fill one
+_BGMV_PROBLEM = "4Q2qi4xQ2i2Q"
+assert struct.calcsize(_BGMV_PROBLEM) == ctypes.sizeof(BgmvProblem)
+
+
+def bgmv_stacked(y, x, jobs, plan, scale=1.0) -> None:
+    """The planned shrink launch and the planned expand launch (lorax_bgmv_multi) of up to 16 projections over stacked
+    weights: `jobs` holds (lora_a [n, r, h_in], lora_b [n, width, r], r, y_offset, width) per projection, `plan` is the
+    batch's routing plan over stack entries.  The operands are checked once for both launches."""
+    if not 1 <= len(jobs) <= MAX_BGMV_PROBLEMS:
+        raise RuntimeError(f"between 1 and {MAX_BGMV_PROBLEMS} problems per launch, got {len(jobs)}")
+    _check_input(y, "y", 2)
+    _check_input(x, "x", 2)
+    _check_input(plan, "plan", 2)
+    _check_same(y, x, plan)
+    if plan.dtype != torch.int64 or plan.size(1) != PLAN_RECORD_WORDS:
+        raise RuntimeError(f"plan must be an int64 [num_groups, {PLAN_RECORD_WORDS}] tensor on the device of x")
+    rows, h_in = x.shape
+    y_rows, y_stride = y.shape
+    if y_rows != rows:
+        raise RuntimeError(f"CHECK_EQ(y.size(0), x.size(0)) failed. {y_rows} vs {rows}")
+    groups = plan.size(0)
+    x_ptr, y_ptr = x.data_ptr(), y.data_ptr()
+    plan_ptr = plan.data_ptr() if groups > 0 else x_ptr  # an empty plan has no storage; any non-null address will do
+    v = torch.empty((rows * sum(r for _, _, r, _, _ in jobs),), dtype=x.dtype, device=x.device)
+    v_ptr = v.data_ptr()
+    shrink, expand = [], []
+    for a, b, r, y_offset, width in jobs:
+        _check_stack(a, x)
+        _check_stack(b, x)
+        shrink += (v_ptr, x_ptr, 0, 0, 0, r, r, plan_ptr, groups, h_in, a.data_ptr(), 0)
+        expand += (y_ptr, v_ptr, 0, 0, y_offset, y_stride, width, plan_ptr, groups, r, 0, b.data_ptr())
+        v_ptr += rows * r * 2
+    layout = struct.Struct(_BGMV_PROBLEM * len(jobs))
+    shrink, expand = layout.pack(*shrink), layout.pack(*expand)
+    code, stream = _dtype_code(x), _stream(x)
+    with _on_device(x):
+        launch = lib().lorax_bgmv_multi
+        rc = launch(shrink, len(jobs), rows, h_in, 0, scale, 0, code, stream)
+        if rc == 0:
+            rc = launch(expand, len(jobs), rows, jobs[0][2], 0, 1.0, 1, code, stream)
     if rc != 0:
         _raise_last(rc)
 
@@ -431,7 +511,7 @@ def bgmv_lora_multi(problems, rank, layer_idx, scale=1.0, stacks=None) -> None:
             a_stack, b_stack = stacks[i][0].data_ptr(), stacks[i][1].data_ptr()
         arr[i] = BgmvProblem(y.data_ptr(), x.data_ptr(), None, None, int(y_offset), y.size(1), h_out, plan_ptr,
                              plan.size(0), 0, a_stack, b_stack)
-    with torch.cuda.device(x0.device):
+    with _on_device(x0):
         rc = lib().lorax_bgmv_lora_multi(arr, len(problems), x0.size(0), x0.size(1), int(rank), int(layer_idx),
                                          float(scale), _dtype_code(x0), _stream(x0))
     if rc != 0:
@@ -473,7 +553,7 @@ def sgmv_expand(y, x, w_ptr, s_start, s_end, tmp, layer_idx, y_offset=0, y_slice
     h_out = y.size(1) if y_slice_size is None else int(y_slice_size)
     if tiles is not None and transposed:
         plan = tiles.c_struct(x.device)
-        with torch.cuda.device(x.device):
+        with _on_device(x):
             rc = lib().lorax_sgmv_expand_planned(
                 y.data_ptr(), x.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
                 x.size(0), x.size(1), h_out, int(y_offset), y.size(1), int(layer_idx), 1 if accumulate else 0,
@@ -482,7 +562,7 @@ def sgmv_expand(y, x, w_ptr, s_start, s_end, tmp, layer_idx, y_offset=0, y_slice
         if rc != 0:
             _raise_last(rc)
         return
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         rc = lib().lorax_sgmv_expand(
             y.data_ptr(), x.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
             x.size(0), x.size(1), h_out, B_HR if transposed else B_RH, int(y_offset), y.size(1), int(layer_idx),
@@ -516,7 +596,7 @@ def sgmv_expand_multi(problems, layer_idx, accumulate: bool = True) -> None:
         h_out = y.size(1) if y_slice_size is None else int(y_slice_size)
         arr[i] = SgmvExpandProblem(y.data_ptr(), v.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(),
                                    s_start.size(0), v.size(1), h_out, int(y_offset), y.size(1), plan)
-    with torch.cuda.device(v0.device):
+    with _on_device(v0):
         rc = lib().lorax_sgmv_expand_multi(arr, len(problems), v0.size(0), int(layer_idx), 1 if accumulate else 0,
                                            _dtype_code(v0), _stream(v0))
     if rc != 0:
@@ -525,9 +605,8 @@ def sgmv_expand_multi(problems, layer_idx, accumulate: bool = True) -> None:
 
 def _sgmv_shrink(y, x, w_ptr, s_start, s_end, tmp, layer_idx, a_layout, scale: float = 1.0) -> None:
     _check_sgmv(y, x, w_ptr, s_start, s_end, tmp)
-    if not torch.cuda.is_current_stream_capturing():
-        init(x.device)
-    with torch.cuda.device(x.device):
+    _ready(x)
+    with _on_device(x):
         rc = lib().lorax_sgmv_shrink(
             y.data_ptr(), x.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
             x.size(0), x.size(1), y.size(1), a_layout, int(layer_idx), float(scale), tmp.data_ptr(),
@@ -558,7 +637,7 @@ def sgmv_shrink_static(y, x, w_ptr, s_start, s_end, layer_idx, a_layout=A_RH, sc
     """lorax_sgmv_shrink_static: sgmv_shrink / the shrink direction of sgmv_cutlass without a tmp tensor; the
     library's own static device array serves as split-K scratch, so the call allocates nothing."""
     _check_sgmv(y, x, w_ptr, s_start, s_end, s_start)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         rc = lib().lorax_sgmv_shrink_static(
             y.data_ptr(), x.data_ptr(), w_ptr.data_ptr(), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
             x.size(0), x.size(1), y.size(1), a_layout, int(layer_idx), float(scale), _dtype_code(x), _stream(x),
@@ -586,10 +665,9 @@ def sgmv_shrink_multi(ys, x, w_ptrs, s_start, s_end, tmp, layer_idx, scale: floa
         if y.size(1) != ys[0].size(1):
             raise RuntimeError("the projections of one call share the rank")
         arr[i] = SgmvShrinkProblem(y.data_ptr(), w_ptr.data_ptr())
-    if not torch.cuda.is_current_stream_capturing():
-        init(x.device)
+    _ready(x)
     plan = tiles.c_struct(x.device) if tiles is not None else None
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         rc = lib().lorax_sgmv_shrink_multi(
             arr, len(ys), x.data_ptr(), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0), x.size(0), x.size(1),
             ys[0].size(1), int(layer_idx), float(scale), 1 if accumulate else 0, tmp.data_ptr(),
@@ -666,12 +744,71 @@ def sgmv_lora_multi(problems, x, s_start, s_end, rank, layer_idx, scale: float =
             raise RuntimeError(f"CHECK_EQ(y.size(0), x.size(0)) failed. {y.size(0)} vs {x.size(0)}")
         h_out = y.size(1) if y_slice_size is None else int(y_slice_size)
         arr[i] = SgmvLoraProblem(y.data_ptr(), a_ptr.data_ptr(), b_ptr.data_ptr(), int(y_offset), y.size(1), h_out)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         rc = lib().lorax_sgmv_lora_multi(arr, len(problems), x.data_ptr(), s_start.data_ptr(), s_end.data_ptr(),
                                          s_start.size(0), x.size(0), x.size(1), int(rank), int(layer_idx),
                                          float(scale), _dtype_code(x), _stream(x))
     if rc != 0:
         _raise_last(rc)
+
+
+class BatchTables:
+    """What lorax_layer_update needs of one batch: the builder's group records (host), the packed tables (device) and the
+    number of rows they were built for.  Owned by the batch data made from them."""
+
+    __slots__ = ("groups", "num_groups", "packed", "rows", "prefill", "device_index", "rank_sum", "_calls")
+
+    def __init__(self, groups, num_groups: int, packed: torch.Tensor, rows: int, prefill: bool):
+        self.groups = groups
+        self.num_groups = num_groups
+        self.packed = packed
+        self.rows = rows
+        self.prefill = prefill
+        self.device_index = packed.get_device()
+        self.rank_sum = {}  # layer type -> sum of the ranks of its groups
+        for g in groups[:num_groups]:
+            self.rank_sum[g.layer_type] = self.rank_sum.get(g.layer_type, 0) + g.rank
+        self._calls = {}  # slices of a call -> (LayerSlice array, columns of v)
+
+    def call(self, slices):
+        """(LayerSlice array, sum of ranks) of `slices`, a tuple of (layer type, first column, end column)."""
+        made = self._calls.get(slices)
+        if made is None:
+            arr = (LayerSlice * len(slices))(*[LayerSlice(t, end - start, start) for t, start, end in slices])
+            made = self._calls[slices] = (arr, sum(self.rank_sum[t] for t, _, _ in slices))
+        return made
+
+
+def layer_update(y, x, tables: BatchTables, slices, layer_idx: int, scratch) -> bool:
+    """lorax_layer_update: y[:, start:end] += the LoRA update of x for every slice, all launches from one call.
+    `scratch`: function that returns the 8 MiB shrink scratch of a device.  False, with nothing launched, where the
+    single entry points have to be used: operands they would refuse or that need another path."""
+    code = _DTYPE_CODES.get(x.dtype)
+    if (code is None or y.dtype != x.dtype or x.dim() != 2 or y.dim() != 2 or not x.is_cuda or not y.is_cuda
+            or not x.is_contiguous() or not y.is_contiguous()):
+        return False
+    rows, h_in = x.shape
+    y_rows, width = y.shape
+    index = tables.device_index
+    if (x.get_device() != index or y.get_device() != index or y_rows != rows or rows == 0
+            or not (tables.prefill or rows == tables.rows)):
+        return False
+    arr, columns = tables.call(slices)
+    tmp = None
+    if tables.prefill:
+        _ready(x)
+        tmp = scratch(x.device)
+    v = torch.empty((rows * columns,), dtype=x.dtype, device=x.device)
+    rc = lib().lorax_layer_update(
+        tables.groups, tables.num_groups, tables.packed.data_ptr(), arr, len(arr), y.data_ptr(), width, x.data_ptr(), rows,
+        h_in, layer_idx, v.data_ptr(), rows * columns * 2, tmp.data_ptr() if tmp is not None else None,
+        tmp.numel() if tmp is not None else 0, code, index, _stream(x),
+    )
+    if rc == EROUTE:
+        return False
+    if rc != 0:
+        _raise_last(rc)
+    return True
 
 
 ENTRY_DTYPE = [("adapter", "<i8"), ("a_addr", "<i8"), ("b_addr", "<i8"), ("rank", "<i4"), ("reserved", "<i4")]
@@ -684,6 +821,12 @@ def build_batch_tables(adapter_indices, entries, entry_counts, prefill: bool):
     """lorax_build_batch_tables on numpy arrays: adapter_indices int64 [T]; entries a structured array of
     ENTRY_DTYPE, the layer types' adapters one after the other, each type sorted by adapter; entry_counts int32
     per type.  Returns (segment bounds int32 [S+1], segment owners int64 [S], packed uint8 buffer, groups)."""
+    bounds, owners, packed, groups, n = batch_tables(adapter_indices, entries, entry_counts, prefill)
+    return bounds, owners, packed, list(groups[:n])
+
+
+def batch_tables(adapter_indices, entries, entry_counts, prefill: bool):
+    """build_batch_tables with the group records as the ctypes array the builder filled and their number."""
     import numpy as np
 
     adapter_indices = np.ascontiguousarray(adapter_indices, dtype=np.int64)
@@ -709,4 +852,4 @@ def build_batch_tables(adapter_indices, entries, entry_counts, prefill: bool):
             continue
         if rc != 0:
             _raise_last(rc)
-        return bounds[: nseg.value + 1], owners[: nseg.value], packed[: nbytes.value], list(groups[: ngroups.value])
+        return bounds[: nseg.value + 1], owners[: nseg.value], packed[: nbytes.value], groups, ngroups.value

@@ -15,7 +15,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "liblorax_hip.so"
 SOURCES = ["capi.hip", "bgmv.hip", "sgmv_shrink.hip", "sgmv_shrink_lds.hip", "sgmv_expand.hip", "sgmv_expand_t.hip",
-           "batch_tables.hip"]
+           "batch_tables.hip", "layer_update.hip"]
 ARCH = "gfx950"
 
 # -packed-fp32-ops is switched off on purpose: the packed fp32 forms hipcc would

@@ -84,6 +84,7 @@ extern "C" int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t 
   std::vector<int64_t> entry_rows;
   std::vector<int32_t> tile_starts, tile_ends;
   std::vector<lorax_sgmv_tile_t> tile_buf;
+  std::vector<std::vector<int32_t>> known_bounds;  // distinct segment lists of the groups so far
   for (int32_t s = 0; s < num_segments; ++s)
     for (int32_t t = segment_bounds[s]; t < segment_bounds[s + 1]; ++t) token_seg[t] = s;
 
@@ -164,7 +165,19 @@ extern "C" int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t 
       desc.starts_off = desc.ends_off = desc.indices_off = desc.plan_off = -1;
       desc.shrink_tiles_off = desc.expand_tiles_off = -1;
       desc.num_long_segments = n;
+      desc.segments_id = -1;
       if (use_sgmv) {
+        // equal bounds get the number of the first group that has them
+        auto same_bounds = [&](const std::vector<int32_t>& other) {
+          if (other.size() != segs.size()) return false;
+          for (int32_t i = 0; i < n; ++i)
+            if (segment_bounds[other[i]] != segment_bounds[segs[i]]) return false;  // runs of tokens: the start names the run
+          return true;
+        };
+        size_t id = 0;
+        while (id < known_bounds.size() && !same_bounds(known_bounds[id])) ++id;
+        if (id == known_bounds.size()) known_bounds.push_back(segs);
+        desc.segments_id = static_cast<int32_t>(id);
         desc.starts_off = pack.reserve(static_cast<int64_t>(n) * 4);
         desc.ends_off = pack.reserve(static_cast<int64_t>(n) * 4);
         if (int32_t* st = pack.at<int32_t>(desc.starts_off)) {

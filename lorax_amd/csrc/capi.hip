@@ -92,6 +92,8 @@ const Tuning& tuning() {
   return t;
 }
 
+int report_error(int code, const char* message) { return fail(code, "%s", message); }
+
 bool fixed_order_shrink() { return g_fixed_order_shrink.load(std::memory_order_relaxed) != 0; }
 
 }  // namespace lorax

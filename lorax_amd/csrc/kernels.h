@@ -180,6 +180,8 @@ struct Tuning {
   int bgmv_scalar_y;    // LORAX_BGMV_SCALAR_Y: BGMV expand that moves y element by element even where rows are aligned
 };
 const Tuning& tuning();
+// Leaves `message` for lorax_last_error and returns `code`.
+int report_error(int code, const char* message);
 // lorax_set_fixed_order_shrink: the SGMV shrinks walk the hidden dimension from k = 0 in every tile and never cut
 // it across workgroups.
 bool fixed_order_shrink();

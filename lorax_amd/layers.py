@@ -76,6 +76,28 @@ class LoraLinear(nn.Module):
             )
         return data
 
+    def _native_update(self, result, input, adapter_data: AdapterBatchData, slices) -> bool:
+        """All launches of the call from one native call (lorax_layer_update), where every projection's tables are
+        the untouched packed ones of the batch; False, with nothing launched, where the general path has to run."""
+        if adapter_data.layer_to_lora_weights and adapter_data.punica_wrapper is not None:
+            return False
+        if not has_sgmv() or self.process_group.size() > 1:
+            return False
+        tables, targets = None, []
+        for name, start, end in slices:
+            layer_data = adapter_data.data.get(name)
+            data = layer_data.get(LORA) if layer_data is not None else None
+            if data is None:
+                continue  # no adapter in the batch targets this projection
+            own = getattr(data, "packed_tables", None)
+            if own is None or (tables is not None and own is not tables):
+                return False
+            tables = own
+            targets.append((data.layer_type, start, end))
+        if tables is None:
+            return False
+        return _native.layer_update(result, input, tables, tuple(targets), self.layer_id, get_shrink_scratch)
+
     def forward_layer_types(
         self,
         result: torch.Tensor,
@@ -85,6 +107,8 @@ class LoraLinear(nn.Module):
     ) -> torch.Tensor:
         """Adds the LoRA deltas of several projections that share `input`; projection `name` owns the
         columns [start, end) of `result`."""
+        if self._native_update(result, input, adapter_data, slices):
+            return result
         tensor_parallel = self.process_group.size() > 1
         decode_jobs = defaultdict(list)  # (wave, rank) -> [(rank_segments, start, width)]
         stacked_jobs = []  # (lora_a_stack, lora_b_stack, start, width) of projections served by stacked weights

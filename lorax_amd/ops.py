@@ -183,7 +183,6 @@ def build_slot_plan(slots) -> "torch.Tensor":
     return torch.from_numpy(records)
 
 
-@torch.inference_mode()
 def bgmv_lora_slices(
     inputs: torch.Tensor,
     slices,
@@ -226,18 +225,14 @@ def bgmv_lora_slices(
     tokens = inputs.size(0)
     for i in range(0, len(jobs), step):
         chunk = jobs[i : i + step]
+        if plan is not None:
+            _native.bgmv_stacked(output_tensor, inputs, chunk, plan, scaling)
+            continue
         flat = torch.empty((tokens * sum(r for _, _, r, _, _ in chunk),), dtype=inputs.dtype, device=inputs.device)
         bufs, pos = [], 0
         for _, _, r, _, _ in chunk:
             bufs.append(flat[pos : pos + tokens * r].view(tokens, r))
             pos += tokens * r
-        if plan is not None:
-            plans = [plan] * len(chunk)
-            _native.bgmv_multi([(v, inputs, None, None, 0, None) for v in bufs], 0, scaling, False, plans,
-                               stacks=[a for a, _, _, _, _ in chunk])
-            _native.bgmv_multi([(output_tensor, v, None, None, off, size) for v, (_, _, _, off, size) in zip(bufs, chunk)],
-                               0, 1.0, True, plans, stacks=[b for _, b, _, _, _ in chunk])
-            continue
         _native.bgmv_multi([(v, inputs, stack_table(a), lora_indices_tensor, 0, None)
                             for v, (a, _, _, _, _) in zip(bufs, chunk)], 0, scaling, False)
         _native.bgmv_multi([(output_tensor, v, stack_table(b), lora_indices_tensor, off, size)
