@@ -714,9 +714,11 @@ SGMV_LORA_MAX_TOKENS = 512
 def sgmv_lora_fits(rank: int, h_in: int, num_tokens: int, h_out: int = 0) -> bool:
     """True where the single-launch prefill update (lorax_sgmv_lora_multi) applies and pays: rank 8 or 16 with a
     small A slab, a batch short enough to be bound by launches, and an output that is not so wide (an LM head)
-    that recomputing the shrink in every column slice would dominate."""
-    return (rank in FUSED_BGMV_RANKS and rank * h_in * 2 <= 128 * 1024 and num_tokens <= SGMV_LORA_MAX_TOKENS
-            and h_out <= 16384)
+    that recomputing the shrink in every column slice would dominate.  (Rank 16: every four rows read A again; a
+    Mistral-7B block of one run takes 49 us per layer in one launch per group and 51 in two at 128 rows, 61 and 54 at
+    192, 116 and 72 at 512.  Rank 8: 56 and 65 us at 512.)"""
+    return (rank in FUSED_BGMV_RANKS and rank * h_in * 2 <= 128 * 1024
+            and num_tokens <= (SGMV_LORA_MAX_TOKENS if rank == 8 else SGMV_LORA_MAX_TOKENS // 4) and h_out <= 16384)
 
 
 def sgmv_lora_multi(problems, x, s_start, s_end, rank, layer_idx, scale: float = 1.0) -> None:

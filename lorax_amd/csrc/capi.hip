@@ -416,11 +416,13 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
   if (num_problems < 1 || num_problems > kMaxShrinkGroup)
     return fail(LORAX_EINVAL, "num_problems=%d (1 to %d per call)", num_problems, kMaxShrinkGroup);
   if (problems == nullptr) return fail(LORAX_EINVAL, "null pointer argument (problems)");
-  // One launch where the LDS-staged kernel takes the stacked rank and the batch is past the streaming
-  // kernel's range; otherwise one launch per projection, with the same result.
+  // One launch where the streaming kernel takes the batch (short ones) or the LDS-staged kernel the stacked rank;
+  // otherwise one launch per projection, with the same result.
   const int rows_max = tuning().shrink_rows_max != 0 ? tuning().shrink_rows_max : 512;
-  const bool stacked = r >= 8 && r % 8 == 0 && num_problems * r <= kMaxRank && h_in > 0 &&
-                       h_in % 128 == 0 && num_tokens > rows_max && tuning().shrink_lds >= 0;
+  const bool shape_ok = r >= 8 && r % 8 == 0 && r <= kMaxRank && h_in > 0;
+  const bool streamed = shape_ok && h_in % 8 == 0 && num_tokens <= rows_max && num_problems > 1;
+  const bool stacked = streamed || (shape_ok && num_problems * r <= kMaxRank && h_in % 128 == 0 && num_tokens > rows_max &&
+                                    tuning().shrink_lds >= 0);
   if (!stacked) {
     for (int i = 0; i < num_problems; ++i) {
       if (tmp_bytes < LORAX_SHRINK_TMP_BYTES)
@@ -442,7 +444,7 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
   if (tmp_bytes < LORAX_SHRINK_TMP_BYTES)
     return fail(LORAX_ETMPSIZE, "CHECK_GE(tmp.size(0), 8 * 1024 * 1024) failed. %lld vs %d", (long long)tmp_bytes,
                 LORAX_SHRINK_TMP_BYTES);
-  if (num_segments == 0) return LORAX_OK;
+  if (num_segments == 0 || (streamed && num_tokens == 0)) return LORAX_OK;
   for (int i = 0; i < num_problems; ++i)
     if (int rc = check_common(problems[i].v, x, problems[i].w_ptrs, dtype)) return rc;
   if (s_start == nullptr || s_end == nullptr || tmp == nullptr)
@@ -474,6 +476,11 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
   for (int i = 0; i < num_problems; ++i) {
     a.group.v[i] = problems[i].v;
     a.group.w[i] = problems[i].w_ptrs;
+  }
+  if (streamed) {
+    const hipError_t e = launch_sgmv_shrink_rows(a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_shrink launch failed: %s", hipGetErrorString(e));
+    return LORAX_OK;
   }
   if (int rc = take_tiles(tiles, a)) return rc;
   if (a.tiles != nullptr && a.num_tiles == 0) return LORAX_OK;  // a plan without tiles: no segment has rows

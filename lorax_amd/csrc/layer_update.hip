@@ -11,7 +11,8 @@ namespace {
 constexpr int kMaxJobs = 256;        // (projection, rank group) pairs of one call
 constexpr int kMaxKernelRank = 128;
 constexpr int64_t kMaxBgmvRows = 65535;  // rows of a BGMV launch and records of one routing plan
-constexpr int64_t kShortBatchRows = 512;  // largest batch of lorax_sgmv_lora_multi
+constexpr int64_t kShortBatchRows = 512;  // largest batch of the streaming shrink and of lorax_sgmv_lora_multi at rank 8
+constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 (measured: _native.sgmv_lora_fits)
 
 struct Job {
   const lorax_table_group_t* g;
@@ -101,7 +102,7 @@ int prefill(const Call& c, Job* const* jobs, int count) {
       widest = jobs[end]->width > widest ? jobs[end]->width : widest;
     const int32_t* starts = static_cast<const int32_t*>(at(c, g.starts_off));
     const int32_t* ends = static_cast<const int32_t*>(at(c, g.ends_off));
-    if (fused_rank(g.rank, c.h_in) && c.rows <= kShortBatchRows && widest <= 16384) {
+    if (fused_rank(g.rank, c.h_in) && c.rows <= (g.rank == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= 16384) {
       for (int k = i; k < end; k += lorax::kMaxSgmvLoraProblems) {
         lorax_sgmv_lora_problem_t p[lorax::kMaxSgmvLoraProblems];
         int n = 0;
@@ -121,7 +122,9 @@ int prefill(const Call& c, Job* const* jobs, int count) {
     for (int k = i; k < end; ++k) split = split && jobs[k]->g->plan_off >= 0 && jobs[k]->g->num_chunks <= kMaxBgmvRows;
     const int32_t n_long = split ? g.num_long_segments : g.num_segments;
     const bool planned = n_long == g.num_long_segments;  // the tables' row-tile plans cover these segments
-    const int step = kMaxKernelRank / g.rank < lorax::kMaxShrinkGroup ? kMaxKernelRank / g.rank : lorax::kMaxShrinkGroup;
+    // one shrink launch for up to four projections: of a short batch at any rank, else of a summed rank of 128
+    const int step = c.rows <= kShortBatchRows || kMaxKernelRank / g.rank >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup
+                                                                                                   : kMaxKernelRank / g.rank;
     for (int k = i; k < end && n_long > 0; k += step) {
       lorax_sgmv_shrink_problem_t p[lorax::kMaxShrinkGroup];
       int n = 0;

@@ -238,6 +238,8 @@ class LoraLinear(nn.Module):
             # v needs no zero-fill: the shrinks overwrite the rows of their segments and the expands read no others
             vs = list(torch.empty((len(group), rows, r), dtype=input.dtype, device=input.device).unbind(0))
             step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, MAX_RANK_CUSTOM // r))
+            if rows <= _native.SGMV_LORA_MAX_TOKENS:
+                step = MAX_SGMV_SHRINK_PROBLEMS  # the streaming shrink of a short batch takes any ranks
             # (no long segment at all: the per-token launches do the whole update)
             for i in range(0, len(group) if n_long > 0 else 0, step):
                 _native.sgmv_shrink_multi(
