@@ -284,6 +284,27 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
                             int32_t accumulate, void* tmp, int64_t tmp_bytes, const lorax_sgmv_tiles_t* tiles,
                             int32_t dtype, void* stream);
 
+/*
+ * lorax_sgmv_shrink_multi for up to 16 groups of projections over the same x - the rank groups of a batch whose
+ * adapters differ in rank, projections whose summed rank exceeds 128 - in one launch (and one that adds the parts of a
+ * split hidden dimension) where every group brings a row-tile plan of tiles of at most 32 rows, has a summed rank of at most
+ * 128 over an h_in that is a multiple of 128, and the batch has more than 512 rows; else one call per group.  The groups'
+ * elements of v must be disjoint.
+ */
+typedef struct lorax_sgmv_shrink_group {
+  const lorax_sgmv_shrink_problem_t* problems; /* host */
+  int32_t num_problems;                        /* 1 to 4 */
+  int32_t r;
+  const int32_t* s_start;                      /* device, num_segments entries, as s_end */
+  const int32_t* s_end;
+  int32_t num_segments;
+  const lorax_sgmv_tiles_t* tiles;             /* host struct or NULL */
+} lorax_sgmv_shrink_group_t;
+
+int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x,
+                             int64_t num_tokens, int32_t h_in, int64_t layer_idx, float scale, int32_t accumulate,
+                             void* tmp, int64_t tmp_bytes, int32_t dtype, void* stream);
+
 /* Process-wide switch (default 0): 1 = the SGMV shrinks add their sums over the hidden dimension in one fixed
  * order whatever the batch (see lorax_sgmv_shrink_multi).  Returns the previous value.  Not meant to be flipped
  * while launches are being issued from other threads. */

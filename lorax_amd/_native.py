@@ -54,6 +54,13 @@ class SgmvShrinkProblem(ctypes.Structure):
     _fields_ = [("v", _c.c_void_p), ("w_ptrs", _c.c_void_p)]
 
 
+class SgmvShrinkGroup(ctypes.Structure):
+    """lorax_sgmv_shrink_group_t of include/lorax_hip.h."""
+
+    _fields_ = [("problems", _c.POINTER(SgmvShrinkProblem)), ("num_problems", _c.c_int32), ("r", _c.c_int32),
+                ("s_start", _c.c_void_p), ("s_end", _c.c_void_p), ("num_segments", _c.c_int32), ("tiles", _c.c_void_p)]
+
+
 class SgmvLoraProblem(ctypes.Structure):
     """lorax_sgmv_lora_problem_t of include/lorax_hip.h."""
 
@@ -161,6 +168,11 @@ _SIGNATURES = {
         [_c.POINTER(SgmvShrinkProblem), _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int64,
          _c.c_int32, _c.c_int32, _c.c_int64, _c.c_float, _c.c_int32, _c.c_void_p, _c.c_int64, _c.POINTER(SgmvTiles),
          _c.c_int32, _c.c_void_p],
+    ),
+    "lorax_sgmv_shrink_groups": (
+        _c.c_int,
+        [_c.POINTER(SgmvShrinkGroup), _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_float, _c.c_int32,
+         _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_void_p],
     ),
     "lorax_sgmv_expand_planned": (
         _c.c_int,
@@ -674,6 +686,39 @@ def sgmv_shrink_multi(ys, x, w_ptrs, s_start, s_end, tmp, layer_idx, scale: floa
             tmp.numel() * tmp.element_size(), ctypes.byref(plan) if plan is not None else None, _dtype_code(x),
             _stream(x),
         )
+    if rc != 0:
+        _raise_last(rc)
+
+
+MAX_SGMV_SHRINK_GROUPS = 16
+
+
+def sgmv_shrink_groups(groups, x, tmp, layer_idx, scale: float = 1.0, accumulate: bool = True) -> None:
+    """lorax_sgmv_shrink_groups: sgmv_shrink_multi for up to 16 groups over the same x, in one launch where they qualify.
+    `groups` is a list of tuples (ys, w_ptrs, s_start, s_end, tiles) as sgmv_shrink_multi takes them."""
+    if not 1 <= len(groups) <= MAX_SGMV_SHRINK_GROUPS:
+        raise RuntimeError(f"between 1 and {MAX_SGMV_SHRINK_GROUPS} groups per call, got {len(groups)}")
+    if isinstance(tmp, torch.Tensor) and tmp.dtype != torch.uint8:
+        raise RuntimeError(f"CHECK_EQ(tmp.scalar_type(), at::ScalarType::Byte) failed. {tmp.dtype}")
+    arr, keep = (SgmvShrinkGroup * len(groups))(), []
+    for i, (ys, w_ptrs, s_start, s_end, tiles) in enumerate(groups):
+        if not 1 <= len(ys) <= MAX_SGMV_SHRINK_PROBLEMS or len(ys) != len(w_ptrs):
+            raise RuntimeError(f"between 1 and {MAX_SGMV_SHRINK_PROBLEMS} outputs with one pointer table each")
+        problems = (SgmvShrinkProblem * len(ys))()
+        for k, (y, w_ptr) in enumerate(zip(ys, w_ptrs)):
+            _check_sgmv(y, x, w_ptr, s_start, s_end, tmp)
+            if y.size(1) != ys[0].size(1):
+                raise RuntimeError("the projections of one group share the rank")
+            problems[k] = SgmvShrinkProblem(y.data_ptr(), w_ptr.data_ptr())
+        plan = tiles.c_struct(x.device) if tiles is not None else None
+        keep.append((problems, plan))
+        arr[i] = SgmvShrinkGroup(problems, len(ys), ys[0].size(1), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
+                                 ctypes.addressof(plan) if plan is not None else None)
+    _ready(x)
+    with _on_device(x):
+        rc = lib().lorax_sgmv_shrink_groups(arr, len(groups), x.data_ptr(), x.size(0), x.size(1), int(layer_idx), float(scale),
+                                            1 if accumulate else 0, tmp.data_ptr(), tmp.numel() * tmp.element_size(),
+                                            _dtype_code(x), _stream(x))
     if rc != 0:
         _raise_last(rc)
 

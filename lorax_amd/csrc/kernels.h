@@ -194,6 +194,10 @@ hipError_t launch_sgmv_expand_t(const ExpandArgs& a, hipStream_t stream);  // B 
 // LDS-staged shrink (sgmv_shrink_lds.hip): [L, r, h_in] layout, h_in a multiple of 128.
 bool sgmv_shrink_lds_applies(const SgmvArgs& a);
 hipError_t launch_sgmv_shrink_lds(const SgmvArgs& a, hipStream_t stream);
+// Several groups of projections over the same x in one launch: all fields but y, w_ptrs, group, d_out, the segment
+// tables and the tile plan are those of groups[0].
+bool sgmv_shrink_groups_applies(const SgmvArgs* groups, int count);
+hipError_t launch_sgmv_shrink_groups(const SgmvArgs* groups, int count, hipStream_t stream);
 // Per-device set-up of the LDS-staged shrink on the current device (the dynamic LDS limit of every instantiation),
 // so that no launch has first-call state; a launch that finds it missing does it itself.
 hipError_t configure_sgmv_shrink_lds();

@@ -94,6 +94,17 @@ int prefill(const Call& c, Job* const* jobs, int count) {
   const Job* shorts[kMaxJobs];
   int32_t expand_segments[kMaxJobs];
   int num_expand = 0, num_shorts = 0;
+  constexpr int kShrinkBatch = 16;
+  lorax_sgmv_shrink_problem_t problems[kShrinkBatch][lorax::kMaxShrinkGroup];
+  lorax_sgmv_tiles_t tiles[kShrinkBatch];
+  lorax_sgmv_shrink_group_t shrinks[kShrinkBatch];
+  int num_shrinks = 0;
+  auto flush_shrinks = [&]() {
+    const int n = num_shrinks;
+    num_shrinks = 0;
+    return lorax_sgmv_shrink_groups(shrinks, n, c.x, c.rows, c.h_in, c.layer_idx, 1.0f, 0, c.tmp, c.tmp_bytes, c.dtype,
+                                    c.stream);
+  };
   // `jobs` is ordered by group of equal rank and segment tables
   for (int i = 0, end = 0; i < count; i = end) {
     const lorax_table_group_t& g = *jobs[i]->g;
@@ -126,15 +137,15 @@ int prefill(const Call& c, Job* const* jobs, int count) {
     const int step = c.rows <= kShortBatchRows || kMaxKernelRank / g.rank >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup
                                                                                                    : kMaxKernelRank / g.rank;
     for (int k = i; k < end && n_long > 0; k += step) {
-      lorax_sgmv_shrink_problem_t p[lorax::kMaxShrinkGroup];
+      lorax_sgmv_shrink_problem_t* p = problems[num_shrinks];
       int n = 0;
       for (; n < step && k + n < end; ++n)
         p[n] = {jobs[k + n]->v, static_cast<const int64_t*>(at(c, jobs[k + n]->g->a_ptr_off))};
-      const lorax_sgmv_tiles_t tiles{static_cast<const lorax_sgmv_tile_t*>(at(c, g.shrink_tiles_off)), g.num_shrink_tiles,
-                                     g.shrink_tile_rows};
-      if (int rc = lorax_sgmv_shrink_multi(p, n, c.x, starts, ends, n_long, c.rows, c.h_in, g.rank, c.layer_idx, 1.0f, 0, c.tmp,
-                                           c.tmp_bytes, planned ? &tiles : nullptr, c.dtype, c.stream))
-        return rc;
+      tiles[num_shrinks] = {static_cast<const lorax_sgmv_tile_t*>(at(c, g.shrink_tiles_off)), g.num_shrink_tiles,
+                            g.shrink_tile_rows};
+      shrinks[num_shrinks] = {p, n, g.rank, starts, ends, n_long, planned ? &tiles[num_shrinks] : nullptr};
+      if (++num_shrinks == kShrinkBatch)
+        if (int rc = flush_shrinks()) return rc;
     }
     for (int k = i; k < end; ++k) {
       if (n_long > 0) {
@@ -144,21 +155,23 @@ int prefill(const Call& c, Job* const* jobs, int count) {
       if (split) shorts[num_shorts++] = jobs[k];
     }
   }
+  if (num_shrinks > 0)
+    if (int rc = flush_shrinks()) return rc;
   for (int i = 0; i < num_shorts; i += lorax::kMaxBgmvProblems) {
     const int n = num_shorts - i < lorax::kMaxBgmvProblems ? num_shorts - i : lorax::kMaxBgmvProblems;
     if (int rc = bgmv_jobs(c, shorts + i, n, true)) return rc;
   }
   for (int i = 0; i < num_expand; i += lorax::kMaxExpandProblems) {
     lorax_sgmv_expand_problem_t p[lorax::kMaxExpandProblems];
-    lorax_sgmv_tiles_t tiles[lorax::kMaxExpandProblems];
+    lorax_sgmv_tiles_t tiles_of[lorax::kMaxExpandProblems];
     int n = 0;
     for (; n < lorax::kMaxExpandProblems && i + n < num_expand; ++n) {
       const Job& j = *expand[i + n];
       const lorax_table_group_t& g = *j.g;
-      tiles[n] = {static_cast<const lorax_sgmv_tile_t*>(at(c, g.expand_tiles_off)), g.num_expand_tiles, g.expand_tile_rows};
+      tiles_of[n] = {static_cast<const lorax_sgmv_tile_t*>(at(c, g.expand_tiles_off)), g.num_expand_tiles, g.expand_tile_rows};
       p[n] = {c.y, j.v, static_cast<const int64_t*>(at(c, g.b_ptr_off)), static_cast<const int32_t*>(at(c, g.starts_off)),
               static_cast<const int32_t*>(at(c, g.ends_off)), expand_segments[i + n], g.rank, j.width, j.y_offset, c.y_stride,
-              expand_segments[i + n] == g.num_long_segments ? &tiles[n] : nullptr};
+              expand_segments[i + n] == g.num_long_segments ? &tiles_of[n] : nullptr};
     }
     if (int rc = lorax_sgmv_expand_multi(p, n, c.rows, c.layer_idx, 1, c.dtype, c.stream)) return rc;
   }

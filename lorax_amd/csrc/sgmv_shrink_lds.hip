@@ -21,6 +21,7 @@
 // The barrier is a bare s_barrier: __syncthreads() would wait for ALL outstanding loads and
 // serialise the pipeline.
 #include <atomic>
+#include <type_traits>
 
 #include "kernels.h"
 #include "sgmv_tiles.h"
@@ -56,12 +57,15 @@ __device__ __forceinline__ void wait_pending(int pending) {
   }
 }
 
+// The row tiles of one group of projections that a workgroup walks: first_tile, first_tile + tile_step, ... over part
+// `kpart` of `kparts` of the hidden dimension.  Parts leave their fp32 sums in partials[kpart][row][R]; with `compact`
+// (several groups in a launch) rows are numbered tile by tile instead of through the batch, ROWS per tile.
 template <typename D, int NB, int MBLK, bool KSPLIT>
-__global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
-    const ShrinkGroup grp, const typename D::E* __restrict__ X, const int32_t* __restrict__ s_start,
+__device__ __forceinline__ void shrink_walk(
+    const ShrinkGroup& grp, const typename D::E* __restrict__ X, const int32_t* __restrict__ s_start,
     const int32_t* __restrict__ s_end, int num_segments, int num_tokens, int h_in, int64_t layer_idx,
-    int stages, float scale, int accumulate_into_v, int rows_per_tile, int kparts, int tile_slots,
-    float* __restrict__ partials, int rotate, const TileList plan) {
+    int stages, float scale, int accumulate_into_v, int rows_per_tile, int kparts, int kpart, int first_tile, int tile_step,
+    int tile_slots, float* __restrict__ partials, bool compact, int rotate, const TileList& plan) {
   using E = typename D::E;
   using vec8 = typename D::vec8;
   // The A tile stacks the A matrices of grp.count projections of rank r: row p * r + i is row i of
@@ -98,12 +102,6 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
   const int g = lane >> 4;
   const int wm = KSPLIT ? 0 : wave % WM;
   const int wn = KSPLIT ? 0 : wave / WM;
-  const VirtualBlock vb = xcd_virtual_block();
-  // K split across workgroups (kparts > 1, launches with few row tiles): workgroup p * tile_slots + t multiplies
-  // part p of the hidden dimension for tile t and leaves its fp32 sums in partials[p][row][R]; a second kernel
-  // adds the parts in a fixed order.  Tiles are numbered fastest: neighbours (one XCD) read the same part of A.
-  const int kpart = kparts > 1 ? vb.x / tile_slots : 0;
-  const int first_tile = kparts > 1 ? vb.x - kpart * tile_slots : vb.x;
   const int st_begin = static_cast<int>(static_cast<int64_t>(kpart) * (h_in / kLdsKc) / kparts);
   const int nst = static_cast<int>(static_cast<int64_t>(kpart + 1) * (h_in / kLdsKc) / kparts) - st_begin;
   const int k_begin = st_begin * kLdsKc;
@@ -113,7 +111,7 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
 #pragma unroll
   for (int p = 0; p < kMaxShrinkGroup; ++p) pre_w[p] = preload_segment_entry(grp.w[p < grp.count ? p : 0], num_segments);
 
-  for (int tile = first_tile;; tile += gridDim.x) {
+  for (int tile = first_tile;; tile += tile_step) {
     if (kparts > 1 && tile != first_tile) break;  // one tile per workgroup when K is split
     RowTile rt;
     // tiles may be lower than the ROWS the buffers hold: rows past a tile's end re-read its last row
@@ -222,7 +220,8 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
       const int proj = col / r;
       if (kparts > 1) {
         if (row < rt.row_end && proj < grp.count)
-          *reinterpret_cast<f32x4*>(partials + (static_cast<int64_t>(kpart) * num_tokens + row) * R + col) = sum;
+          *reinterpret_cast<f32x4*>(partials + (compact ? (static_cast<int64_t>(kpart) * tile_slots + tile) * ROWS + row - rt.row0
+                                                        : static_cast<int64_t>(kpart) * num_tokens + row) * R + col) = sum;
       } else if (row < rt.row_end && proj < grp.count) {
         E* Vp = static_cast<E*>(proj == 0 ? grp.v[0] : (proj == 1 ? grp.v[1] : (proj == 2 ? grp.v[2] : grp.v[3])));
         update4<D>(accumulate_into_v != 0, Vp + static_cast<int64_t>(row) * r + (col - proj * r), sum * scale);
@@ -267,6 +266,91 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
   }
 }
 
+template <typename D, int NB, int MBLK, bool KSPLIT>
+__global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_lds_kernel(
+    const ShrinkGroup grp, const typename D::E* __restrict__ X, const int32_t* __restrict__ s_start,
+    const int32_t* __restrict__ s_end, int num_segments, int num_tokens, int h_in, int64_t layer_idx,
+    int stages, float scale, int accumulate_into_v, int rows_per_tile, int kparts, int tile_slots,
+    float* __restrict__ partials, int rotate, const TileList plan) {
+  // K split across workgroups (kparts > 1, launches with few row tiles): workgroup p * tile_slots + t multiplies
+  // part p of the hidden dimension for tile t and leaves its fp32 sums in partials[p][row][R]; a second kernel
+  // adds the parts in a fixed order.  Tiles are numbered fastest: neighbours (one XCD) read the same part of A.
+  const VirtualBlock vb = xcd_virtual_block();
+  const int kpart = kparts > 1 ? vb.x / tile_slots : 0;
+  const int first_tile = kparts > 1 ? vb.x - kpart * tile_slots : vb.x;
+  shrink_walk<D, NB, MBLK, KSPLIT>(grp, X, s_start, s_end, num_segments, num_tokens, h_in, layer_idx, stages, scale,
+                                   accumulate_into_v, rows_per_tile, kparts, kpart, first_tile, gridDim.x, tile_slots, partials,
+                                   false, rotate, plan);
+}
+
+// One launch for several groups of projections over the same x: the rank groups of a batch whose adapters differ in
+// rank, and projections whose summed rank exceeds one A tile.  A prefill of 2000 rows with four ranks issued 4 to 5
+// shrinks per layer group, each of 20 to 70 row tiles cut into K parts and followed by a launch that adds them: 12 us
+// and 4 us apiece, for 100 MB through the L1s (8 us) in all.  Together the tiles fill the chip without cutting K so
+// far: GPU time of two Mistral-7B layers of 2062 rows with ranks 8 to 64 815 -> 615 us, of four layers of 786 rows at
+// rank 64 (q + k and v apart) 621 -> 598 us, of a 70B layer of 4096 + 260 rows at rank 128 1926 -> 1878 us.  The workgroup
+// picks the body for its group's rank blocks and tile height (16 or 32 rows: a group of 48-row tiles or higher has
+// enough of them for a launch of its own); tiles come from the callers' plans.
+struct ShrinkSlot {
+  ShrinkGroup grp;
+  const int32_t* s_start;
+  const int32_t* s_end;
+  const int32_t* tiles;
+  float* partials;
+  int num_segments;
+  int num_tiles;
+  int nb;      // 16-column rank blocks of the stacked A tile
+  int mblk;    // 16-row blocks of the stage buffers, 1 or 2
+  int stages;
+};
+constexpr int kMaxShrinkSlots = 16;
+struct ShrinkLaunch {
+  ShrinkSlot p[kMaxShrinkSlots];
+  int wg_end[kMaxShrinkSlots];    // slot i owns the workgroups [wg_end[i - 1], wg_end[i])
+  int tile_end[kMaxShrinkSlots];  // the same in row tiles (the launch that adds the parts)
+};
+
+// Slot of workgroup `id`; turns id into its number inside the slot.
+__device__ __forceinline__ int shrink_slot_of(const int* ends, int count, int& id) {
+  const int lane = lane_id();
+  const int end = ends[lane < kMaxShrinkSlots ? lane : kMaxShrinkSlots - 1];
+  const int slot = __popcll(__ballot(lane + 1 < count && id >= end));
+  if (slot > 0) id -= read_lane(end, slot - 1);
+  return slot;
+}
+
+template <typename D>
+__global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_kernel(const ShrinkLaunch batch, int count,
+                                                                         const typename D::E* __restrict__ X, int num_tokens,
+                                                                         int h_in, int64_t layer_idx, float scale,
+                                                                         int accumulate_into_v, int kparts, int rotate) {
+  int id = static_cast<int>(xcd_virtual_id());
+  const ShrinkSlot& S = batch.p[shrink_slot_of(batch.wg_end, count, id)];
+  const int kpart = id / S.num_tiles;
+  const int tile = id - kpart * S.num_tiles;
+  auto walk = [&](auto nb, auto mblk) {
+    constexpr int NB = decltype(nb)::value, MBLK = decltype(mblk)::value;
+    const TileList plan{S.tiles, S.num_tiles, MBLK * 16};
+    shrink_walk<D, NB, MBLK, true>(S.grp, X, S.s_start, S.s_end, S.num_segments, num_tokens, h_in, layer_idx, S.stages, scale,
+                                   accumulate_into_v, MBLK * 16, kparts, kpart, tile, S.num_tiles, S.num_tiles, S.partials, true,
+                                   rotate, plan);
+  };
+  auto pick = [&](auto mblk) {
+    switch (S.nb) {
+      case 1: walk(std::integral_constant<int, 1>{}, mblk); break;
+      case 2: walk(std::integral_constant<int, 2>{}, mblk); break;
+      case 3: walk(std::integral_constant<int, 3>{}, mblk); break;
+      case 4: walk(std::integral_constant<int, 4>{}, mblk); break;
+      case 5: walk(std::integral_constant<int, 5>{}, mblk); break;
+      case 6: walk(std::integral_constant<int, 6>{}, mblk); break;
+      case 7: walk(std::integral_constant<int, 7>{}, mblk); break;
+      default: walk(std::integral_constant<int, 8>{}, mblk); break;
+    }
+  };
+  if (S.mblk == 1) pick(std::integral_constant<int, 1>{});
+  else pick(std::integral_constant<int, 2>{});
+}
+
 // Second pass of a launch that split K across workgroups: adds the parts of every row of every tile in a fixed
 // order and finishes the row exactly as the one-pass kernel does (scale, round, add or overwrite).
 template <typename D>
@@ -294,6 +378,38 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_parts_kernel(
       E* Vp = static_cast<E*>(proj == 0 ? grp.v[0] : (proj == 1 ? grp.v[1] : (proj == 2 ? grp.v[2] : grp.v[3])));
       update4<D>(accumulate_into_v != 0, Vp + static_cast<int64_t>(row) * r + (col - proj * r), sum * scale);
     }
+  }
+}
+
+// The same for a launch of several groups, whose sums are numbered tile by tile.
+template <typename D>
+__global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_parts_kernel(const ShrinkLaunch batch, int count,
+                                                                               int num_tokens, int kparts, float scale,
+                                                                               int accumulate_into_v) {
+  using E = typename D::E;
+  int tile = static_cast<int>(blockIdx.x);
+  const ShrinkSlot& S = batch.p[shrink_slot_of(batch.tile_end, count, tile)];
+  const ShrinkGroup& grp = S.grp;
+  const int r = grp.rank, R = S.nb * 16, rows = S.mblk * 16;
+  RowTile rt;
+  if (!get_row_tile(TileList{S.tiles, S.num_tiles, rows}, S.s_start, S.s_end, S.num_segments, num_tokens, rows, tile, rt)) return;
+  // a plan's tile whose segment has no stack was not multiplied
+  for (int p = 0; p < grp.count; ++p)
+    if (grp.w[p][rt.seg] == 0) return;
+  const int n4 = grp.count * r / 4;
+  const int n = (rt.row_end - rt.row0) * n4;
+  for (int i = threadIdx.x; i < n; i += kLdsThreads) {
+    const int row = i / n4;
+    const int col = (i - row * n4) * 4;
+    f32x4 sum{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < kparts; ++p) {
+      const f32x4 part = *reinterpret_cast<const f32x4*>(
+          S.partials + ((static_cast<int64_t>(p) * S.num_tiles + tile) * rows + row) * R + col);
+      sum[0] += part[0]; sum[1] += part[1]; sum[2] += part[2]; sum[3] += part[3];
+    }
+    const int proj = col / r;
+    E* Vp = static_cast<E*>(grp.v[proj]);
+    update4<D>(accumulate_into_v != 0, Vp + static_cast<int64_t>(rt.row0 + row) * r + (col - proj * r), sum * scale);
   }
 }
 
@@ -399,6 +515,19 @@ static LdsLaunch lds_launch_shape(const SgmvArgs& a, size_t room) {
   return l;
 }
 
+// The call's projections; one projection makes a group of its own.
+static ShrinkGroup whole_group(const SgmvArgs& a) {
+  ShrinkGroup grp = a.group;
+  if (grp.count <= 1) {
+    grp = ShrinkGroup{};
+    grp.v[0] = a.y;
+    grp.w[0] = a.w_ptrs;
+    grp.count = 1;
+    grp.rank = a.d_out;
+  }
+  return grp;
+}
+
 template <typename D, int NB, int MBLK, bool KSPLIT>
 static hipError_t launch_lds_m(const SgmvArgs& a, const LdsLaunch& l, hipStream_t stream) {
   constexpr int kStageBytes = (MBLK + NB) * 16 * kLdsRowBytes;
@@ -423,14 +552,7 @@ static hipError_t launch_lds_m(const SgmvArgs& a, const LdsLaunch& l, hipStream_
   // lorax_init has raised the dynamic LDS limit of every instantiation; a caller that skipped it gets it here.
   if (hipError_t e = raise_lds_limit<D, NB, MBLK, KSPLIT>(); e != hipSuccess) return e;
   dim3 grid(static_cast<unsigned>(kparts > 1 ? wgs : (tiles < (1 << 20) ? tiles : (1 << 20))));
-  ShrinkGroup grp = a.group;
-  if (grp.count <= 1) {
-    grp = ShrinkGroup{};
-    grp.v[0] = a.y;
-    grp.w[0] = a.w_ptrs;
-    grp.count = 1;
-    grp.rank = a.d_out;
-  }
+  const ShrinkGroup grp = whole_group(a);
   const TileList plan{l.planned ? a.tiles : nullptr, l.planned ? a.num_tiles : 0, l.rows_per_tile};
   const int rotate = (tuning().shrink_no_rotate || fixed_order_shrink()) ? 0 : 1;
   hipLaunchKernelGGL(kernel, grid, dim3(kLdsThreads), lds_bytes, stream, grp, static_cast<const typename D::E*>(a.x),
@@ -493,6 +615,110 @@ static hipError_t launch_lds_dtype(const SgmvArgs& a, hipStream_t stream) {
   }
 }
 
+template <typename D>
+static hipError_t raise_groups_lds_limit() {
+  static std::atomic<bool> configured[64] = {};
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  if (device >= 0 && device < 64 && configured[device].load(std::memory_order_acquire)) return hipSuccess;
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(sgmv_shrink_groups_kernel<D>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMaxBytes);
+  if (e == hipSuccess && device >= 0 && device < 64) configured[device].store(true, std::memory_order_release);
+  return e;
+}
+
+template <typename D>
+static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStream_t stream) {
+  const SgmvArgs& a = groups[0];
+  const int nst = a.d_in / kLdsKc;
+  ShrinkLaunch b{};
+  int64_t tiles = 0;
+  double tile_us = 0, sum_bytes = 0;  // of all tiles: time at a CU's 50 KB/us, fp32 sums of one part
+  int stage_max = 0;
+  for (int i = 0; i < count; ++i) {
+    const SgmvArgs& g = groups[i];
+    ShrinkSlot& s = b.p[i];
+    s.grp = whole_group(g);
+    s.s_start = g.s_start;
+    s.s_end = g.s_end;
+    s.tiles = g.tiles;
+    s.num_segments = g.num_segments;
+    s.num_tiles = g.num_tiles;
+    s.nb = (g.d_out + 15) / 16;
+    s.mblk = (g.tile_rows + 15) / 16;
+    tiles += s.num_tiles;
+    const int stage = (s.mblk + s.nb) * 16 * kLdsRowBytes;
+    stage_max = stage > stage_max ? stage : stage_max;
+    tile_us += s.num_tiles * static_cast<double>(stage) * nst / 50e3;
+    sum_bytes += static_cast<double>(s.num_tiles) * s.mblk * 16 * s.nb * 16 * sizeof(float);
+  }
+  // K parts: a CU streams about 50 KB/us, so the launch takes as long as the workgroups of its busiest CU; parts are
+  // worth their second launch (4 us, and the sums written and read) where they even that out.
+  int kparts = 1;
+  if (!fixed_order_shrink()) {
+    double best = 0;
+    for (int k = 1; k <= 8 && k <= (nst >= 16 ? nst / 8 : 1); ++k) {
+      if (k > 1 && k * sum_bytes > static_cast<double>(kPartialBytes)) break;
+      const double us = static_cast<double>((tiles * k + 255) / 256) * (tile_us / tiles) / k + (k > 1 ? 4.0 + 2e-6 * k * sum_bytes / 2.0 : 0.0);
+      if (k == 1 || us < best) best = us, kparts = k;
+    }
+    if (tuning().shrink_ksplit > 0 && tuning().shrink_ksplit <= nst && tuning().shrink_ksplit * sum_bytes <= static_cast<double>(kPartialBytes))
+      kparts = tuning().shrink_ksplit;
+  }
+  const int64_t wgs = tiles * kparts;
+  // stage buffers as in launch_lds_m, but never less than two stages of the largest group
+  int budget = wgs <= 256 ? 150 * 1024 : (wgs <= 768 ? 50 * 1024 : 76 * 1024);
+  if (tuning().shrink_lds_kb > 0) budget = tuning().shrink_lds_kb * 1024;
+  if (budget < 2 * stage_max) budget = 2 * stage_max;
+  int lds_bytes = 0;
+  int64_t wg = 0, tile = 0;
+  float* sums = a.partials;
+  for (int i = 0; i < count; ++i) {
+    ShrinkSlot& s = b.p[i];
+    const int stage = (s.mblk + s.nb) * 16 * kLdsRowBytes;
+    const int red = 4 * s.mblk * s.nb * 1024;
+    s.stages = budget / stage < kLdsMaxStages ? budget / stage : kLdsMaxStages;
+    if (s.stages * stage > lds_bytes) lds_bytes = s.stages * stage;
+    if (red > lds_bytes) lds_bytes = red;
+    s.partials = sums;
+    sums += static_cast<int64_t>(kparts) * s.num_tiles * s.mblk * 16 * s.nb * 16;
+    wg += static_cast<int64_t>(s.num_tiles) * kparts;
+    tile += s.num_tiles;
+    b.wg_end[i] = static_cast<int>(wg);
+    b.tile_end[i] = static_cast<int>(tile);
+  }
+  static_assert(2 * (2 + 8) * 16 * kLdsRowBytes <= kLdsMaxBytes, "two stages of the largest group must fit in LDS");
+  if (hipError_t e = raise_groups_lds_limit<D>(); e != hipSuccess) return e;
+  const int rotate = (tuning().shrink_no_rotate || fixed_order_shrink()) ? 0 : 1;
+  hipLaunchKernelGGL(sgmv_shrink_groups_kernel<D>, dim3(static_cast<unsigned>(wgs)), dim3(kLdsThreads), lds_bytes, stream, b,
+                     count, static_cast<const typename D::E*>(a.x), static_cast<int>(a.num_tokens), a.d_in, a.layer_idx,
+                     a.scale, a.accumulate, kparts, rotate);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || kparts == 1) return e;
+  hipLaunchKernelGGL(sgmv_shrink_groups_parts_kernel<D>, dim3(static_cast<unsigned>(tiles)), dim3(kLdsThreads), 0, stream, b,
+                     count, static_cast<int>(a.num_tokens), kparts, a.scale, a.accumulate);
+  return hipGetLastError();
+}
+
+bool sgmv_shrink_groups_applies(const SgmvArgs* groups, int count) {
+  if (count < 2 || count > kMaxShrinkSlots || groups[0].partials == nullptr || groups[0].partial_bytes < kPartialBytes ||
+      tuning().shrink_mb != 0 || tuning().shrink_lds < 0)
+    return false;
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) {
+    const SgmvArgs& g = groups[i];
+    if (!sgmv_shrink_lds_applies(g) || g.tiles == nullptr || g.num_tiles < 1 || g.tile_rows < 1 || g.tile_rows > 32) return false;
+    tiles += g.num_tiles;
+  }
+  return tiles < (1 << 20);
+}
+
+hipError_t launch_sgmv_shrink_groups(const SgmvArgs* groups, int count, hipStream_t stream) {
+  return groups[0].dtype == LORAX_F16 ? launch_groups_dtype<F16>(groups, count, stream)
+                                      : launch_groups_dtype<BF16>(groups, count, stream);
+}
+
 // Every instantiation launch_lds_nb can reach, for the per-device set-up: the same case analysis as the launchers.
 template <typename D, int NB>
 static hipError_t raise_lds_limits_nb() {
@@ -522,6 +748,7 @@ static hipError_t raise_lds_limits_dtype() {
   also(raise_lds_limits_nb<D, 6>());
   also(raise_lds_limits_nb<D, 7>());
   also(raise_lds_limits_nb<D, 8>());
+  also(raise_groups_lds_limit<D>());
   return e;
 }
 hipError_t configure_sgmv_shrink_lds() {

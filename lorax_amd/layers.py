@@ -208,7 +208,7 @@ class LoraLinear(nn.Module):
         projections and ranks are one launch.  (The reference issues a shrink and an expand per projection and rank,
         utils/layers.py:121-143.)"""
         rows = input.size(0)
-        expands, short_shrinks, short_expands = [], [], []
+        shrinks, expands, short_shrinks, short_expands = [], [], [], []
         for group in groups:
             r = group[0][0].rank
             if _native.sgmv_lora_fits(r, input.size(1), rows, max(width for _, _, width in group)):
@@ -242,11 +242,8 @@ class LoraLinear(nn.Module):
                 step = MAX_SGMV_SHRINK_PROBLEMS  # the streaming shrink of a short batch takes any ranks
             # (no long segment at all: the per-token launches do the whole update)
             for i in range(0, len(group) if n_long > 0 else 0, step):
-                _native.sgmv_shrink_multi(
-                    vs[i : i + step], input, [rs.lora_a_t_ptr[:n_long] for rs, _, _ in group[i : i + step]],
-                    starts, ends, get_shrink_scratch(input.device), self.layer_id, 1.0, False,
-                    first.shrink_tiles if planned else None,
-                )
+                shrinks.append((vs[i : i + step], [rs.lora_a_t_ptr[:n_long] for rs, _, _ in group[i : i + step]], starts, ends,
+                                first.shrink_tiles if planned else None))
             for v, plan, (rs, start, width) in zip(vs, plans, group):
                 if n_long > 0:
                     expands.append((result, v, rs.lora_b_t_ptr[:n_long], starts, ends, start, width,
@@ -255,6 +252,15 @@ class LoraLinear(nn.Module):
                 if split:
                     short_shrinks.append(((v, input, None, None, 0, None), plan))
                     short_expands.append(((result, v, None, None, start, width), plan))
+        if len(shrinks) == 1:
+            (v, tables, starts, ends, tiles), = shrinks
+            _native.sgmv_shrink_multi(v, input, tables, starts, ends, get_shrink_scratch(input.device), self.layer_id, 1.0, False,
+                                      tiles)
+        else:
+            step = _native.MAX_SGMV_SHRINK_GROUPS
+            for i in range(0, len(shrinks), step):
+                _native.sgmv_shrink_groups(shrinks[i : i + step], input, get_shrink_scratch(input.device), self.layer_id, 1.0,
+                                           False)
         batch = _native.MAX_BGMV_PROBLEMS
         for i in range(0, len(short_shrinks), batch):
             chunk = short_shrinks[i : i + batch]
