@@ -472,14 +472,25 @@ def bgmv_stacked(y, x, jobs, plan, scale=1.0) -> None:
 FUSED_BGMV_RANKS = (8, 16)
 
 
-def bgmv_lora_fits(rank: int, h_in: int, h_out: int) -> bool:
+FEW_CHUNKS = {8: 64, 16: 16}  # plan records up to which wide projections run fused, by rank
+
+
+def bgmv_lora_fits(rank: int, h_in: int, h_out: int, few_chunks: bool = False) -> bool:
     """True where the single-launch shrink+expand (lorax_bgmv_lora_multi) is the better choice: the adapter's
     A slab is small (<= 128 KiB) and one workgroup covers all output columns of the projection (4096 at
     rank 8, 2048 at rank 16), so no column slice has to repeat the shrink. Wider or deeper projections are
-    faster as a shrink launch plus an expand launch."""
-    if rank not in FUSED_BGMV_RANKS:
+    faster as a shrink launch plus an expand launch - unless the batch has few routing records (`few_chunks`: all jobs of one
+    rank, FEW_CHUNKS records at most): then the repeated shrinks run on idle CUs and the second launch is what costs.  A
+    Mistral-7B block at rank 16, fused against two launches: 18.6 and 23.5 us per layer at one record, 29 and 33 at 10, 39.5
+    both at 20, 61 and 58 at 43; at rank 8 16 and 18 us, 34.0 and 34.3 at 43, 53.2 and 53.0 at 84."""
+    if rank not in FUSED_BGMV_RANKS or rank * h_in * 2 > 128 * 1024:
         return False
-    return rank * h_in * 2 <= 128 * 1024 and h_out <= (256 // (rank // 8)) * 16
+    return h_out <= (256 // (rank // 8)) * 16 or (few_chunks and h_out <= 16384)
+
+
+def few_chunks(ranks, plan_sizes) -> bool:
+    """Whether a batch's jobs (their ranks and numbers of routing records) count as few in bgmv_lora_fits."""
+    return len(set(ranks)) == 1 and all(n <= FEW_CHUNKS.get(r, 0) for r, n in zip(ranks, plan_sizes))
 
 
 def _check_stack(stack, x) -> None:

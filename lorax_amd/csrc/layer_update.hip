@@ -12,6 +12,7 @@ constexpr int kMaxJobs = 256;        // (projection, rank group) pairs of one ca
 constexpr int kMaxKernelRank = 128;
 constexpr int64_t kMaxBgmvRows = 65535;  // rows of a BGMV launch and records of one routing plan
 constexpr int64_t kShortBatchRows = 512;  // largest batch of the streaming shrink and of lorax_sgmv_lora_multi at rank 8
+constexpr int kFewChunks8 = 64, kFewChunks16 = 16;  // plan records up to which wide projections run fused, by rank
 constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 (measured: _native.sgmv_lora_fits)
 
 struct Job {
@@ -37,10 +38,12 @@ struct Call {
 };
 
 // The single-launch update pays where the A slab is small and, in decode, one workgroup covers the projection's
-// columns (the rules of _native.bgmv_lora_fits and sgmv_lora_fits, where they are explained).
+// columns or the batch has few records (the rules of _native.bgmv_lora_fits and sgmv_lora_fits, where they are explained).
 bool fused_rank(int r, int h_in) { return (r == 8 || r == 16) && r * h_in * 2 <= 128 * 1024; }
-bool decode_fused(const Job& j, int h_in) {
-  return fused_rank(j.g->rank, h_in) && j.width <= (256 / (j.g->rank / 8)) * 16;
+bool decode_fused(const Job& j, int h_in, bool one_rank) {
+  const int r = j.g->rank;
+  return fused_rank(r, h_in) && (j.width <= (256 / (r / 8)) * 16 ||
+                                 (one_rank && j.width <= 16384 && j.g->num_chunks <= (r == 8 ? kFewChunks8 : kFewChunks16)));
 }
 
 const void* at(const Call& c, int64_t off) { return c.tables + off; }
@@ -65,7 +68,9 @@ int bgmv_jobs(const Call& c, const Job* const* jobs, int count, bool shrink) {
 
 int decode(const Call& c, Job* const* jobs, int count) {
   bool fused = true;
-  for (int i = 0; i < count; ++i) fused = fused && decode_fused(*jobs[i], c.h_in);
+  bool one_rank = true;
+  for (int i = 0; i < count; ++i) one_rank = one_rank && jobs[i]->g->rank == jobs[0]->g->rank;
+  for (int i = 0; i < count; ++i) fused = fused && decode_fused(*jobs[i], c.h_in, one_rank);
   if (fused) {
     for (int r : {8, 16}) {
       lorax_bgmv_problem_t p[lorax::kMaxFusedBgmvProblems];

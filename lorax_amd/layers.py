@@ -280,9 +280,9 @@ class LoraLinear(nn.Module):
         """The decode launches of forward_layer_types for jobs that touch disjoint elements of `result`:
         decode_jobs maps (wave, rank) to [(rank_segments, start, width)]."""
         jobs = [(r, rs, start, width) for (_, r), rank_jobs in decode_jobs.items() for rs, start, width in rank_jobs]
-        all_fused = bool(jobs) and not tensor_parallel and all(
-            rs.plan is not None and _native.bgmv_lora_fits(r, input.size(1), width) for r, rs, _, width in jobs
-        )
+        planned = bool(jobs) and not tensor_parallel and all(rs.plan is not None for _, rs, _, _ in jobs)
+        few = planned and _native.few_chunks([r for r, _, _, _ in jobs], [rs.plan.size(0) for _, rs, _, _ in jobs])
+        all_fused = planned and all(_native.bgmv_lora_fits(r, input.size(1), width, few) for r, _, _, width in jobs)
         if all_fused:
             step = _native.MAX_FUSED_BGMV_PROBLEMS
             for r in sorted({r for _, r in decode_jobs}):

@@ -211,8 +211,9 @@ def bgmv_lora_slices(
         assert a.dtype == inputs.dtype and b.dtype == inputs.dtype
         assert inputs.size(1) == a.size(-1) and a.size(-2) == b.size(-1) and slice_size == b.size(-2)
         jobs.append((a, b, a.size(-2), slice_offset, slice_size))
+    few = plan is not None and _native.few_chunks([r for _, _, r, _, _ in jobs], [plan.size(0)] * len(jobs))
     if plan is not None and scaling == 1.0 and all(
-            _native.bgmv_lora_fits(r, inputs.size(1), size) for _, _, r, _, size in jobs):
+            _native.bgmv_lora_fits(r, inputs.size(1), size, few) for _, _, r, _, size in jobs):
         step = _native.MAX_FUSED_BGMV_PROBLEMS
         for rank in sorted({r for _, _, r, _, _ in jobs}):
             same = [j for j in jobs if j[2] == rank]

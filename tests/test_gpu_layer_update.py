@@ -29,6 +29,10 @@ CASES = {
     "one row": ([16], 512, [512, 128, 128], False, [1]),
     "fused decode": ([8, 16], 512, [512, 128, 128], False, [1] * 23),
     "decode of four ranks, two launches of problems": ([8, 16, 32, 64, 24, 40], 512, [512, 2048, 128], False, [1] * 37),
+    "wide projections, 16 records of rank 16": ([16] * 16, 1024, [14336, 128, 128], False, [1] * 24),
+    "wide projections, 17 records of rank 16": ([16] * 17, 1024, [14336, 128, 2056], False, [1] * 26),
+    "wide projections, rank 8": ([8] * 3, 1024, [16384, 16392, 128], False, [1] * 9),
+    "wide projections, two ranks": ([8, 16], 1024, [14336, 128, 4104], False, [1] * 5),
     "short prefill, rank 16": ([16], 1024, [512, 128, 128], True, [3, 1, 40, 17]),
     "prefill of four ranks": ([8, 16, 32, 64], 1024, [512, 136, 128], True, [200, 90, 1, 300, 33]),
     "prefill with decode rows": ([16, 32], 1024, [512, 128, 128], True, [400, 300] + [1] * 90),
@@ -69,6 +73,30 @@ def test_layer_update_matches_the_general_path(case, dtype):
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
     assert not torch.equal(outs[0], y0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank,h_out,adapters,tokens", [(16, 14336, 1, 1), (16, 16384, 16, 16), (16, 2056, 5, 23), (8, 16384, 64, 64),
+                                                       (8, 4104, 2, 7)])
+def test_few_decode_rows_of_wide_projections(rank, h_out, adapters, tokens, dtype):
+    """The single-launch update of wide projections of a small decode batch against fp64."""
+    gen = torch.Generator().manual_seed(h_out + tokens)
+    weights = {"up_proj": _layer([rank] * adapters, 4096, h_out, dtype, gen)}
+    owners = [1 + i % adapters for i in range(tokens)]
+    meta = make_meta(owners, torch.device("cuda", 0))
+    data = AdapterBatchData.from_meta(meta, weights)
+    x = torch.randn((tokens, 4096), generator=gen).to(dtype).cuda()
+    y0 = torch.randn((tokens, h_out), generator=gen).to(dtype).cuda()
+    y = y0.clone()
+    TensorParallelMultiAdapterLinear.load(lambda _: y, 1, ["up_proj"], [h_out])(x, data)
+    want = y0.double()
+    for t, a in enumerate(owners):
+        w = weights["up_proj"].adapter_weights[a]
+        v = (x[t].double() @ w.weights_a_t[1].double().t()).to(dtype).double()
+        want[t] += (v @ w.weights_b_t[1].double().t()).to(dtype).double()
+    # roundings of v, of the update and of the sum, each at most half an ulp, and fp32 sums
+    eps = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    assert torch.linalg.norm(y.double() - want) <= 2 * eps * torch.linalg.norm(want)
 
 
 def test_layer_update_leaves_other_operands_to_the_general_path():
