@@ -497,7 +497,9 @@ int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t nu
     return fail(LORAX_EINVAL, "num_groups=%d (at most %d per call)", num_groups, kMaxGroups);
   if (num_groups > 0 && groups == nullptr) return fail(LORAX_EINVAL, "null pointer argument (groups)");
   const int rows_max = tuning().shrink_rows_max != 0 ? tuning().shrink_rows_max : 512;
-  // one launch: planned tiles of a batch past the streaming kernel's range, stacked ranks of one A tile each
+  // one launch: planned tiles of a batch past the streaming kernel's range, stacked ranks of one A tile each.  The
+  // kernels store four columns of v at a time and take a store's projection from its first column, so each projection's
+  // own rank has to be a multiple of 8, not only their sum; other ranks go to the calls below, which refuse them.
   SgmvArgs args[kMaxGroups];
   int count = 0;
   bool together = num_groups > 1 && num_tokens > rows_max && num_tokens <= INT32_MAX / 2 && h_in > 0 && layer_idx >= 0 &&
@@ -506,7 +508,7 @@ int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t nu
   for (int i = 0; i < num_groups && together; ++i) {
     const lorax_sgmv_shrink_group_t& g = groups[i];
     together = g.num_problems >= 1 && g.num_problems <= kMaxShrinkGroup && g.problems != nullptr && g.r >= 8 &&
-               g.num_problems * g.r <= kMaxRank && g.s_start != nullptr && g.s_end != nullptr && g.num_segments > 0 &&
+               g.r % 8 == 0 && g.r <= kMaxRank / g.num_problems && g.s_start != nullptr && g.s_end != nullptr && g.num_segments > 0 &&
                g.tiles != nullptr && g.tiles->tiles != nullptr;
     if (!together) break;
     SgmvArgs& a = args[count];

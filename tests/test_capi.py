@@ -102,6 +102,25 @@ def test_sgmv_shrink_multi_validation():
     assert f(two, 2, P, P, P, 2, 1000, 4096, 64, 0, 1.0, 1, P, big, ctypes.byref(empty), 1, None) == OK
 
 
+def _shrink_groups(rank, num_problems, num_groups, tile_rows=16):
+    problems = (_native.SgmvShrinkProblem * num_problems)(*[_native.SgmvShrinkProblem(P, P)] * num_problems)
+    tiles = _native.SgmvTiles(P, 40, tile_rows)
+    group = _native.SgmvShrinkGroup(problems, num_problems, rank, P, P, 2, ctypes.addressof(tiles))
+    return (_native.SgmvShrinkGroup * num_groups)(*[group] * num_groups), (problems, tiles)
+
+
+@pytest.mark.parametrize("rank", [10, 12, 18, 30, 4, 136])
+@pytest.mark.parametrize("num_problems", [2, 4])
+def test_sgmv_shrink_groups_refuses_the_ranks_that_shrink_multi_refuses(rank, num_problems):
+    """A rank that is no multiple of 8 is refused whatever the summed rank of the group (two problems of rank 12 and four
+    of rank 10 or 18 have a sum that is one): a store of four columns would cross into the next row of v."""
+    f = _native.lib().lorax_sgmv_shrink_groups
+    for num_groups in (1, 2):
+        groups, _keep = _shrink_groups(rank, num_problems, num_groups)
+        assert f(groups, num_groups, P, 1000, 4096, 0, 1.0, 0, P, 8 * 1024 * 1024, 1, None) == ENOKERNEL
+        assert "No suitable kernel" in _err()
+
+
 def test_sgmv_lora_multi_validation():
     f = _native.lib().lorax_sgmv_lora_multi
     one = (_native.SgmvLoraProblem * 1)(_native.SgmvLoraProblem(P, P, P, 0, 4096, 4096))
