@@ -450,7 +450,7 @@ typedef struct lorax_table_group {
   int32_t expand_tile_rows;
   int32_t segments_id;  /* use_sgmv = 1: equal for groups whose segment bounds hold the same values
                            (their shrinks can share one pass over x); else -1                     */
-  int32_t reserved;
+  int32_t num_tokens;   /* rows of the batch the tables were built for; a routing plan names rows below it */
 } lorax_table_group_t;
 
 int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
@@ -472,7 +472,8 @@ int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
  *   tmp, tmp_bytes      device, LORAX_SHRINK_TMP_BYTES (read by prefill tables only)
  *   device              the GPU the pointers live on; made current for the call
  * Returns LORAX_EROUTE, before anything is launched, for tables that need a path of the caller's own (ranks that are
- * no multiple of 8, shapes that only the reference's prefill layouts serve).
+ * no multiple of 8, shapes that only the reference's prefill layouts serve), and LORAX_EINVAL for a num_tokens below
+ * that of a table with a routing plan, whose records may name rows that x and y do not have.
  */
 typedef struct lorax_layer_slice {
   int32_t layer_type;

@@ -85,7 +85,7 @@ class TableGroup(ctypes.Structure):
                 ("shrink_tiles_off", _c.c_int64), ("expand_tiles_off", _c.c_int64),
                 ("num_shrink_tiles", _c.c_int32), ("shrink_tile_rows", _c.c_int32),
                 ("num_expand_tiles", _c.c_int32), ("expand_tile_rows", _c.c_int32),
-                ("segments_id", _c.c_int32), ("reserved", _c.c_int32)]
+                ("segments_id", _c.c_int32), ("num_tokens", _c.c_int32)]
 
 
 class LayerSlice(ctypes.Structure):

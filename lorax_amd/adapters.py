@@ -193,7 +193,7 @@ class RankSegments:
                  plan: Optional[torch.Tensor] = None, lora_a_t_ptr: Optional[torch.Tensor] = None,
                  lora_b_t_ptr: Optional[torch.Tensor] = None, segments_key=None,
                  num_long_segments: Optional[int] = None, short_plan: Optional[torch.Tensor] = None,
-                 shrink_tiles=None, expand_tiles=None):
+                 shrink_tiles=None, expand_tiles=None, num_rows: Optional[int] = None):
         self.rank = rank
         self._lora_a_ptr = lora_a_ptr  # a tensor, or a function that builds it
         self._lora_b_ptr = lora_b_ptr
@@ -226,6 +226,9 @@ class RankSegments:
         # the device
         self.shrink_tiles = shrink_tiles
         self.expand_tiles = expand_tiles
+        # rows of the batch that `plan` / `short_plan` were built for: their records may name any row below it, so an
+        # input of fewer rows cannot be served from them; None = unknown
+        self.num_rows = num_rows
 
     @property
     def lora_a_ptr(self) -> Optional[torch.Tensor]:
@@ -522,6 +525,7 @@ class BatchLoraWeights(BatchAdapterWeights):
                 short_plan=short_plan,
                 shrink_tiles=shrink_tiles,
                 expand_tiles=expand_tiles,
+                num_rows=meta.adapter_indices.size(0),
             )
 
         return cls(
@@ -807,6 +811,7 @@ class _TableViews:
                     expand_tiles=_native.TilePlan(
                         dev32[g.expand_tiles_off // 4 : g.expand_tiles_off // 4 + 4 * g.num_expand_tiles].view(-1, 4),
                         g.expand_tile_rows) if g.expand_tiles_off >= 0 else None,
+                    num_rows=T,
                 )
             else:
                 rank_data[g.rank] = RankSegments(
@@ -820,6 +825,7 @@ class _TableViews:
                     indices=dev64[g.indices_off // 8 : g.indices_off // 8 + T],
                     plan=dev64[g.plan_off // 8 : g.plan_off // 8 + g.num_chunks * BGMV_PLAN_WORDS].view(
                         g.num_chunks, BGMV_PLAN_WORDS),
+                    num_rows=T,
                 )
         return rank_data
 

@@ -153,6 +153,7 @@ extern "C" int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t 
       desc.rank = group_of_rank[g];
       desc.use_sgmv = use_sgmv ? 1 : 0;
       desc.num_segments = n;
+      desc.num_tokens = static_cast<int32_t>(num_tokens);
       desc.a_ptr_off = pack.reserve(static_cast<int64_t>(n) * 8);
       desc.b_ptr_off = pack.reserve(static_cast<int64_t>(n) * 8);
       if (int64_t* a = pack.at<int64_t>(desc.a_ptr_off)) {

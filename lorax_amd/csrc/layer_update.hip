@@ -46,6 +46,11 @@ bool decode_fused(const Job& j, int h_in, bool one_rank) {
                                  (one_rank && j.width <= 16384 && j.g->num_chunks <= (r == 8 ? kFewChunks8 : kFewChunks16)));
 }
 
+// A short prefill batch runs shrink and expand of a rank's projections in one launch over the segments.
+bool prefill_fused(int r, int h_in, int64_t rows, int widest) {
+  return fused_rank(r, h_in) && rows <= (r == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= 16384;
+}
+
 const void* at(const Call& c, int64_t off) { return c.tables + off; }
 
 lorax_bgmv_problem_t plan_problem(const Call& c, const Job& j, void* y, const void* x, int64_t y_offset, int64_t y_stride,
@@ -118,7 +123,7 @@ int prefill(const Call& c, Job* const* jobs, int count) {
       widest = jobs[end]->width > widest ? jobs[end]->width : widest;
     const int32_t* starts = static_cast<const int32_t*>(at(c, g.starts_off));
     const int32_t* ends = static_cast<const int32_t*>(at(c, g.ends_off));
-    if (fused_rank(g.rank, c.h_in) && c.rows <= (g.rank == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= 16384) {
+    if (prefill_fused(g.rank, c.h_in, c.rows, widest)) {
       for (int k = i; k < end; k += lorax::kMaxSgmvLoraProblems) {
         lorax_sgmv_lora_problem_t p[lorax::kMaxSgmvLoraProblems];
         int n = 0;
@@ -240,6 +245,16 @@ extern "C" int lorax_layer_update(const lorax_table_group_t* groups, int32_t num
   if (num_groups == 0 || num_slices == 0 || num_tokens == 0) return LORAX_OK;
   if (groups == nullptr || tables == nullptr || slices == nullptr || y == nullptr || x == nullptr || v == nullptr)
     return lorax::report_error(LORAX_EINVAL, "null pointer argument (groups, tables, slices, y, x or v)");
+  // The segment kernels clamp their rows to num_tokens; the per-token kernels take them from the plan's records.
+  int widest = 0;
+  for (int s = 0; s < num_slices; ++s) widest = slices[s].width > widest ? slices[s].width : widest;
+  for (int s = 0; s < num_slices; ++s)
+    for (int i = 0; i < num_groups; ++i) {
+      const lorax_table_group_t& g = groups[i];
+      if (g.layer_type != slices[s].layer_type || g.plan_off < 0 || num_tokens >= g.num_tokens) continue;
+      if (g.use_sgmv == 0 || !prefill_fused(g.rank, h_in, num_tokens, widest))
+        return lorax::report_error(LORAX_EINVAL, "layer update: x and y have fewer rows than the batch of the routing tables");
+    }
   const Call c{static_cast<const char*>(tables), y, y_stride, x, num_tokens, h_in, layer_idx, tmp, tmp_bytes, dtype, stream};
   int current = 0;
   if (hipError_t e = hipGetDevice(&current)) return lorax::report_error(LORAX_ELAUNCH, hipGetErrorString(e));

@@ -55,6 +55,14 @@ class SingleProcessGroup:
         return 0
 
 
+def _check_plan_rows(rows: int, segments) -> None:
+    """The per-token kernels take row numbers from the plans' records as they are."""
+    for rs in segments:
+        if rs.num_rows is not None and rows < rs.num_rows:
+            raise RuntimeError(f"the input has {rows} rows, fewer than the {rs.num_rows} of the batch that its routing plan "
+                               "was built for")
+
+
 class LoraLinear(nn.Module):
     def __init__(self, base_layer, layer_id: int, process_group=None):
         super().__init__()
@@ -231,6 +239,8 @@ class LoraLinear(nn.Module):
             # take the whole tables, which still list every segment)
             split = (all(p is not None for p in plans) and rows <= _native.MAX_BGMV_TOKENS
                      and all(p.size(0) <= _native.MAX_BGMV_TOKENS for p in plans))
+            if split:
+                _check_plan_rows(rows, [rs for rs, _, _ in group])
             n_long = first.num_long_segments if split else first.segment_starts.numel()
             starts, ends = first.segment_starts[:n_long], first.segment_ends[:n_long]
             # the tables' row-tile plans cover their first num_long_segments entries
@@ -281,6 +291,7 @@ class LoraLinear(nn.Module):
         decode_jobs maps (wave, rank) to [(rank_segments, start, width)]."""
         jobs = [(r, rs, start, width) for (_, r), rank_jobs in decode_jobs.items() for rs, start, width in rank_jobs]
         planned = bool(jobs) and not tensor_parallel and all(rs.plan is not None for _, rs, _, _ in jobs)
+        _check_plan_rows(input.size(0), [rs for _, rs, _, _ in jobs if rs.plan is not None])
         few = planned and _native.few_chunks([r for r, _, _, _ in jobs], [rs.plan.size(0) for _, rs, _, _ in jobs])
         all_fused = planned and all(_native.bgmv_lora_fits(r, input.size(1), width, few) for r, _, _, width in jobs)
         if all_fused:

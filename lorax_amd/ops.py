@@ -211,6 +211,9 @@ def bgmv_lora_slices(
         assert a.dtype == inputs.dtype and b.dtype == inputs.dtype
         assert inputs.size(1) == a.size(-1) and a.size(-2) == b.size(-1) and slice_size == b.size(-2)
         jobs.append((a, b, a.size(-2), slice_offset, slice_size))
+    if plan is not None and lora_indices_tensor.size(0) > inputs.size(0):
+        raise RuntimeError(f"the input has {inputs.size(0)} rows, fewer than the {lora_indices_tensor.size(0)} of the batch "
+                           "that its routing plan was built for")
     few = plan is not None and _native.few_chunks([r for _, _, r, _, _ in jobs], [plan.size(0)] * len(jobs))
     if plan is not None and scaling == 1.0 and all(
             _native.bgmv_lora_fits(r, inputs.size(1), size, few) for _, _, r, _, size in jobs):

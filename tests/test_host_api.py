@@ -540,3 +540,71 @@ def test_prefill_batches_beyond_the_per_token_kernels_range_stay_on_the_segment_
     lin.forward_layer_type(y, x, data, "q_proj", 0, h)
     n_all = rd.segment_starts.numel()
     assert calls == [("shrink", n_all), ("expand", n_all)]  # beyond it: every segment on the segment kernels
+
+
+def _decode_rows_in_a_prefill_batch(rank, h=128):
+    """A prefill batch with forty one-row segments behind a long one: their rows get a routing plan."""
+    from lorax_amd.adapters import LayerAdapterWeights, LoraConfig, LoraWeights
+    from lorax_amd.synthetic import make_meta
+
+    layer = LayerAdapterWeights()
+    for idx in range(6):
+        layer.add_adapter(idx, LoraWeights([torch.randn(h, rank)], [torch.randn(rank, h)], LoraConfig(r=rank)))
+    indices = [0] * 40 + [a for i in range(40) for a in (1 + i % 5, -1)]
+    return layer, make_meta(indices, torch.device("cpu"))
+
+
+@pytest.mark.parametrize("prefill,rank,rows,refused", [
+    (True, 32, 119, True), (True, 32, 1, True), (True, 32, 120, False), (True, 32, 200, False),
+    (True, 8, 119, False),  # one launch over the segments, which the kernel clamps: the plan is not read
+    (False, 32, 119, True), (False, 8, 119, True), (False, 8, 120, False),
+])
+def test_layer_update_refuses_fewer_rows_than_its_routing_plan_names(prefill, rank, rows, refused):
+    """lorax_layer_update (the C entry; without a GPU a call that passes the check ends at the device query)."""
+    import numpy as np
+
+    from lorax_amd import _native
+
+    layer, meta = _decode_rows_in_a_prefill_batch(rank)
+    _, _, packed, groups, n = _native.batch_tables(meta.adapter_indices.numpy(), layer.lora_entries(),
+                                                   np.array([6], dtype=np.int32), prefill)
+    assert groups[0].num_tokens == 120 and groups[0].plan_off >= 0
+    P = 0x1000
+    slices = (_native.LayerSlice * 1)(_native.LayerSlice(0, 128, 0))
+    rc = _native.lib().lorax_layer_update(groups, n, packed.ctypes.data, slices, 1, P, 128, P, rows, 128, 0, P, 1, P, 0, 1, 0,
+                                          None)
+    message = _native.lib().lorax_last_error().decode()
+    if refused:
+        assert rc == 1 and "fewer rows" in message
+    else:
+        assert rc != 0 and "fewer rows" not in message  # no device, or (with one) the workspace of one byte
+
+
+@pytest.mark.parametrize("prefill,rank", [(True, 32), (False, 32), (False, 8)])
+def test_layers_refuse_fewer_rows_than_their_routing_plan_names(monkeypatch, prefill, rank):
+    from lorax_amd import _native, layers
+
+    layer, meta = _decode_rows_in_a_prefill_batch(rank)
+    monkeypatch.setattr(layers, "has_sgmv", lambda: True)
+    for launch in ("bgmv_multi", "bgmv_lora_multi", "sgmv_shrink_multi"):
+        monkeypatch.setattr(_native, launch, lambda *a, **k: pytest.fail("launched"))
+    for native in (True, False):
+        data = AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill)
+        if not native:
+            monkeypatch.setattr("lorax_amd.adapters._native_batch_tables", lambda *a: None)
+            data = AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill)
+        x, y = (torch.zeros((119, 128), dtype=torch.bfloat16) for _ in range(2))
+        with pytest.raises(RuntimeError, match="119 rows, fewer than the 120"):
+            layers.LoraLinear(None, 0).forward_layer_type(y, x, data, "q_proj", 0, 128)
+
+
+def test_stacked_decode_refuses_fewer_rows_than_its_routing_plan_names(monkeypatch):
+    from lorax_amd import _native, ops
+
+    for launch in ("bgmv_stacked", "bgmv_lora_multi"):
+        monkeypatch.setattr(_native, launch, lambda *a, **k: pytest.fail("launched"))
+    slots = torch.tensor([0, 1, -1, 1])
+    a, b = torch.zeros(2, 16, 128, dtype=torch.bfloat16), torch.zeros(2, 256, 16, dtype=torch.bfloat16)
+    x, y = torch.zeros(3, 128, dtype=torch.bfloat16), torch.zeros(3, 256, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="3 rows, fewer than the 4"):
+        ops.bgmv_lora_slices(x, [(a, b, 0, 256)], y, slots, 1.0, plan=ops.build_slot_plan(slots))
