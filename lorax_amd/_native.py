@@ -837,10 +837,10 @@ class BatchTables:
         return made
 
 
-def layer_update(y, x, tables: BatchTables, slices, layer_idx: int, scratch) -> bool:
+def layer_update(y, x, tables: BatchTables, slices, layer_idx: int) -> bool:
     """lorax_layer_update: y[:, start:end] += the LoRA update of x for every slice, all launches from one call.
-    `scratch`: function that returns the 8 MiB shrink scratch of a device.  False, with nothing launched, where the
-    single entry points have to be used: operands they would refuse or that need another path."""
+    False, with nothing launched, where the single entry points have to be used: operands they would refuse or that
+    need another path."""
     code = _DTYPE_CODES.get(x.dtype)
     if (code is None or y.dtype != x.dtype or x.dim() != 2 or y.dim() != 2 or not x.is_cuda or not y.is_cuda
             or not x.is_contiguous() or not y.is_contiguous()):
@@ -852,15 +852,16 @@ def layer_update(y, x, tables: BatchTables, slices, layer_idx: int, scratch) -> 
             or not (tables.prefill or rows == tables.rows)):
         return False
     arr, columns = tables.call(slices)
-    tmp = None
+    # the call's own workspace, on its stream: [shrink scratch | v] in prefill, v alone in decode
+    tmp_bytes, v_bytes = 0, rows * columns * 2
     if tables.prefill:
         _ready(x)
-        tmp = scratch(x.device)
-    v = torch.empty((rows * columns,), dtype=x.dtype, device=x.device)
+        tmp_bytes = SHRINK_TMP_BYTES
+    work = torch.empty((tmp_bytes + v_bytes,), dtype=torch.uint8, device=x.device)
+    tmp = work.data_ptr()
     rc = lib().lorax_layer_update(
         tables.groups, tables.num_groups, tables.packed.data_ptr(), arr, len(arr), y.data_ptr(), width, x.data_ptr(), rows,
-        h_in, layer_idx, v.data_ptr(), rows * columns * 2, tmp.data_ptr() if tmp is not None else None,
-        tmp.numel() if tmp is not None else 0, code, index, _stream(x),
+        h_in, layer_idx, tmp + tmp_bytes, v_bytes, tmp if tmp_bytes else None, tmp_bytes, code, index, _stream(x),
     )
     if rc == EROUTE:
         return False

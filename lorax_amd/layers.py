@@ -104,7 +104,7 @@ class LoraLinear(nn.Module):
             targets.append((data.layer_type, start, end))
         if tables is None:
             return False
-        return _native.layer_update(result, input, tables, tuple(targets), self.layer_id, get_shrink_scratch)
+        return _native.layer_update(result, input, tables, tuple(targets), self.layer_id)
 
     def forward_layer_types(
         self,

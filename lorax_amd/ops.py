@@ -25,7 +25,7 @@ from typing import Dict, Optional, Tuple
 import torch
 
 from lorax_amd import _native
-from lorax_amd.sgmv import get_tmp_tensor, get_tmp_tensor_for_size
+from lorax_amd.sgmv import get_shrink_scratch, get_tmp_tensor_for_size
 
 _TABLE_CACHE: "OrderedDict[Tuple[int, int, int, str], torch.Tensor]" = OrderedDict()
 _TABLE_CACHE_SIZE = 1024
@@ -270,7 +270,7 @@ def sgmv_shrink(
                                                                         lora_indices_tensor)
     out, finish = _shrink_output(inputs, output_tensor)
     _native.sgmv_shrink(out, inputs, _segment_pointers(lora_a_weights, lora_indices_tensor), s_start, s_end,
-                        get_tmp_tensor(inputs.device), 0, scaling)
+                        get_shrink_scratch(inputs.device), 0, scaling)
     if finish is not None:
         finish()
 
@@ -306,7 +306,7 @@ def sgmv_lora_slices(
         assert a.dtype == inputs.dtype and b.dtype == inputs.dtype
         assert inputs.size(1) == a.size(-1) and a.size(-2) == b.size(-1) and slice_size == b.size(-2)
         by_rank.setdefault(a.size(-2), []).append((a, b, slice_offset, slice_size))
-    tmp = get_tmp_tensor(inputs.device)
+    tmp = get_shrink_scratch(inputs.device)
     tmp_expand = get_tmp_tensor_for_size(batches, inputs.device)
     tokens = inputs.size(0)
     for r, jobs in by_rank.items():

@@ -106,9 +106,12 @@ def get_tmp_tensor(device: torch.device) -> torch.Tensor:
 def get_shrink_scratch(device: torch.device) -> torch.Tensor:
     """Scratch of the resident-layout shrink entries (lora_a_sgmv_resident, lora_a_sgmv_resident_multi): where a
     batch has fewer row tiles than the GPU has CUs, the hidden dimension is cut into parts across workgroups and
-    the parts' fp32 sums (parts x rows x summed rank) go here.  It is the reference's 8 MiB buffer: the kernels
-    keep their sums inside the first 8 MiB whatever a caller passes, so that the result does not depend on it."""
-    return get_tmp_tensor(device)
+    the parts' fp32 sums (parts x rows x summed rank) go here.  It has the size of the reference's 8 MiB buffer: the
+    kernels keep their sums inside the first 8 MiB whatever a caller passes, so that the result does not depend on it.
+    Every call returns a buffer of its own, from the caching allocator and for the current stream: layers that run on
+    several streams or threads of one GPU at once must not share their sums (two shrinks that are in flight together
+    may not have one scratch), and inside a captured graph the buffer belongs to the graph."""
+    return torch.empty((_SHRINK_TMP_BYTES,), dtype=torch.uint8, device=device)
 
 
 def get_tmp_expand_size(size: int) -> int:
@@ -161,7 +164,7 @@ def lora_a_sgmv_resident(
     tiles=None,
 ) -> torch.Tensor:
     """As lora_a_sgmv_cutlass, reading the [L, r, h_in] stacks of the decode path (weights_a_t) whatever
-    the rank.  `tmp` is get_shrink_scratch(device) or the 8 MiB buffer of get_tmp_tensor.
+    the rank.  `tmp` is get_shrink_scratch(device) or the process's 8 MiB buffer of get_tmp_tensor.
     zero_fill=False skips the zero-fill launch: the kernel overwrites the rows of the segments and the rows
     outside every segment hold garbage - fine for a v that only goes to the expand of the same segments."""
     alloc = torch.zeros if zero_fill else torch.empty

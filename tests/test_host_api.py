@@ -608,3 +608,46 @@ def test_stacked_decode_refuses_fewer_rows_than_its_routing_plan_names(monkeypat
     x, y = torch.zeros(3, 128, dtype=torch.bfloat16), torch.zeros(3, 256, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="3 rows, fewer than the 4"):
         ops.bgmv_lora_slices(x, [(a, b, 0, 256)], y, slots, 1.0, plan=ops.build_slot_plan(slots))
+
+
+def test_shrink_scratch_is_the_callers_own(monkeypatch):
+    """Two prefill calls in flight at once (two streams or threads) must not keep their partial sums in one place: every
+    call of the layers, native or general, gets a scratch of its own from the allocator."""
+    from types import SimpleNamespace
+
+    from lorax_amd import _native, ops
+
+    cpu = torch.device("cpu")
+    a, b = sgmv.get_shrink_scratch(cpu), sgmv.get_shrink_scratch(cpu)
+    assert a.numel() == b.numel() == _native.SHRINK_TMP_BYTES and a.dtype == torch.uint8
+    assert abs(a.data_ptr() - b.data_ptr()) >= _native.SHRINK_TMP_BYTES
+    assert not hasattr(ops, "get_tmp_tensor")  # the stacked-weight operators take the same
+
+    allocated, passed = [], []
+    empty = torch.empty
+
+    def recording_empty(*args, **kwargs):
+        allocated.append(empty(*args, **kwargs))
+        return allocated[-1]
+
+    def layer_update(groups, num_groups, packed, slices, n, y, width, x, rows, h_in, layer, v, v_bytes, tmp, tmp_bytes, *rest):
+        passed.append((v, v_bytes, tmp, tmp_bytes))
+        return 0
+
+    def operand(cols):
+        return SimpleNamespace(dtype=torch.bfloat16, device=cpu, is_cuda=True, shape=(700, cols), dim=lambda: 2,
+                               is_contiguous=lambda: True, get_device=lambda: -1, data_ptr=lambda: 0x1000)
+
+    monkeypatch.setattr(_native, "lib", lambda: SimpleNamespace(lorax_layer_update=layer_update))
+    monkeypatch.setattr(_native, "_ready", lambda t: None)
+    monkeypatch.setattr(_native, "_stream", lambda t: 0)
+    monkeypatch.setattr(torch, "empty", recording_empty)
+    group = _native.TableGroup(layer_type=0, rank=16)
+    for prefill in (True, True, False):
+        tables = _native.BatchTables([group], 1, torch.zeros(8, dtype=torch.uint8), 700, prefill)
+        assert _native.layer_update(operand(256), operand(512), tables, ((0, 0, 256),), 0)
+    for work, (v, v_bytes, tmp, tmp_bytes), prefill in zip(allocated, passed, (True, True, False)):
+        assert v_bytes == 700 * 16 * 2 and v == work.data_ptr() + tmp_bytes
+        assert (tmp, tmp_bytes) == ((work.data_ptr(), _native.SHRINK_TMP_BYTES) if prefill else (None, 0))
+        assert work.numel() == tmp_bytes + v_bytes
+    assert len(allocated) == 3
