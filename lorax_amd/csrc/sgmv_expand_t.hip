@@ -52,9 +52,9 @@ struct ExpandSlot {
   int r;
   int h_out;
   int num_tiles;   // records of the plan
-  int tile_rows;   // height bound of the plan's tiles; without a plan the height the search cuts
+  int tile_rows;   // no record of the plan is taken higher; without a plan the height the search cuts
   int tile_slots;  // row tiles counted for the grid
-  int subs;        // pieces of sub_rows rows a tile is cut into
+  int subs;        // pieces of sub_rows rows a tile is cut into; the last one takes what is left
 };
 struct ExpandLaunch {
   ExpandSlot p[kMaxExpandProblems];
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const Expan
     if (P.tiles != nullptr && stack == 0) break;  // a caller's plan that names a segment without a stack
     if (P.subs > 1) {
       rt.row0 += sub * sub_rows;
-      rt.row_end = min(rt.row_end, rt.row0 + sub_rows);
+      if (sub + 1 < P.subs) rt.row_end = min(rt.row_end, rt.row0 + sub_rows);
       if (rt.row0 >= rt.row_end) continue;
     }
     if (panel * kCols >= P.h_out) break;
@@ -247,7 +247,10 @@ static hipError_t launch_expand_t_ks(const ExpandArgs& a, hipStream_t stream) {
     if (q.tiles != nullptr && q.num_tiles > 0 && q.tile_rows >= 1 && tuning().expand_rows == 0 && fits(q.tile_rows, q.y_stride)) {
       s.tiles = q.tiles;
       s.num_tiles = s.tile_slots = q.num_tiles;
-      s.tile_rows = height[i] = q.tile_rows;
+      // The pieces are counted for the plan's own height, but its records may be rewritten between the replays of a
+      // captured launch: one that is higher (to the highest the planner cuts) is walked to its end by its last piece.
+      height[i] = q.tile_rows;
+      s.tile_rows = q.tile_rows < kExpandTileRowsMax && fits(kExpandTileRowsMax, q.y_stride) ? kExpandTileRowsMax : q.tile_rows;
     } else {
       int rows = tuning().expand_rows > 0 ? (tuning().expand_rows + 15) / 16 * 16 : kExpandTileRows;
       while (rows > 16 && !fits(rows + rows / 8 + 16, q.y_stride)) rows /= 2;

@@ -19,6 +19,7 @@ namespace lorax {
 
 constexpr int kShrinkTileRowsMax = 64;   // the LDS-staged shrink's buffers hold up to four 16-row blocks
 constexpr int kExpandTileRows = 256;     // nominal height of an expand tile
+constexpr int kExpandTileRowsMax = kExpandTileRows + kExpandTileRows / 8 + 16;  // with a merged remainder
 
 struct SegmentSpan {
   int32_t seg, start, end;  // clamped to [0, num_tokens], end > start
@@ -86,7 +87,7 @@ inline int plan_shrink_tiles(const std::vector<SegmentSpan>& segs, std::vector<l
 // Expand tiles: nominally 256 rows; a remainder of at most an eighth of the segment's full tiles is shared out
 // among them instead of becoming a tile of its own (a tile's prologue costs as much as a hundred rows), and the
 // segment's tiles get equal heights in 16-row blocks - the rule of the device-side search (merged_tile_count).
-// Returns the height of the tallest tile (the launcher sizes its grid by it).
+// Returns the height of the tallest tile (the launcher cuts tiles into pieces by it); none is above kExpandTileRowsMax.
 inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<lorax_sgmv_tile_t>& out) {
   int tallest = 1;
   for (const SegmentSpan& s : segs) {

@@ -198,3 +198,47 @@ def test_a_tile_that_names_a_segment_without_a_stack_is_skipped():
         differ = (outs[0] != outs[1]).nonzero()
         assert differ.numel() == 0, f"kind {kind}: {differ.size(0)} elements differ, first {differ[:8].tolist()}"
         assert torch.count_nonzero(outs[0]) > 0
+
+
+@pytest.mark.parametrize("r,h_out,y_stride", [(16, 512, 640), (64, 1024, 1024)])
+def test_expand_captured_with_low_tiles_replays_higher_ones(r, h_out, y_stride):
+    """A captured planned expand whose tables and records are rewritten for a batch of longer segments: the tiles are
+    higher than the captured plan's tile_rows, up to the highest the planner cuts, and no row is lost."""
+    dtype, T, layer, slots = torch.bfloat16, 1400, 0, 40
+    gen = torch.Generator().manual_seed(r)
+    v = randn((T, r), 1.0, gen, dtype, DEV)
+    bt = [randn((1, h_out, r), 0.05, gen, dtype, DEV) for _ in range(3)]
+    table = ptr_table(bt, DEV)
+    y0 = randn((T, y_stride), 0.5, gen, dtype, DEV)
+    y = y0.clone()
+    tmp = sgmv.get_tmp_tensor_for_size(3, torch.device(DEV))
+    s_start, s_end = (torch.zeros(3, dtype=torch.int32, device=DEV) for _ in range(2))
+    records = torch.zeros((slots, 4), dtype=torch.int32, device=DEV)
+
+    def load(lens):
+        ends = [sum(lens[: i + 1]) for i in range(3)]
+        starts = [e - n for e, n in zip(ends, lens)]
+        cut, tile_rows = _native.plan_tiles(starts, ends, T, _native.TILES_EXPAND)
+        records.zero_()
+        records[: len(cut)].copy_(torch.from_numpy(cut.copy()))
+        s_start.copy_(torch.tensor(starts, dtype=torch.int32))
+        s_end.copy_(torch.tensor(ends, dtype=torch.int32))
+        return tile_rows
+
+    low = load([40, 3, 17])
+    assert low == 40
+    plan = _native.TilePlan(records, low)
+    call = lambda out, tiles: _native.sgmv_expand(out, v, table, s_start, s_end, tmp, layer, 0, h_out, True, True, tiles)
+    call(y.clone(), plan)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(y, plan)
+    for lens in ([40, 3, 17], [304, 256, 287], [1, 700, 33], [0, 1400, 0], [16, 0, 9]):
+        height = load(lens)
+        y.copy_(y0)
+        graph.replay()
+        want = y0.clone()
+        call(want, None)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), f"lens {lens}, tiles of up to {height} rows"
