@@ -145,6 +145,10 @@ __device__ __forceinline__ void expand_tile(const ExpandSlot& P, const typename 
     f32x4 acc[NJ];
 #pragma unroll
     for (int s = 0; s < KS; ++s) vf[s] = to_operand_lanes(vf[s]);
+    if (r < KS * 32) {  // uniform; chunks beyond the rank hold chunk 0: an infinity there times B's zeros would be NaN
+#pragma unroll
+      for (int s = 0; s < KS; ++s) vf[s] = keep_if<D>(k_ok[s], vf[s]);
+    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};

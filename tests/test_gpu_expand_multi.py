@@ -60,6 +60,34 @@ def test_expands_of_one_launch_equal_single_launches(dtype, planned, parts):
     assert_close(y_a, want, "expands of one launch")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ranks", [[8], [16], [24], [40], [72], [96], [96, 128], [16, 64], [8, 24, 32, 40, 72, 104]])
+def test_infinities_of_v_stay_infinities(ranks, dtype):
+    """An element of v that overflowed gives an infinite update, as a dot product over the rank does, whether or not the
+    rank fills the matrix instruction's steps and whatever other ranks share the launch."""
+    print(f"case dtype={dtype} ranks={ranks}", flush=True)
+    gen = torch.Generator().manual_seed(sum(ranks))
+    h_out, rows = 264, 37
+    problems, wants, ys, stacks = [], [], [], []
+    for r in ranks:
+        v = randn((rows, r), 1.0, gen, dtype, DEV)
+        v[3, 0], v[20, r - 1], v[36, 5] = float("inf"), float("-inf"), float("inf")
+        bt = randn((1, h_out, r), 0.05, gen, dtype, DEV)
+        bt[0, :, [0, 5, r - 1]] = torch.where(bt[0, :, [0, 5, r - 1]] == 0, 0.05, bt[0, :, [0, 5, r - 1]])  # no inf * 0
+        s, e = (torch.tensor([t], dtype=torch.int32, device=DEV) for t in (0, rows))
+        ys.append(randn((rows, h_out), 0.5, gen, dtype, DEV))
+        wants.append((ys[-1].cpu().double() + v.cpu().double() @ bt[0].cpu().double().t()).to(DEV))
+        problems.append((ys[-1], v, ptr_table([bt], DEV), s, e, 0, h_out, None))
+        stacks.append(bt)
+    _native.sgmv_expand_multi(problems, 0)
+    torch.cuda.synchronize()
+    for r, y, want in zip(ranks, ys, wants):
+        inf = torch.isinf(want)
+        assert inf[[3, 20, 36]].all() and inf.sum() == 3 * h_out
+        assert torch.equal(y.double()[inf], want[inf]), f"rank {r}"
+        assert_close(y[~inf], want[~inf].to(dtype), f"rank {r}")
+
+
 def test_expand_multi_checks_its_problems():
     y = torch.zeros((4, 64), dtype=torch.bfloat16, device=DEV)
     v = torch.zeros((4, 16), dtype=torch.bfloat16, device=DEV)
