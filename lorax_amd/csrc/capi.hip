@@ -275,13 +275,13 @@ int expand_batch(const lorax_sgmv_expand_problem_t* problems, int32_t count, int
   if (count < 0 || count > kMaxExpandProblems)
     return fail(LORAX_EINVAL, "num_problems=%d (at most %d per launch)", count, kMaxExpandProblems);
   if (num_tokens < 0) return fail(LORAX_EINVAL, "num_tokens=%lld is negative", (long long)num_tokens);
-  if (count == 0 || num_tokens == 0) return LORAX_OK;
+  if (count == 0) return LORAX_OK;
   if (problems == nullptr) return fail(LORAX_EINVAL, "null pointer argument (problems)");
   ExpandArgs a{};
   for (int i = 0; i < count; ++i) {
     const lorax_sgmv_expand_problem_t& q = problems[i];
     if (q.num_segments < 0) return fail(LORAX_EINVAL, "negative size (num_segments=%d)", q.num_segments);
-    if (q.num_segments == 0) continue;
+    if (q.num_segments == 0 || num_tokens == 0) continue;
     if (int rc = check_expand(q.y, q.v, q.w_ptrs, q.s_start, q.s_end, num_tokens, q.r, q.h_out, q.y_offset, q.y_stride, dtype))
       return rc;
     if (layer_idx < 0) return fail(LORAX_EINVAL, "layer_idx=%lld is negative", (long long)layer_idx);
@@ -306,17 +306,17 @@ int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int
                         int32_t num_segments, int64_t num_tokens, int32_t r, int32_t h_out, int32_t b_layout,
                         int64_t y_offset, int64_t y_stride, int64_t layer_idx, int32_t accumulate,
                         const lorax_sgmv_tiles_t* tiles, int32_t dtype, void* stream) {
-  if (b_layout == LORAX_B_HR) {
-    const lorax_sgmv_expand_problem_t one{y, v, w_ptrs, s_start, s_end, num_segments, r, h_out, y_offset, y_stride, tiles};
-    return expand_batch(&one, 1, num_tokens, layer_idx, accumulate, dtype, stream);
-  }
   if (accumulate != 0 && accumulate != 1)
     return fail(LORAX_EINVAL, "accumulate=%d (0 = overwrite, 1 = add)", accumulate);
-  if (b_layout != LORAX_B_RH) return fail(LORAX_EINVAL, "b_layout=%d", b_layout);
+  if (b_layout != LORAX_B_RH && b_layout != LORAX_B_HR) return fail(LORAX_EINVAL, "b_layout=%d", b_layout);
   if (num_segments < 0 || num_tokens < 0)
     return fail(LORAX_EINVAL, "negative size (num_segments=%d num_tokens=%lld)", num_segments,
                 (long long)num_tokens);
   if (num_segments == 0 || num_tokens == 0) return LORAX_OK;
+  if (b_layout == LORAX_B_HR) {
+    const lorax_sgmv_expand_problem_t one{y, v, w_ptrs, s_start, s_end, num_segments, r, h_out, y_offset, y_stride, tiles};
+    return expand_batch(&one, 1, num_tokens, layer_idx, accumulate, dtype, stream);
+  }
   if (int rc = check_expand(y, v, w_ptrs, s_start, s_end, num_tokens, r, h_out, y_offset, y_stride, dtype)) return rc;
   if (layer_idx < 0) return fail(LORAX_EINVAL, "layer_idx=%lld is negative", (long long)layer_idx);
   SgmvArgs a{};

@@ -150,6 +150,17 @@ def test_sgmv_expand_validation():
     assert f(P, P, P, P, P, 2, 16, 16, 4096, 2, 0, 4096, 0, 1, P, 120, 1, None) == EINVAL  # unknown layout
 
 
+@pytest.mark.parametrize("num_segments,num_tokens", [(-1, 0), (-1, 16), (2, -1), (0, -1)])
+def test_sgmv_expand_refuses_negative_sizes_whatever_else_is_empty(num_segments, num_tokens):
+    lib = _native.lib()
+    for layout in (_native.B_RH, _native.B_HR):
+        assert lib.lorax_sgmv_expand(P, P, P, P, P, num_segments, num_tokens, 16, 4096, layout, 0, 4096, 0, 1, P,
+                                     60 * max(num_segments, 0), 1, None) == EINVAL, layout
+    assert lib.lorax_sgmv_expand_planned(P, P, P, P, P, num_segments, num_tokens, 16, 4096, 0, 4096, 0, 1, None, 1, None) == EINVAL
+    one = (_native.SgmvExpandProblem * 1)(_native.SgmvExpandProblem(P, P, P, P, P, num_segments, 16, 4096, 0, 4096, None))
+    assert lib.lorax_sgmv_expand_multi(one, 1, num_tokens, 0, 1, 1, None) == EINVAL and "negative" in _err()
+
+
 def test_sgmv_expand_planned_validation():
     f = _native.lib().lorax_sgmv_expand_planned
     assert f(P, P, P, P, P, 0, 16, 16, 4096, 0, 4096, 0, 1, None, 1, None) == OK  # no segments
