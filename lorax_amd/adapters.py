@@ -745,7 +745,7 @@ def _native_batch_tables(meta: AdapterBatchMetadata, weights: Dict[str, LayerAda
     for lt, type_groups in by_type.items():
         every = weights[names[lt]].unwrapped()
         loras = {a: every[a] for a in batch_adapters & every.keys()}
-        data[names[lt]] = {LORA: _PackedLoraWeights(names[lt], lt, loras, build, type_groups, shared)}
+        data[names[lt]] = {LORA: _PackedLoraWeights.over(names[lt], lt, loras, build, type_groups, shared)}
     return data
 
 
@@ -835,13 +835,21 @@ class _PackedLoraWeights(BatchLoraWeights):
     made on first access; making all of them took longer than the native builder and the upload together (a batch of
     four ranks and seven layer types: 0.35 of 0.42 ms).  Until then `packed_tables` is the batch's BatchTables, from which
     a layer's launches are issued natively; from the first access on it is None, because whoever holds the tables' views
-    may put others in their place, and the launches follow rank_data."""
+    may put others in their place, and the launches follow rank_data.  (Printing or comparing a batch hands nothing out.)
+    Constructed from the dataclass's fields - dataclasses.replace does that - it is a plain BatchLoraWeights."""
 
-    def __init__(self, layer_name: str, layer_type: int, loras: Dict[int, LoraWeights], views: _TableViews, groups, shared):
+    _configs: Optional[Dict[int, LoraConfig]] = None
+    _rank_data: Optional[Dict[object, RankSegments]] = None
+    _handed_out = False
+    packed_tables = None
+
+    @classmethod
+    def over(cls, layer_name: str, layer_type: int, loras: Dict[int, LoraWeights], views: _TableViews, groups,
+             shared) -> "_PackedLoraWeights":
+        self = cls.__new__(cls)
         self._loras = loras
         self._views = views
         self._groups = groups
-        self._rank_data: Optional[Dict[object, RankSegments]] = None
         self.layer_type = layer_type
         self.packed_tables = shared
         self.lora_a = _LayoutView(loras, "weights_a")
@@ -849,6 +857,7 @@ class _PackedLoraWeights(BatchLoraWeights):
         self.use_sgmv = bool(groups[0].use_sgmv)
         self.layer_name = layer_name
         self.prefill_head_indices = None
+        return self
 
     @property
     def adapter_index_configs(self) -> Dict[int, LoraConfig]:
@@ -856,27 +865,40 @@ class _PackedLoraWeights(BatchLoraWeights):
             self._configs = {a: lw.adapter_config for a, lw in self._loras.items()}
         return self._configs
 
-    _configs = None
-
     @adapter_index_configs.setter
     def adapter_index_configs(self, configs) -> None:
         self._configs = configs
 
-    @property
-    def rank_data(self) -> Dict[object, RankSegments]:
+    def _own_rank_data(self) -> Dict[object, RankSegments]:
         if self._rank_data is None:
             self._rank_data = self._views.rank_data(self._groups, self._loras)
-            self.packed_tables = None
         return self._rank_data
+
+    @property
+    def rank_data(self) -> Dict[object, RankSegments]:
+        self._handed_out = True
+        self.packed_tables = None
+        return self._own_rank_data()
 
     @rank_data.setter
     def rank_data(self, rank_data) -> None:
         self._rank_data = rank_data
+        self._handed_out = True
         self.packed_tables = None
 
-    def can_vectorize(self, pg) -> bool:
-        # the native builder takes adapters of the kernels' ranks only
-        return True if self._rank_data is None else super().can_vectorize(pg)
-
     def ranks(self) -> Set[int]:
-        return {g.rank for g in self._groups} if self._rank_data is None else super().ranks()
+        return super().ranks() if self._handed_out else {g.rank for g in self._groups}
+
+    def _plain(self) -> BatchLoraWeights:
+        return BatchLoraWeights(self.lora_a, self.lora_b, self.adapter_index_configs, self._own_rank_data(), self.use_sgmv,
+                                self.layer_name, self.prefill_head_indices)
+
+    def __repr__(self) -> str:
+        return repr(self._plain())
+
+    def __eq__(self, other) -> bool:
+        if not isinstance(other, BatchLoraWeights):
+            return NotImplemented
+        return self._plain() == (other._plain() if isinstance(other, _PackedLoraWeights) else other)
+
+    __hash__ = None

@@ -651,3 +651,35 @@ def test_shrink_scratch_is_the_callers_own(monkeypatch):
         assert (tmp, tmp_bytes) == ((work.data_ptr(), _native.SHRINK_TMP_BYTES) if prefill else (None, 0))
         assert work.numel() == tmp_bytes + v_bytes
     assert len(allocated) == 3
+
+
+@pytest.mark.parametrize("prefill", [True, False])
+def test_batches_from_the_native_builder_are_dataclasses_like_any_other(prefill):
+    """dataclasses.replace works, and printing, comparing or asking for ranks does not hand the tables out (which would
+    take the batch's layers off their native call)."""
+    import dataclasses
+
+    from lorax_amd.adapters import BatchLoraWeights
+
+    layer, meta = _decode_rows_in_a_prefill_batch(16)
+    batch, other = (AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data["q_proj"][LORA] for _ in range(2))
+    for b in (batch, other):
+        b.packed_tables = object()  # stands for the device tables, which a CPU batch does not have
+    assert isinstance(batch, BatchLoraWeights)
+    text = repr(batch)
+    assert text.startswith("BatchLoraWeights(") and "rank_data={16:" in text and "layer_name='q_proj'" in text
+    assert batch == batch and batch != other and batch != "q_proj" and (batch == None) is False  # noqa: E711
+    assert batch.ranks() == {16} and batch.can_vectorize(SingleProcessGroup()) and batch.has_adapter(1)
+    assert batch.packed_tables is not None and other.packed_tables is not None
+    with pytest.raises(TypeError):
+        hash(batch)
+
+    head = torch.tensor([3])
+    changed = dataclasses.replace(batch, prefill_head_indices=head, layer_name="lm_head")
+    assert isinstance(changed, BatchLoraWeights) and changed.packed_tables is None
+    assert changed.prefill_head_indices is head and changed.layer_name == "lm_head"
+    assert changed.rank_data is batch.rank_data and changed.use_sgmv == prefill and changed.ranks() == {16}
+    assert changed.adapter_index_configs == batch.adapter_index_configs and changed.lora_a is batch.lora_a
+    assert batch.packed_tables is None  # its tables are shared with another object now
+    assert dataclasses.replace(batch) == batch and changed != batch
+    assert [f.name for f in dataclasses.fields(batch)] == [f.name for f in dataclasses.fields(BatchLoraWeights)]
