@@ -539,26 +539,54 @@ class BatchLoraWeights(BatchAdapterWeights):
         )
 
 
+class _AdapterDict(dict):
+    """A dict that counts its changes, so that what is derived from it is rebuilt after any of them."""
+
+    version = 0
+
+
+def _counting(method):
+    def change(self, *args, **kwargs):
+        self.version += 1
+        return method(self, *args, **kwargs)
+
+    return change
+
+
+for _name in ("__setitem__", "__delitem__", "__ior__", "clear", "pop", "popitem", "setdefault", "update"):
+    setattr(_AdapterDict, _name, _counting(getattr(dict, _name)))
+
+
 class LayerAdapterWeights:
     """All adapters loaded for one layer type (adapters/weights.py:66-105)."""
 
     def __init__(self):
-        self.adapter_weights: Dict[int, AdapterWeights] = {}
-        self._lora_entries = None  # cached argument of the native table builder
-        self._unwrapped = None
+        self.adapter_weights = {}
+
+    @property
+    def adapter_weights(self) -> Dict[int, AdapterWeights]:
+        return self._adapter_weights
+
+    @adapter_weights.setter
+    def adapter_weights(self, weights: Dict[int, AdapterWeights]) -> None:
+        self._adapter_weights = _AdapterDict(weights)
+        self._derived_from = None
 
     def add_adapter(self, adapter_idx: int, weights: AdapterWeights):
-        self.adapter_weights[adapter_idx] = weights
-        self._lora_entries = None
-        self._unwrapped = None
+        self._adapter_weights[adapter_idx] = weights
 
     def remove_adapter(self, adapter_idx: int):
-        self.adapter_weights.pop(adapter_idx, None)
-        self._lora_entries = None
-        self._unwrapped = None
+        self._adapter_weights.pop(adapter_idx, None)
+
+    def _drop_stale(self) -> None:
+        if self._derived_from != self._adapter_weights.version:
+            self._derived_from = self._adapter_weights.version
+            self._lora_entries = None  # cached argument of the native table builder
+            self._unwrapped = None
 
     def unwrapped(self) -> Dict[int, "AdapterWeights"]:
         """adapter index -> the adapter's weights without their wrapper; rebuilt only when adapters come or go."""
+        self._drop_stale()
         if self._unwrapped is None:
             self._unwrapped = {idx: _unwrap(w) for idx, w in self.adapter_weights.items()}
         return self._unwrapped
@@ -567,6 +595,7 @@ class LayerAdapterWeights:
         """(adapter, address of the [L, r, h_in] stack, address of the [L, h_out, r] stack, rank) of every LoRA
         adapter of the layer type, sorted by adapter, as a numpy array of _native.ENTRY_DTYPE; None if an adapter
         of another kind, or of a rank above the kernels' 128, is loaded.  Rebuilt only when adapters come or go."""
+        self._drop_stale()
         if self._lora_entries is None:
             import numpy as np
 

@@ -683,3 +683,49 @@ def test_batches_from_the_native_builder_are_dataclasses_like_any_other(prefill)
     assert batch.packed_tables is None  # its tables are shared with another object now
     assert dataclasses.replace(batch) == batch and changed != batch
     assert [f.name for f in dataclasses.fields(batch)] == [f.name for f in dataclasses.fields(BatchLoraWeights)]
+
+
+def _assign(layer, weights):
+    layer.adapter_weights[1] = weights
+
+
+def _update(layer, weights):
+    layer.adapter_weights.update({1: weights})
+
+
+def _replace_dict(layer, weights):
+    layer.adapter_weights = {**layer.adapter_weights, 1: weights}
+
+
+def _merge(layer, weights):
+    layer.adapter_weights |= {1: weights}
+
+
+def _delete_and_add(layer, weights):
+    del layer.adapter_weights[1]
+    layer.adapter_weights.setdefault(1, weights)
+
+
+@pytest.mark.parametrize("change", [_assign, _update, _replace_dict, _merge, _delete_and_add])
+@pytest.mark.parametrize("prefill", [True, False])
+def test_adapters_changed_in_the_dict_itself_reach_the_next_batch(change, prefill):
+    """The tables and configurations of a batch are those of the adapters loaded now, also when one was put into
+    LayerAdapterWeights.adapter_weights without add_adapter (the old one's stacks may be gone)."""
+    def adapter(rank):
+        return LoraWeights([torch.randn(64, rank)], [torch.randn(rank, 64)], LoraConfig(r=rank))
+
+    layer, meta = _decode_rows_in_a_prefill_batch(16, h=64)
+    first = AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data["q_proj"][LORA]
+    assert first.ranks() == {16}
+    new = adapter(32)
+    change(layer, new)
+    batch = AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data["q_proj"][LORA]
+    assert batch.adapter_index_configs[1] is new.adapter_config
+    assert batch.ranks() == {16, 32}
+    rd = batch.rank_data[32]
+    table = rd.lora_a_t_ptr if prefill else rd.lora_a_ptr
+    assert set(table.tolist()) == {new.weights_a_t.data_ptr()}
+    layer.adapter_weights.pop(1)
+    assert AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data["q_proj"][LORA].ranks() == {16}
+    layer.adapter_weights.clear()
+    assert layer.is_empty() and "q_proj" not in AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data
