@@ -915,6 +915,10 @@ class _PackedLoraWeights(BatchLoraWeights):
         self._handed_out = True
         self.packed_tables = None
 
+    def can_vectorize(self, pg) -> bool:
+        # the native builder takes adapters of the kernels' ranks only
+        return super().can_vectorize(pg) if self._handed_out else True
+
     def ranks(self) -> Set[int]:
         return super().ranks() if self._handed_out else {g.rank for g in self._groups}
 
