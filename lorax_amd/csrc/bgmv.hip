@@ -856,7 +856,9 @@ __device__ __forceinline__ bool balanced_slot(int count, int chunks, int chunks_
   return true;
 }
 
-template <typename D, int R, int U, int NBLK, bool VEC4>
+// NUMBERED: problems of several column slices, numbered without gaps (launch_lora_blk).  An instantiation of its own: the
+// table walk in the same one cost the others 1 %.
+template <typename D, int R, int U, int NBLK, bool VEC4, bool NUMBERED>
 __global__ __launch_bounds__(kBgmvThreads) void bgmv_lora_kernel(const BgmvBatch batch, int h_in,
                                                                  int64_t layer_idx, float scale, int count,
                                                                  int balanced_chunks, int chunks_per_xcd) {
@@ -865,7 +867,12 @@ __global__ __launch_bounds__(kBgmvThreads) void bgmv_lora_kernel(const BgmvBatch
   __shared__ __attribute__((aligned(16))) E vsh[R * kGroup];
   const ProblemFields fields = preload_problems(batch);  // before anything waits: see select_problem
   VirtualBlock vb;
-  if (balanced_chunks > 0) {
+  if constexpr (NUMBERED) {
+    const BatchSlot slot = batch_slot(batch, count);
+    vb.x = slot.sub;
+    vb.y = slot.chunk;
+    vb.z = slot.problem;
+  } else if (balanced_chunks > 0) {
     if (!balanced_slot(count, balanced_chunks, chunks_per_xcd, vb)) return;
   } else {
     vb = xcd_virtual_block();
@@ -1085,6 +1092,15 @@ static hipError_t launch_expand(const BgmvArgs& a, hipStream_t stream) {
   return launch_expand_u<D, 4>(a, stream);
 }
 
+constexpr int kNumCus = 256;
+
+// Whether the problems of a fused launch have different numbers of slices of `cols` columns.
+static bool unequal_slices(const BgmvArgs& a, int cols) {
+  for (int i = 0; i < a.count; ++i)
+    if ((a.batch.p[i].width + cols - 1) / cols != (a.wide_max + cols - 1) / cols) return true;
+  return false;
+}
+
 template <typename D, int R, int NBLK>
 static hipError_t launch_lora_blk(const BgmvArgs& a, hipStream_t stream) {
   constexpr int U = 4;
@@ -1109,6 +1125,23 @@ static hipError_t launch_lora_blk(const BgmvArgs& a, hipStream_t stream) {
       grid = dim3(kXcds * slots);
     }
   }
+  // Unequal numbers of column slices: a grid of (slices of the widest) x chunks x projections is mostly workgroups
+  // without work, and its numbering puts the wide projection's on two or three of the eight XCDs.  Numbered without
+  // gaps, one workgroup per CU: 8192 + 1024 + 1024 columns, 16 records of 4 tokens, 9.7 -> 7.5 us at rank 8 (hidden size
+  // 8192), 10.1 -> 8.8 at rank 16 (4096); the two-launch update takes 8.9 and 9.7.  The numbering is a table walk in
+  // front of the first load, so a grid that has a CU for each workgroup even with the gaps stays (4.2 -> 4.3 us), and
+  // so do slices of half a projection that are more than the CUs (66 records of 4096 + 1024 + 1024: 7.5 -> 8.5 us).
+  bool numbered_launch = false;
+  if (unequal_slices(a, cols_per_wg) && static_cast<int64_t>(grid.x) * grid.y * grid.z > kNumCus) {
+    BgmvArgs numbered = a;
+    const int64_t total = number_workgroups(numbered, [](const BgmvProblem& p) { return (p.width + cols_per_wg - 1) / cols_per_wg; });
+    if (total >= INT32_MAX) return hipErrorInvalidValue;
+    if (total <= kNumCus || NBLK == 4) {
+      batch = numbered.batch;
+      numbered_launch = true;
+      grid = dim3(static_cast<unsigned>(total));
+    }
+  }
   // 8-byte y accesses need every problem's rows 8-byte aligned and no ragged last column group
   bool vec4 = true;
   for (int i = 0; i < a.count; ++i) {
@@ -1116,12 +1149,14 @@ static hipError_t launch_lora_blk(const BgmvArgs& a, hipStream_t stream) {
     vec4 = vec4 && p.width % 4 == 0 && p.y_stride % 4 == 0 && p.y_offset % 4 == 0 &&
            reinterpret_cast<uintptr_t>(p.y) % 8 == 0;
   }
-  if (vec4)
-    hipLaunchKernelGGL((bgmv_lora_kernel<D, R, U, NBLK, true>), grid, dim3(kBgmvThreads), 0, stream, batch, a.h_in,
-                       a.layer_idx, a.scale, a.count, balanced_chunks, chunks_per_xcd);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBgmvThreads), 0, stream, batch, a.h_in, a.layer_idx, a.scale, a.count,
+                       balanced_chunks, chunks_per_xcd);
+  };
+  if (numbered_launch)
+    vec4 ? launch(bgmv_lora_kernel<D, R, U, NBLK, true, true>) : launch(bgmv_lora_kernel<D, R, U, NBLK, false, true>);
   else
-    hipLaunchKernelGGL((bgmv_lora_kernel<D, R, U, NBLK, false>), grid, dim3(kBgmvThreads), 0, stream, batch,
-                       a.h_in, a.layer_idx, a.scale, a.count, balanced_chunks, chunks_per_xcd);
+    vec4 ? launch(bgmv_lora_kernel<D, R, U, NBLK, true, false>) : launch(bgmv_lora_kernel<D, R, U, NBLK, false, false>);
   return hipGetLastError();
 }
 
@@ -1136,6 +1171,14 @@ static hipError_t launch_lora_r(const BgmvArgs& a, hipStream_t stream) {
   int64_t wgs4 = 0;
   for (int i = 0; i < a.count; ++i) wgs4 += a.grid_rows * ((a.batch.p[i].width + cols4 - 1) / cols4);
   int nblk = wgs4 >= 200 ? 4 : (wgs4 >= 100 ? 2 : 1);
+  // (a wide projection among narrow ones is cut into more slices than these bounds foresee: not into more than the CUs,
+  // as far as wider slices are fewer)
+  auto slices = [&](int cols) {
+    int64_t n = 0;
+    for (int i = 0; i < a.count; ++i) n += a.grid_rows * ((a.batch.p[i].width + cols - 1) / cols);
+    return n;
+  };
+  while (nblk < (a.wide_max > cols4 ? 4 : 2) && unequal_slices(a, cols4 / 4 * nblk) && slices(cols4 / 4 * nblk) > kNumCus) nblk *= 2;
   if (tuning().bgmv_lora_blocks > 0) nblk = tuning().bgmv_lora_blocks;
   if (nblk >= 4) return launch_lora_blk<D, R, 4>(a, stream);
   if (nblk >= 2) return launch_lora_blk<D, R, 2>(a, stream);

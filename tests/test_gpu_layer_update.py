@@ -6,6 +6,7 @@ import random
 import pytest
 import torch
 
+from lorax_amd import _native
 from lorax_amd.adapters import LORA, AdapterBatchData, LayerAdapterWeights, LoraConfig, LoraWeights
 from lorax_amd.layers import TensorParallelMultiAdapterLinear
 from lorax_amd.synthetic import make_meta
@@ -111,3 +112,44 @@ def test_layer_update_leaves_other_operands_to_the_general_path():
         with pytest.raises(RuntimeError):
             linear(bad_x, data)
     assert torch.count_nonzero(y).item() == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank,h_in,widths,records", [
+    (8, 1024, [8192, 1024, 1024], [16, 16, 16]),    # one-block slices, gaps in the plain grid
+    (8, 512, [1024, 8200, 264], [20, 41, 3]),       # projections of different record counts, the wide one not first
+    (8, 512, [8192, 1024, 1024], [43, 43, 43]),     # more half slices than CUs: whole ones
+    (8, 512, [14336, 1024], [64, 64]),              # more whole slices than CUs
+    (16, 1024, [8192, 1024, 1024, 16], [16, 16, 16, 0]),
+    (16, 512, [4096, 1024, 1024], [12, 15, 9]),
+    (16, 512, [2048, 512, 512], [50, 50, 50]),
+])
+def test_one_launch_for_unequal_projections(rank, h_in, widths, records, dtype):
+    """The single-launch update of wide and narrow projections together, whose workgroups are numbered without gaps,
+    against one launch each: the same bits, and nothing outside their columns."""
+    print(f"case rank={rank} h_in={h_in} widths={widths} records={records} dtype={dtype}", flush=True)
+    gen = torch.Generator().manual_seed(rank + sum(widths))
+    tokens = 3 * max(records) + 2
+    x = torch.randn((tokens, h_in), generator=gen).to(dtype).cuda()
+    y0 = torch.randn((tokens, sum(widths) + 16), generator=gen).to(dtype).cuda()
+    problems, keep, off = [], [], 8
+    for width, n in zip(widths, records):
+        a = torch.randn((max(n, 1), 2, rank, h_in), generator=gen).mul_(0.05).to(dtype).cuda()
+        b = torch.randn((max(n, 1), 2, width, rank), generator=gen).mul_(0.05).to(dtype).cuda()
+        plan = torch.zeros((n, 8), dtype=torch.int64)
+        for i in range(n):  # one to three tokens each; every seventh record is padding
+            toks = [3 * i + k for k in range(1 + i % 3)]
+            plan[i] = torch.tensor([0 if i % 7 == 6 else len(toks), *toks, *[toks[0]] * (4 - len(toks)), a[i].data_ptr(),
+                                    b[i].data_ptr(), 0])
+        keep.append((a, b))
+        problems.append((plan.cuda(), off, width))
+        off += width
+    together, apart = y0.clone(), y0.clone()
+    _native.bgmv_lora_multi([(together, x, plan, o, w) for plan, o, w in problems], rank, 1)
+    for plan, o, w in problems:
+        _native.bgmv_lora_multi([(apart, x, plan, o, w)], rank, 1)
+    torch.cuda.synchronize()
+    # (launches of another size may cut other column slices; an element's sums do not depend on it)
+    assert torch.equal(together, apart)
+    assert not torch.equal(together, y0)
+    assert torch.equal(together[:, :8], y0[:, :8]) and torch.equal(together[:, off:], y0[:, off:])
