@@ -477,6 +477,21 @@ int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
  * no multiple of 8, shapes that only the reference's prefill layouts serve), and LORAX_EINVAL for a num_tokens below
  * that of a table with a routing plan, whose records may name rows that x and y do not have.
  */
+/*
+ * The two routing rules of lorax_layer_update, for callers that issue the single entry points themselves (host only, no
+ * GPU state): whether the update of these projections of a decode batch goes out as single-launch updates
+ * (lorax_bgmv_lora_multi, one per rank) rather than as a shrink and an expand launch, and whether that of a rank's
+ * projections (the widest of `widest` columns) in a prefill batch does (lorax_sgmv_lora_multi).  1 = yes.
+ */
+typedef struct lorax_decode_job {
+  int32_t rank;
+  int32_t width;   /* columns of the projection  */
+  int32_t records; /* of its routing plan        */
+} lorax_decode_job_t;
+
+int lorax_decode_in_one_launch(const lorax_decode_job_t* jobs, int32_t num_jobs, int64_t num_tokens, int32_t h_in);
+int lorax_prefill_in_one_launch(int32_t rank, int32_t h_in, int64_t num_tokens, int32_t widest);
+
 typedef struct lorax_layer_slice {
   int32_t layer_type;
   int32_t width;

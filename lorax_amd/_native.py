@@ -207,6 +207,8 @@ _SIGNATURES = {
          _c.POINTER(_c.c_int32), _c.c_void_p, _c.c_int64, _c.POINTER(_c.c_int64), _c.POINTER(TableGroup), _c.c_int32,
          _c.POINTER(_c.c_int32)],
     ),
+    "lorax_decode_in_one_launch": (_c.c_int, [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32]),
+    "lorax_prefill_in_one_launch": (_c.c_int, [_c.c_int32, _c.c_int32, _c.c_int64, _c.c_int32]),
     "lorax_layer_update": (
         _c.c_int,
         [_c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64,
@@ -469,28 +471,20 @@ def bgmv_stacked(y, x, jobs, plan, scale=1.0) -> None:
         _raise_last(rc)
 
 
-FUSED_BGMV_RANKS = (8, 16)
+_DECODE_JOB = struct.Struct("3i")  # lorax_decode_job_t
 
 
-FEW_CHUNKS = {8: 64, 16: 16}  # plan records up to which wide projections run fused, by rank
+def decode_in_one_launch(jobs, num_tokens: int, h_in: int) -> bool:
+    """lorax_decode_in_one_launch: whether a decode batch's projections go out as single-launch updates (bgmv_lora_multi, one
+    per rank) rather than as a shrink and an expand launch.  `jobs`: (rank, columns, routing records) per projection."""
+    packed = b"".join([_DECODE_JOB.pack(*job) for job in jobs])
+    return lib().lorax_decode_in_one_launch(packed, len(jobs), num_tokens, h_in) != 0
 
 
-def bgmv_lora_fits(rank: int, h_in: int, h_out: int, few_chunks: bool = False) -> bool:
-    """True where the single-launch shrink+expand (lorax_bgmv_lora_multi) is the better choice: the adapter's
-    A slab is small (<= 128 KiB) and one workgroup covers all output columns of the projection (4096 at
-    rank 8, 2048 at rank 16), so no column slice has to repeat the shrink. Wider or deeper projections are
-    faster as a shrink launch plus an expand launch - unless the batch has few routing records (`few_chunks`: all jobs of one
-    rank, FEW_CHUNKS records at most): then the repeated shrinks run on idle CUs and the second launch is what costs.  A
-    Mistral-7B block at rank 16, fused against two launches: 18.6 and 23.5 us per layer at one record, 29 and 33 at 10, 39.5
-    both at 20, 61 and 58 at 43; at rank 8 16 and 18 us, 34.0 and 34.3 at 43, 53.2 and 53.0 at 84."""
-    if rank not in FUSED_BGMV_RANKS or rank * h_in * 2 > 128 * 1024:
-        return False
-    return h_out <= (256 // (rank // 8)) * 16 or (few_chunks and h_out <= 16384)
-
-
-def few_chunks(ranks, plan_sizes) -> bool:
-    """Whether a batch's jobs (their ranks and numbers of routing records) count as few in bgmv_lora_fits."""
-    return len(set(ranks)) == 1 and all(n <= FEW_CHUNKS.get(r, 0) for r, n in zip(ranks, plan_sizes))
+def bgmv_lora_fits(rank: int, h_in: int, h_out: int) -> bool:
+    """True where the single-launch shrink+expand (lorax_bgmv_lora_multi) is the better choice whatever the batch: the
+    adapter's A slab is small and one workgroup covers all output columns of the projection."""
+    return decode_in_one_launch([(rank, h_out, MAX_BGMV_TOKENS)], MAX_BGMV_TOKENS, h_in)
 
 
 def _check_stack(stack, x) -> None:
@@ -768,13 +762,10 @@ SGMV_LORA_MAX_TOKENS = 512
 
 
 def sgmv_lora_fits(rank: int, h_in: int, num_tokens: int, h_out: int = 0) -> bool:
-    """True where the single-launch prefill update (lorax_sgmv_lora_multi) applies and pays: rank 8 or 16 with a
-    small A slab, a batch short enough to be bound by launches, and an output that is not so wide (an LM head)
-    that recomputing the shrink in every column slice would dominate.  (Rank 16: every four rows read A again; a
-    Mistral-7B block of one run takes 49 us per layer in one launch per group and 51 in two at 128 rows, 61 and 54 at
-    192, 116 and 72 at 512.  Rank 8: 56 and 65 us at 512.)"""
-    return (rank in FUSED_BGMV_RANKS and rank * h_in * 2 <= 128 * 1024
-            and num_tokens <= (SGMV_LORA_MAX_TOKENS if rank == 8 else SGMV_LORA_MAX_TOKENS // 4) and h_out <= 16384)
+    """lorax_prefill_in_one_launch: True where the single-launch prefill update (lorax_sgmv_lora_multi) applies and pays -
+    rank 8 or 16 with a small A slab, a batch short enough to be bound by launches, and an output that is not so wide (an
+    LM head) that recomputing the shrink in every column slice would dominate."""
+    return lib().lorax_prefill_in_one_launch(rank, h_in, num_tokens, h_out) != 0
 
 
 def sgmv_lora_multi(problems, x, s_start, s_end, rank, layer_idx, scale: float = 1.0) -> None:

@@ -12,8 +12,10 @@ constexpr int kMaxJobs = 256;        // (projection, rank group) pairs of one ca
 constexpr int kMaxKernelRank = 128;
 constexpr int64_t kMaxBgmvRows = 65535;  // rows of a BGMV launch and records of one routing plan
 constexpr int64_t kShortBatchRows = 512;  // largest batch of the streaming shrink and of lorax_sgmv_lora_multi at rank 8
-constexpr int kFewChunks8 = 64, kFewChunks16 = 16;  // plan records up to which wide projections run fused, by rank
-constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 (measured: _native.sgmv_lora_fits)
+constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 (lorax_prefill_in_one_launch)
+constexpr int kFusedSlab = 128 * 1024;      // bytes of A that the single-launch updates read again per slice or row chunk
+constexpr int kFusedWidthMax = 16384;       // columns up to which repeating the shrink per slice can pay (an LM head: no)
+constexpr int kNumCus = 256;
 
 struct Job {
   const lorax_table_group_t* g;
@@ -37,19 +39,7 @@ struct Call {
   void* stream;
 };
 
-// The single-launch update pays where the A slab is small and, in decode, one workgroup covers the projection's
-// columns or the batch has few records (the rules of _native.bgmv_lora_fits and sgmv_lora_fits, where they are explained).
-bool fused_rank(int r, int h_in) { return (r == 8 || r == 16) && r * h_in * 2 <= 128 * 1024; }
-bool decode_fused(const Job& j, int h_in, bool one_rank) {
-  const int r = j.g->rank;
-  return fused_rank(r, h_in) && (j.width <= (256 / (r / 8)) * 16 ||
-                                 (one_rank && j.width <= 16384 && j.g->num_chunks <= (r == 8 ? kFewChunks8 : kFewChunks16)));
-}
-
-// A short prefill batch runs shrink and expand of a rank's projections in one launch over the segments.
-bool prefill_fused(int r, int h_in, int64_t rows, int widest) {
-  return fused_rank(r, h_in) && rows <= (r == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= 16384;
-}
+bool fused_rank(int r, int64_t h_in) { return (r == 8 || r == 16) && r * h_in * 2 <= kFusedSlab; }
 
 const void* at(const Call& c, int64_t off) { return c.tables + off; }
 
@@ -72,11 +62,9 @@ int bgmv_jobs(const Call& c, const Job* const* jobs, int count, bool shrink) {
 }
 
 int decode(const Call& c, Job* const* jobs, int count) {
-  bool fused = true;
-  bool one_rank = true;
-  for (int i = 0; i < count; ++i) one_rank = one_rank && jobs[i]->g->rank == jobs[0]->g->rank;
-  for (int i = 0; i < count; ++i) fused = fused && decode_fused(*jobs[i], c.h_in, one_rank);
-  if (fused) {
+  lorax_decode_job_t route[kMaxJobs];
+  for (int i = 0; i < count; ++i) route[i] = {jobs[i]->g->rank, jobs[i]->width, jobs[i]->g->num_chunks};
+  if (lorax_decode_in_one_launch(route, count, c.rows, c.h_in)) {
     for (int r : {8, 16}) {
       lorax_bgmv_problem_t p[lorax::kMaxFusedBgmvProblems];
       int n = 0;
@@ -123,7 +111,7 @@ int prefill(const Call& c, Job* const* jobs, int count) {
       widest = jobs[end]->width > widest ? jobs[end]->width : widest;
     const int32_t* starts = static_cast<const int32_t*>(at(c, g.starts_off));
     const int32_t* ends = static_cast<const int32_t*>(at(c, g.ends_off));
-    if (prefill_fused(g.rank, c.h_in, c.rows, widest)) {
+    if (lorax_prefill_in_one_launch(g.rank, c.h_in, c.rows, widest)) {
       for (int k = i; k < end; k += lorax::kMaxSgmvLoraProblems) {
         lorax_sgmv_lora_problem_t p[lorax::kMaxSgmvLoraProblems];
         int n = 0;
@@ -236,6 +224,40 @@ int update(const Call& c, const lorax_table_group_t* groups, int32_t num_groups,
 
 }  // namespace
 
+// The single-launch update (lorax_bgmv_lora_multi) pays where the A slab is small and one workgroup covers a
+// projection's columns (4096 at rank 8, 2048 at rank 16).  A wider projection is cut into slices that each repeat the
+// shrink, and is faster as a shrink launch plus an expand launch - unless the batch has few routing records: then the
+// repeated shrinks run on idle CUs and the second launch is what costs.  Measured at hidden sizes 1024 to 8192, 1 to 4
+// tokens per record, fused against two launches in us: 2 x 14336 columns at rank 8 (hidden 4096) 4.3 and 6.1 at 1
+// record, 9.9 and 11.0 at 32 of 4 tokens, 18.9 and 17.6 at 64 of 4 (512 slices for 256 CUs), 11.8 and 13.3 at 64 of 1;
+// one of 14336 9.8 and 10.6 at 64 of 4 (256 slices); 8192 + 1024 + 1024 over 8192 at rank 8 13.0 and 13.7 at 64 of 4;
+// 2 x 14336 at rank 16 (4096) 10.7 and 11.3 at 16 of 4, 19.6 and 17.0 at 32 of 4.  More slices than CUs pay only where
+// the records hold about one token each and the slab is at most half the limit (14336 + 1024 over 8192, 64 of 1: 12.2
+// and 11.2).
+extern "C" int lorax_decode_in_one_launch(const lorax_decode_job_t* jobs, int32_t num_jobs, int64_t num_tokens, int32_t h_in) {
+  if (num_jobs < 1 || jobs == nullptr) return 0;
+  bool wide = false, few = true;
+  int64_t slices = 0;
+  const int few_records = jobs[0].rank == 8 ? 64 : 16;
+  for (int i = 0; i < num_jobs; ++i) {
+    const lorax_decode_job_t& j = jobs[i];
+    if (!fused_rank(j.rank, h_in)) return 0;
+    const int cols = 256 / (j.rank / 8) * 16;
+    wide = wide || j.width > cols;
+    few = few && j.rank == jobs[0].rank && j.records <= few_records && j.width <= kFusedWidthMax;
+    slices += static_cast<int64_t>(j.records) * ((j.width + cols - 1) / cols);
+  }
+  if (!wide) return 1;
+  return few && (slices <= kNumCus || (num_tokens <= few_records && jobs[0].rank * h_in * 2 <= kFusedSlab / 2));
+}
+
+// The single-launch update of a short prefill batch (lorax_sgmv_lora_multi) reads A again for every four rows: a
+// Mistral-7B block of one run at rank 16 takes 49 us per layer in one launch per group and 51 in two at 128 rows, 61 and
+// 54 at 192, 116 and 72 at 512; at rank 8 56 and 65 at 512.
+extern "C" int lorax_prefill_in_one_launch(int32_t rank, int32_t h_in, int64_t num_tokens, int32_t widest) {
+  return fused_rank(rank, h_in) && num_tokens <= (rank == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= kFusedWidthMax;
+}
+
 extern "C" int lorax_layer_update(const lorax_table_group_t* groups, int32_t num_groups, const void* tables,
                                   const lorax_layer_slice_t* slices, int32_t num_slices, void* y, int64_t y_stride,
                                   const void* x, int64_t num_tokens, int32_t h_in, int64_t layer_idx, void* v, int64_t v_bytes,
@@ -252,7 +274,7 @@ extern "C" int lorax_layer_update(const lorax_table_group_t* groups, int32_t num
     for (int i = 0; i < num_groups; ++i) {
       const lorax_table_group_t& g = groups[i];
       if (g.layer_type != slices[s].layer_type || g.plan_off < 0 || num_tokens >= g.num_tokens) continue;
-      if (g.use_sgmv == 0 || !prefill_fused(g.rank, h_in, num_tokens, widest))
+      if (g.use_sgmv == 0 || !lorax_prefill_in_one_launch(g.rank, h_in, num_tokens, widest))
         return lorax::report_error(LORAX_EINVAL, "layer update: x and y have fewer rows than the batch of the routing tables");
     }
   const Call c{static_cast<const char*>(tables), y, y_stride, x, num_tokens, h_in, layer_idx, tmp, tmp_bytes, dtype, stream};

@@ -292,8 +292,8 @@ class LoraLinear(nn.Module):
         jobs = [(r, rs, start, width) for (_, r), rank_jobs in decode_jobs.items() for rs, start, width in rank_jobs]
         planned = bool(jobs) and not tensor_parallel and all(rs.plan is not None for _, rs, _, _ in jobs)
         _check_plan_rows(input.size(0), [rs for _, rs, _, _ in jobs if rs.plan is not None])
-        few = planned and _native.few_chunks([r for r, _, _, _ in jobs], [rs.plan.size(0) for _, rs, _, _ in jobs])
-        all_fused = planned and all(_native.bgmv_lora_fits(r, input.size(1), width, few) for r, _, _, width in jobs)
+        all_fused = planned and _native.decode_in_one_launch(
+            [(r, width, rs.plan.size(0)) for r, rs, _, width in jobs], input.size(0), input.size(1))
         if all_fused:
             step = _native.MAX_FUSED_BGMV_PROBLEMS
             for r in sorted({r for _, r in decode_jobs}):

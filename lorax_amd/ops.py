@@ -203,20 +203,22 @@ def bgmv_lora_slices(
     intermediate, and only at 1 do both round alike)."""
     assert inputs.dtype in (torch.float16, torch.bfloat16)
     assert inputs.is_contiguous() and output_tensor.is_contiguous()
-    assert inputs.size(0) == output_tensor.size(0)
+    tokens, h_in = inputs.shape
+    assert tokens == output_tensor.size(0)
     jobs = []
     for lora_a_weights, lora_b_weights, slice_offset, slice_size in slices:
         a = _stacked(lora_a_weights, "lora_a_weights")
         b = _stacked(lora_b_weights, "lora_b_weights")
         assert a.dtype == inputs.dtype and b.dtype == inputs.dtype
-        assert inputs.size(1) == a.size(-1) and a.size(-2) == b.size(-1) and slice_size == b.size(-2)
-        jobs.append((a, b, a.size(-2), slice_offset, slice_size))
-    if plan is not None and lora_indices_tensor.size(0) > inputs.size(0):
-        raise RuntimeError(f"the input has {inputs.size(0)} rows, fewer than the {lora_indices_tensor.size(0)} of the batch "
-                           "that its routing plan was built for")
-    few = plan is not None and _native.few_chunks([r for _, _, r, _, _ in jobs], [plan.size(0)] * len(jobs))
-    if plan is not None and scaling == 1.0 and all(
-            _native.bgmv_lora_fits(r, inputs.size(1), size, few) for _, _, r, _, size in jobs):
+        r = a.size(-2)
+        assert h_in == a.size(-1) and r == b.size(-1) and slice_size == b.size(-2)
+        jobs.append((a, b, r, slice_offset, slice_size))
+    records = plan.size(0) if plan is not None else 0
+    if plan is not None and lora_indices_tensor.size(0) > tokens:
+        raise RuntimeError(f"the input has {tokens} rows, fewer than the {lora_indices_tensor.size(0)} of the batch that its "
+                           "routing plan was built for")
+    if plan is not None and scaling == 1.0 and _native.decode_in_one_launch(
+            [(r, size, records) for _, _, r, _, size in jobs], tokens, h_in):
         step = _native.MAX_FUSED_BGMV_PROBLEMS
         for rank in sorted({r for _, _, r, _, _ in jobs}):
             same = [j for j in jobs if j[2] == rank]
@@ -226,7 +228,6 @@ def bgmv_lora_slices(
                                         rank, 0, 1.0, stacks=[(a, b) for a, b, _, _, _ in chunk])
         return
     step = _native.MAX_BGMV_PROBLEMS
-    tokens = inputs.size(0)
     for i in range(0, len(jobs), step):
         chunk = jobs[i : i + step]
         if plan is not None:

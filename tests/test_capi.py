@@ -121,6 +121,39 @@ def test_sgmv_shrink_groups_refuses_the_ranks_that_shrink_multi_refuses(rank, nu
         assert "No suitable kernel" in _err()
 
 
+@pytest.mark.parametrize("jobs,tokens,h_in,together", [
+    # one slice per projection: whatever the batch and the mix of ranks 8 and 16
+    ([(8, 4096, 65535), (16, 2048, 3)], 60000, 4096, True),
+    ([(8, 4096, 1)], 1, 8192, True), ([(8, 4096, 1)], 1, 8200, False), ([(16, 2048, 1)], 1, 4104, False),  # the slab
+    ([(32, 512, 1)], 1, 1024, False), ([(8, 512, 1), (24, 512, 1)], 1, 1024, False), ([], 1, 1024, False),
+    # wide projections: few records, one rank
+    ([(8, 14336, 64)], 256, 4096, True), ([(8, 14336, 65)], 65, 4096, False),
+    ([(16, 2056, 16)], 64, 4096, True), ([(16, 2056, 17)], 17, 4096, False),
+    ([(8, 4104, 1), (16, 512, 1)], 1, 1024, False),
+    ([(16, 4096, 16), (16, 1024, 17)], 17, 4096, False), ([(8, 8192, 3), (8, 1024, 65)], 65, 4096, False),  # a narrow one's count too
+    ([(8, 16384, 1)], 1, 1024, True), ([(8, 16392, 1)], 1, 1024, False), ([(8, 32000, 1), (8, 64, 1)], 1, 1024, False),
+    # more slices than CUs: about one token per record and at most half the slab
+    ([(8, 14336, 32)] * 2, 128, 8192, True), ([(8, 14336, 33)] * 2, 65, 4096, False), ([(8, 14336, 64)] * 2, 64, 4096, True),
+    ([(8, 14336, 64)] * 2, 65, 4096, False), ([(8, 14336, 64)] * 2, 64, 4104, False),
+    ([(8, 8192, 64), (8, 1024, 64), (8, 1024, 64)], 256, 8192, True), ([(16, 14336, 16)] * 2, 64, 4096, True),
+    ([(16, 14336, 16)] * 3, 64, 2048, False), ([(16, 14336, 16)] * 3, 16, 2048, True),
+])
+def test_decode_route(jobs, tokens, h_in, together):
+    """lorax_decode_in_one_launch at its bounds: the rule that the native layer call, the general path of the layers and the
+    stacked-weight operators share."""
+    assert _native.decode_in_one_launch(jobs, tokens, h_in) is together
+
+
+def test_single_launch_rules_for_one_projection():
+    for rank, width in ((8, 4096), (16, 2048)):
+        assert _native.bgmv_lora_fits(rank, 4096, width) and not _native.bgmv_lora_fits(rank, 4096, width + 8)
+    assert not _native.bgmv_lora_fits(32, 1024, 64) and not _native.bgmv_lora_fits(16, 8192, 64)
+    for rank, rows in ((8, 512), (16, 128)):
+        assert _native.sgmv_lora_fits(rank, 4096, rows, 16384) and not _native.sgmv_lora_fits(rank, 4096, rows + 1)
+        assert not _native.sgmv_lora_fits(rank, 4096, 1, 16392) and not _native.sgmv_lora_fits(rank, 65536 // rank + 8, 1)
+    assert not _native.sgmv_lora_fits(32, 1024, 1)
+
+
 def test_sgmv_lora_multi_validation():
     f = _native.lib().lorax_sgmv_lora_multi
     one = (_native.SgmvLoraProblem * 1)(_native.SgmvLoraProblem(P, P, P, 0, 4096, 4096))

@@ -729,3 +729,30 @@ def test_adapters_changed_in_the_dict_itself_reach_the_next_batch(change, prefil
     assert AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data["q_proj"][LORA].ranks() == {16}
     layer.adapter_weights.clear()
     assert layer.is_empty() and "q_proj" not in AdapterBatchData.from_meta(meta, {"q_proj": layer}, prefill=prefill).data
+
+
+@pytest.mark.parametrize("records,together", [((16, 9), True), ((17, 9), False), ((9, 17), False), ((16, 16), True)])
+def test_decode_paths_follow_the_one_rule(monkeypatch, records, together):
+    """The general path of the layers and the stacked-weight operators take the single launch exactly where the native
+    router does (lorax_decode_in_one_launch), also for projections of different record counts."""
+    from types import SimpleNamespace
+
+    from lorax_amd import _native, layers, ops
+
+    calls = []
+    for launch in ("bgmv_multi", "bgmv_lora_multi", "bgmv_stacked"):
+        monkeypatch.setattr(_native, launch, lambda *a, launch=launch, **k: calls.append(launch))
+    x, y = (torch.zeros((20, cols), dtype=torch.bfloat16) for cols in (1024, 4096 + 512))
+
+    def segments(n):
+        return SimpleNamespace(plan=torch.zeros((n, 8), dtype=torch.int64), num_rows=20, lora_a_ptr=None, lora_b_ptr=None,
+                               indices=None)
+
+    layers.LoraLinear(None, 0)._decode(y, x, {(0, 16): [(segments(records[0]), 0, 4096), (segments(records[1]), 4096, 512)]}, False)
+    assert calls == (["bgmv_lora_multi"] if together else ["bgmv_multi", "bgmv_multi"])
+    assert _native.decode_in_one_launch([(16, 4096, records[0]), (16, 512, records[1])], 20, 1024) is together
+    calls.clear()
+    a = torch.zeros(2, 16, 1024, dtype=torch.bfloat16)
+    ops.bgmv_lora_slices(x, [(a, torch.zeros(2, 4096, 16, dtype=torch.bfloat16), 0, 4096)], y, torch.zeros(20, dtype=torch.int64),
+                         1.0, plan=torch.zeros((records[0], 8), dtype=torch.int64))
+    assert calls == (["bgmv_lora_multi"] if records[0] <= 16 else ["bgmv_stacked"])
