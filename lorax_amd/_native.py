@@ -174,6 +174,11 @@ _SIGNATURES = {
         [_c.POINTER(SgmvShrinkGroup), _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_float, _c.c_int32,
          _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_void_p],
     ),
+    "lorax_sgmv_shrink_groups_parts": (
+        _c.c_int,
+        [_c.POINTER(SgmvShrinkGroup), _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_void_p,
+         _c.c_int64, _c.c_int32],
+    ),
     "lorax_sgmv_expand_planned": (
         _c.c_int,
         [_c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32,
@@ -698,9 +703,8 @@ def sgmv_shrink_multi(ys, x, w_ptrs, s_start, s_end, tmp, layer_idx, scale: floa
 MAX_SGMV_SHRINK_GROUPS = 16
 
 
-def sgmv_shrink_groups(groups, x, tmp, layer_idx, scale: float = 1.0, accumulate: bool = True) -> None:
-    """lorax_sgmv_shrink_groups: sgmv_shrink_multi for up to 16 groups over the same x, in one launch where they qualify.
-    `groups` is a list of tuples (ys, w_ptrs, s_start, s_end, tiles) as sgmv_shrink_multi takes them."""
+def _shrink_groups(groups, x, tmp):
+    """The C descriptors of `groups`, checked, and what they point to."""
     if not 1 <= len(groups) <= MAX_SGMV_SHRINK_GROUPS:
         raise RuntimeError(f"between 1 and {MAX_SGMV_SHRINK_GROUPS} groups per call, got {len(groups)}")
     if isinstance(tmp, torch.Tensor) and tmp.dtype != torch.uint8:
@@ -719,6 +723,13 @@ def sgmv_shrink_groups(groups, x, tmp, layer_idx, scale: float = 1.0, accumulate
         keep.append((problems, plan))
         arr[i] = SgmvShrinkGroup(problems, len(ys), ys[0].size(1), s_start.data_ptr(), s_end.data_ptr(), s_start.size(0),
                                  ctypes.addressof(plan) if plan is not None else None)
+    return arr, keep
+
+
+def sgmv_shrink_groups(groups, x, tmp, layer_idx, scale: float = 1.0, accumulate: bool = True) -> None:
+    """lorax_sgmv_shrink_groups: sgmv_shrink_multi for up to 16 groups over the same x, in one launch where they qualify.
+    `groups` is a list of tuples (ys, w_ptrs, s_start, s_end, tiles) as sgmv_shrink_multi takes them."""
+    arr, _keep = _shrink_groups(groups, x, tmp)
     _ready(x)
     with _on_device(x):
         rc = lib().lorax_sgmv_shrink_groups(arr, len(groups), x.data_ptr(), x.size(0), x.size(1), int(layer_idx), float(scale),
@@ -726,6 +737,15 @@ def sgmv_shrink_groups(groups, x, tmp, layer_idx, scale: float = 1.0, accumulate
                                             _dtype_code(x), _stream(x))
     if rc != 0:
         _raise_last(rc)
+
+
+def sgmv_shrink_groups_parts(groups, x, tmp, layer_idx, accumulate: bool = True) -> int:
+    """lorax_sgmv_shrink_groups_parts: the parts of the hidden dimension that sgmv_shrink_groups cuts for these arguments, 0
+    where it issues one call per group."""
+    arr, _keep = _shrink_groups(groups, x, tmp)
+    return lib().lorax_sgmv_shrink_groups_parts(arr, len(groups), x.data_ptr(), x.size(0), x.size(1), int(layer_idx),
+                                                1 if accumulate else 0, tmp.data_ptr(), tmp.numel() * tmp.element_size(),
+                                                _dtype_code(x))
 
 
 def plan_tiles(s_start, s_end, num_tokens: int, kind: int, rank: int = 0):

@@ -250,6 +250,8 @@ int sgmv_shrink_checked(void* v, const void* x, const int64_t* w_ptrs, const int
   return LORAX_OK;
 }
 
+constexpr int kMaxShrinkGroups = 16;
+
 // Shape checks of one expand problem (both B layouts).
 int check_expand(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start, const int32_t* s_end, int64_t num_tokens,
                  int32_t r, int32_t h_out, int64_t y_offset, int64_t y_stride, int32_t dtype) {
@@ -338,6 +340,57 @@ int sgmv_expand_checked(void* y, const void* v, const int64_t* w_ptrs, const int
   const hipError_t e = launch_sgmv_expand(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_expand launch failed: %s", hipGetErrorString(e));
   return LORAX_OK;
+}
+
+// The launch arguments of groups that can go out as one launch: fills args and returns how many have rows, 0 where the
+// groups have to be shrunk one call each.
+int shrink_groups_together(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x, int64_t num_tokens,
+                           int32_t h_in, int64_t layer_idx, float scale, int32_t accumulate, void* tmp, int64_t tmp_bytes,
+                           int32_t dtype, SgmvArgs (&args)[kMaxShrinkGroups]) {
+  const int rows_max = tuning().shrink_rows_max != 0 ? tuning().shrink_rows_max : 512;
+  // one launch: planned tiles of a batch past the streaming kernel's range, stacked ranks of one A tile each.  The
+  // kernels store four columns of v at a time and take a store's projection from its first column, so each projection's
+  // own rank has to be a multiple of 8, not only their sum; other ranks go to lorax_sgmv_shrink_multi, which refuses them.
+  int count = 0;
+  bool together = num_groups > 1 && num_tokens > rows_max && num_tokens <= INT32_MAX / 2 && h_in > 0 && layer_idx >= 0 &&
+                  (accumulate == 0 || accumulate == 1) && tmp != nullptr && aligned16(tmp) &&
+                  tmp_bytes >= LORAX_SHRINK_TMP_BYTES;
+  for (int i = 0; i < num_groups && together; ++i) {
+    const lorax_sgmv_shrink_group_t& g = groups[i];
+    together = g.num_problems >= 1 && g.num_problems <= kMaxShrinkGroup && g.problems != nullptr && g.r >= 8 &&
+               g.r % 8 == 0 && g.r <= kMaxRank / g.num_problems && g.s_start != nullptr && g.s_end != nullptr && g.num_segments > 0 &&
+               g.tiles != nullptr && g.tiles->tiles != nullptr;
+    if (!together) break;
+    SgmvArgs& a = args[count];
+    a = SgmvArgs{};
+    if (take_tiles(g.tiles, a) != LORAX_OK) together = false;
+    if (g.tiles->num_tiles == 0) continue;  // no segment has rows
+    for (int k = 0; k < g.num_problems && together; ++k) {
+      together = check_common(g.problems[k].v, x, g.problems[k].w_ptrs, dtype) == LORAX_OK;
+      a.group.v[k] = g.problems[k].v;
+      a.group.w[k] = g.problems[k].w_ptrs;
+    }
+    a.group.count = g.num_problems;
+    a.group.rank = g.r;
+    a.y = g.problems[0].v;
+    a.w_ptrs = g.problems[0].w_ptrs;
+    a.x = x;
+    a.s_start = g.s_start;
+    a.s_end = g.s_end;
+    a.num_segments = g.num_segments;
+    a.num_tokens = num_tokens;
+    a.d_in = h_in;
+    a.d_out = g.num_problems * g.r;
+    a.a_layout = LORAX_A_RH;
+    a.layer_idx = layer_idx;
+    a.dtype = dtype;
+    a.scale = scale;
+    a.accumulate = accumulate;
+    a.partials = static_cast<float*>(tmp);
+    a.partial_bytes = static_cast<size_t>(tmp_bytes);
+    ++count;
+  }
+  return together && sgmv_shrink_groups_applies(args, count) ? count : 0;
 }
 
 }  // namespace
@@ -492,55 +545,13 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
 int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x, int64_t num_tokens,
                              int32_t h_in, int64_t layer_idx, float scale, int32_t accumulate, void* tmp, int64_t tmp_bytes,
                              int32_t dtype, void* stream) {
-  constexpr int kMaxGroups = 16;
-  if (num_groups < 0 || num_groups > kMaxGroups)
-    return fail(LORAX_EINVAL, "num_groups=%d (at most %d per call)", num_groups, kMaxGroups);
+  if (num_groups < 0 || num_groups > kMaxShrinkGroups)
+    return fail(LORAX_EINVAL, "num_groups=%d (at most %d per call)", num_groups, kMaxShrinkGroups);
   if (num_groups > 0 && groups == nullptr) return fail(LORAX_EINVAL, "null pointer argument (groups)");
-  const int rows_max = tuning().shrink_rows_max != 0 ? tuning().shrink_rows_max : 512;
-  // one launch: planned tiles of a batch past the streaming kernel's range, stacked ranks of one A tile each.  The
-  // kernels store four columns of v at a time and take a store's projection from its first column, so each projection's
-  // own rank has to be a multiple of 8, not only their sum; other ranks go to the calls below, which refuse them.
-  SgmvArgs args[kMaxGroups];
-  int count = 0;
-  bool together = num_groups > 1 && num_tokens > rows_max && num_tokens <= INT32_MAX / 2 && h_in > 0 && layer_idx >= 0 &&
-                  (accumulate == 0 || accumulate == 1) && tmp != nullptr && aligned16(tmp) &&
-                  tmp_bytes >= LORAX_SHRINK_TMP_BYTES;
-  for (int i = 0; i < num_groups && together; ++i) {
-    const lorax_sgmv_shrink_group_t& g = groups[i];
-    together = g.num_problems >= 1 && g.num_problems <= kMaxShrinkGroup && g.problems != nullptr && g.r >= 8 &&
-               g.r % 8 == 0 && g.r <= kMaxRank / g.num_problems && g.s_start != nullptr && g.s_end != nullptr && g.num_segments > 0 &&
-               g.tiles != nullptr && g.tiles->tiles != nullptr;
-    if (!together) break;
-    SgmvArgs& a = args[count];
-    a = SgmvArgs{};
-    if (take_tiles(g.tiles, a) != LORAX_OK) together = false;
-    if (g.tiles->num_tiles == 0) continue;  // no segment has rows
-    for (int k = 0; k < g.num_problems && together; ++k) {
-      together = check_common(g.problems[k].v, x, g.problems[k].w_ptrs, dtype) == LORAX_OK;
-      a.group.v[k] = g.problems[k].v;
-      a.group.w[k] = g.problems[k].w_ptrs;
-    }
-    a.group.count = g.num_problems;
-    a.group.rank = g.r;
-    a.y = g.problems[0].v;
-    a.w_ptrs = g.problems[0].w_ptrs;
-    a.x = x;
-    a.s_start = g.s_start;
-    a.s_end = g.s_end;
-    a.num_segments = g.num_segments;
-    a.num_tokens = num_tokens;
-    a.d_in = h_in;
-    a.d_out = g.num_problems * g.r;
-    a.a_layout = LORAX_A_RH;
-    a.layer_idx = layer_idx;
-    a.dtype = dtype;
-    a.scale = scale;
-    a.accumulate = accumulate;
-    a.partials = static_cast<float*>(tmp);
-    a.partial_bytes = static_cast<size_t>(tmp_bytes);
-    ++count;
-  }
-  if (together && sgmv_shrink_groups_applies(args, count)) {
+  SgmvArgs args[kMaxShrinkGroups];
+  const int count = shrink_groups_together(groups, num_groups, x, num_tokens, h_in, layer_idx, scale, accumulate, tmp, tmp_bytes,
+                                           dtype, args);
+  if (count > 0) {
     const hipError_t e = launch_sgmv_shrink_groups(args, count, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_shrink launch failed: %s", hipGetErrorString(e));
     return LORAX_OK;
@@ -552,6 +563,16 @@ int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t nu
       return rc;
   }
   return LORAX_OK;
+}
+
+int lorax_sgmv_shrink_groups_parts(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x,
+                                   int64_t num_tokens, int32_t h_in, int64_t layer_idx, int32_t accumulate, void* tmp,
+                                   int64_t tmp_bytes, int32_t dtype) {
+  if (num_groups < 0 || num_groups > kMaxShrinkGroups || groups == nullptr) return 0;
+  SgmvArgs args[kMaxShrinkGroups];
+  const int count = shrink_groups_together(groups, num_groups, x, num_tokens, h_in, layer_idx, 1.0f, accumulate, tmp, tmp_bytes,
+                                           dtype, args);
+  return count > 0 ? sgmv_shrink_groups_kparts(args, count) : 0;
 }
 
 int lorax_sgmv_expand(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start,

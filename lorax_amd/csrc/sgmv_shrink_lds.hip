@@ -628,13 +628,42 @@ static hipError_t raise_groups_lds_limit() {
   return e;
 }
 
+// Blocks of a group's stage buffers and A tile.
+static int group_nb(const SgmvArgs& g) { return (g.d_out + 15) / 16; }
+static int group_mblk(const SgmvArgs& g) { return (g.tile_rows + 15) / 16; }
+static int group_stage_bytes(const SgmvArgs& g) { return (group_mblk(g) + group_nb(g)) * 16 * kLdsRowBytes; }
+
+// Parts the hidden dimension of a launch of several groups is cut into.  A CU streams about 50 KB/us, so the launch takes
+// as long as the workgroups of its busiest CU; parts are worth their second launch (4 us, and the sums written and read)
+// where they even that out.
+int sgmv_shrink_groups_kparts(const SgmvArgs* groups, int count) {
+  if (fixed_order_shrink()) return 1;
+  const int nst = groups[0].d_in / kLdsKc;
+  int64_t tiles = 0;
+  double tile_us = 0, sum_bytes = 0;  // of all tiles: time at a CU's 50 KB/us, fp32 sums of one part
+  for (int i = 0; i < count; ++i) {
+    const SgmvArgs& g = groups[i];
+    tiles += g.num_tiles;
+    tile_us += g.num_tiles * static_cast<double>(group_stage_bytes(g)) * nst / 50e3;
+    sum_bytes += static_cast<double>(g.num_tiles) * group_mblk(g) * 16 * group_nb(g) * 16 * sizeof(float);
+  }
+  int kparts = 1;
+  double best = 0;
+  for (int k = 1; k <= 8 && k <= (nst >= 16 ? nst / 8 : 1); ++k) {
+    if (k > 1 && k * sum_bytes > static_cast<double>(kPartialBytes)) break;
+    const double us = static_cast<double>((tiles * k + 255) / 256) * (tile_us / tiles) / k + (k > 1 ? 4.0 + 2e-6 * k * sum_bytes / 2.0 : 0.0);
+    if (k == 1 || us < best) best = us, kparts = k;
+  }
+  if (tuning().shrink_ksplit > 0 && tuning().shrink_ksplit <= nst && tuning().shrink_ksplit * sum_bytes <= static_cast<double>(kPartialBytes))
+    kparts = tuning().shrink_ksplit;
+  return kparts;
+}
+
 template <typename D>
 static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStream_t stream) {
   const SgmvArgs& a = groups[0];
-  const int nst = a.d_in / kLdsKc;
   ShrinkLaunch b{};
   int64_t tiles = 0;
-  double tile_us = 0, sum_bytes = 0;  // of all tiles: time at a CU's 50 KB/us, fp32 sums of one part
   int stage_max = 0;
   for (int i = 0; i < count; ++i) {
     const SgmvArgs& g = groups[i];
@@ -645,27 +674,13 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
     s.tiles = g.tiles;
     s.num_segments = g.num_segments;
     s.num_tiles = g.num_tiles;
-    s.nb = (g.d_out + 15) / 16;
-    s.mblk = (g.tile_rows + 15) / 16;
+    s.nb = group_nb(g);
+    s.mblk = group_mblk(g);
     tiles += s.num_tiles;
-    const int stage = (s.mblk + s.nb) * 16 * kLdsRowBytes;
+    const int stage = group_stage_bytes(g);
     stage_max = stage > stage_max ? stage : stage_max;
-    tile_us += s.num_tiles * static_cast<double>(stage) * nst / 50e3;
-    sum_bytes += static_cast<double>(s.num_tiles) * s.mblk * 16 * s.nb * 16 * sizeof(float);
   }
-  // K parts: a CU streams about 50 KB/us, so the launch takes as long as the workgroups of its busiest CU; parts are
-  // worth their second launch (4 us, and the sums written and read) where they even that out.
-  int kparts = 1;
-  if (!fixed_order_shrink()) {
-    double best = 0;
-    for (int k = 1; k <= 8 && k <= (nst >= 16 ? nst / 8 : 1); ++k) {
-      if (k > 1 && k * sum_bytes > static_cast<double>(kPartialBytes)) break;
-      const double us = static_cast<double>((tiles * k + 255) / 256) * (tile_us / tiles) / k + (k > 1 ? 4.0 + 2e-6 * k * sum_bytes / 2.0 : 0.0);
-      if (k == 1 || us < best) best = us, kparts = k;
-    }
-    if (tuning().shrink_ksplit > 0 && tuning().shrink_ksplit <= nst && tuning().shrink_ksplit * sum_bytes <= static_cast<double>(kPartialBytes))
-      kparts = tuning().shrink_ksplit;
-  }
+  const int kparts = sgmv_shrink_groups_kparts(groups, count);
   const int64_t wgs = tiles * kparts;
   // stage buffers as in launch_lds_m, but never less than two stages of the largest group
   int budget = wgs <= 256 ? 150 * 1024 : (wgs <= 768 ? 50 * 1024 : 76 * 1024);
@@ -676,7 +691,7 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
   float* sums = a.partials;
   for (int i = 0; i < count; ++i) {
     ShrinkSlot& s = b.p[i];
-    const int stage = (s.mblk + s.nb) * 16 * kLdsRowBytes;
+    const int stage = group_stage_bytes(groups[i]);
     const int red = 4 * s.mblk * s.nb * 1024;
     s.stages = budget / stage < kLdsMaxStages ? budget / stage : kLdsMaxStages;
     if (s.stages * stage > lds_bytes) lds_bytes = s.stages * stage;

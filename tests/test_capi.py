@@ -154,6 +154,27 @@ def test_single_launch_rules_for_one_projection():
     assert not _native.sgmv_lora_fits(32, 1024, 1)
 
 
+@pytest.mark.parametrize("ranks,problems,tile_rows,rows,h_in,one_launch", [
+    ((16, 64), 2, 16, 1000, 4096, True), ((8, 128), 1, 32, 513, 256, True), ((16, 32), 4, 16, 1000, 1024, True),
+    ((16, 64), 2, 16, 512, 4096, False), ((16, 64), 2, 48, 1000, 4096, False), ((16, 64), 2, 16, 1000, 4104, False),
+    ((16, 64), 4, 16, 1000, 4096, False), ((16, 12), 2, 16, 1000, 4096, False), ((16,), 2, 16, 1000, 4096, False),
+])
+def test_sgmv_shrink_groups_route(ranks, problems, tile_rows, rows, h_in, one_launch):
+    f = _native.lib().lorax_sgmv_shrink_groups_parts
+    made = [_shrink_groups(r, problems, 1, tile_rows) for r in ranks]
+    groups = (_native.SgmvShrinkGroup * len(ranks))(*[g[0] for g, _ in made])
+    big = 8 * 1024 * 1024
+    assert (f(groups, len(ranks), P, rows, h_in, 0, 0, P, big, 1) > 0) is one_launch
+    for layer, accumulate, tmp, size, dtype in ((-1, 0, P, big, 1), (0, 2, P, big, 1), (0, 0, None, big, 1), (0, 0, P + 4, big, 1),
+                                                (0, 0, P, big - 1, 1), (0, 0, P, big, 2)):
+        assert f(groups, len(ranks), P, rows, h_in, layer, accumulate, tmp, size, dtype) == 0
+    # parts only as far as their fp32 sums fit the scratch: 40 tiles of rank 128 take 320 KB each
+    made = [_shrink_groups(64, 2, 1, 16) for _ in range(16)]
+    groups = (_native.SgmvShrinkGroup * 16)(*[g[0] for g, _ in made])
+    for count in range(2, 17):
+        assert 1 <= f(groups, count, P, 12000, 128 * 67, 0, 0, P, big, 1) <= max(1, (big - 65536) // (count * 40 * 16 * 128 * 4))
+
+
 def test_sgmv_lora_multi_validation():
     f = _native.lib().lorax_sgmv_lora_multi
     one = (_native.SgmvLoraProblem * 1)(_native.SgmvLoraProblem(P, P, P, 0, 4096, 4096))

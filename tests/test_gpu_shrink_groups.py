@@ -1,6 +1,7 @@
 """lorax_sgmv_shrink_groups: the shrinks of several rank groups over one x in one launch, against fp64 and against one
-launch per group.  Sizes at the edges: one-row tiles, 16- and 32-row tiles, every stacked rank, hidden sizes whose stages do
-not divide among the parts, groups without rows, more tiles than CUs."""
+launch per group.  Sizes at the edges: one-row tiles, 16- and 32-row tiles, every stacked rank, groups without rows, more
+tiles than CUs; and launches that cut the hidden dimension into parts, of stages that do not divide among them.  ROUTES says
+what each case has to run as, so that none compares the calls per group with themselves."""
 
 import pytest
 import torch
@@ -28,9 +29,22 @@ CASES = {
     "four ranks": (1024, [(8, 3, [100, 1, 33]), (16, 3, [17, 200]), (32, 3, [90, 16]), (64, 2, [130])]),
     "every stacked rank": (384, [(8, 1, [70]), (32, 1, [71]), (24, 2, [72]), (64, 1, [73]), (40, 2, [74]), (48, 2, [75]),
                                  (56, 2, [76]), (128, 1, [77])]),
-    "stages that do not divide": (128 * 17, [(16, 1, [300]), (64, 2, [300, 1, 1])]),
+    "an odd number of stages": (128 * 17, [(16, 1, [300]), (64, 2, [300, 1, 1])]),
     "a group without rows": (512, [(16, 2, [300]), (8, 1, [0]), (32, 1, [250])]),
     "many tiles": (256, [(64, 2, [1500]), (128, 1, [33] * 60)]),
+    "32-row tiles": (256, [(128, 1, [4096]), (64, 1, [64])]),
+    # 67 stages in 6, 7, 5 and 3 parts
+    "parts, four ranks": (128 * 67, [(8, 3, [100, 1, 33]), (16, 3, [17, 200]), (32, 3, [90, 16]), (64, 2, [130])]),
+    "parts, a group without rows": (128 * 67, [(16, 2, [300]), (8, 1, [0]), (32, 1, [250])]),
+    "parts, every stacked rank": (128 * 67, [(8, 1, [700]), (16, 1, [33] * 9), (24, 1, [71]), (40, 2, [9]), (48, 2, [17]),
+                                             (56, 2, [31]), (128, 1, [65])]),
+    "parts, 32-row tiles": (128 * 67, [(128, 1, [4096]), (64, 1, [64])]),
+}
+# (parts of the hidden dimension, heights of the groups' tiles)
+ROUTES = {
+    "four ranks": (1, {16}), "every stacked rank": (1, {16}), "an odd number of stages": (1, {16}),
+    "a group without rows": (1, {16}), "many tiles": (1, {16}), "32-row tiles": (1, {16, 32}), "parts, four ranks": (6, {16}),
+    "parts, a group without rows": (7, {16}), "parts, every stacked rank": (5, {16}), "parts, 32-row tiles": (3, {16, 32}),
 }
 
 
@@ -51,6 +65,10 @@ def test_groups_in_one_launch(case, accumulate, dtype):
             pos += n
         groups.append(_group(rank, count, spans, rows, h_in, dtype, gen))
     tmp = get_shrink_scratch(DEV)
+    shrinks = [(list(g[5].unbind(0)), g[1], g[2], g[3], g[4]) for g in groups]
+    parts, heights = ROUTES[case]
+    assert {g[4].tile_rows for g in groups} == heights
+    assert _native.sgmv_shrink_groups_parts(shrinks, x, tmp, 1, accumulate) == parts
 
     def run(apart):
         vs = [g[5].clone() for g in groups]
@@ -81,7 +99,23 @@ def test_groups_in_one_launch(case, accumulate, dtype):
     # fixed-order sums do not depend on how the groups are launched
     before = _native.set_fixed_order_shrink(True)
     try:
+        assert _native.sgmv_shrink_groups_parts(shrinks, x, tmp, 1, accumulate) == 1
         for a, b in zip(run(False), run(True)):
             assert torch.equal(a, b)
     finally:
         _native.set_fixed_order_shrink(before)
+
+
+@pytest.mark.parametrize("rank,count", [(10, 4), (12, 2), (18, 4), (12, 4)])
+def test_other_ranks_are_refused(rank, count):
+    gen = torch.Generator().manual_seed(rank)
+    x = torch.randn((600, 256), generator=gen).to(torch.bfloat16).cuda()
+    calls = []
+    for start in (0, 300):
+        _, tables, s, e, tiles, v = _group(rank, count, [(start, start + 300)], 600, 256, torch.bfloat16, gen)
+        calls.append((list(v.unbind(0)), tables, s, e, tiles))
+    before = [[v.clone() for v in vs] for vs, *_ in calls]
+    with pytest.raises(RuntimeError, match="No suitable kernel"):
+        _native.sgmv_shrink_groups(calls, x, get_shrink_scratch(DEV), 0)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for vs, old in zip((c[0] for c in calls), before) for a, b in zip(vs, old))
