@@ -255,18 +255,20 @@ int lorax_sgmv_plan_tiles(const int32_t* s_start, const int32_t* s_end, int32_t 
  * SGMV shrink of up to 4 projections that share x, the segments and the rank (q/k/v, gate/up), LORAX_A_RH
  * stacks: problem p gets v_p[s:e, :] += dtype(scale * x[s:e, :] @ A_p^T) exactly as from lorax_sgmv_shrink
  * with (v_p, w_ptrs_p).  The reference launches one shrink per projection (lorax_server/utils/layers.py:
- * 121-133, punica_ops.cc:369-411) and reads x once per launch; here, when num_problems * r <= 128, h_in is a
- * multiple of 128 and the batch has more than 512 rows, the projections run as ONE launch that reads x once
- * (their A matrices are stacked into one rank-(num_problems * r) tile).  Otherwise the call issues one
- * launch per projection.  `tmp`/`tmp_bytes`: at least LORAX_SHRINK_TMP_BYTES of scratch, as for lorax_sgmv_shrink
+ * 121-133, punica_ops.cc:369-411) and reads x once per launch; here the projections run as ONE launch
+ *   - in a batch of up to 512 rows, whatever their summed rank (a streaming kernel; h_in a multiple of 8),
+ *   - in a larger one when num_problems * r <= 128 and h_in is a multiple of 128: it reads x once (their A matrices are
+ *     stacked into one rank-(num_problems * r) tile) and may be followed by one that adds the parts of a split h_in.
+ * Otherwise the call issues one launch per projection.
+ * `tmp`/`tmp_bytes`: at least LORAX_SHRINK_TMP_BYTES of scratch, as for lorax_sgmv_shrink
  * with LORAX_A_RH; a larger buffer is accepted and changes nothing (a launch that splits the hidden dimension
  * across workgroups keeps its fp32 partial sums in the first 8 MiB, so that the result does not depend on the
  * buffer's size).  num_problems = 1 is allowed.
  * accumulate = 1 adds to v as lorax_sgmv_shrink does; accumulate = 0 stores dtype(scale * x @ A^T) into the rows
  * of the segments instead, so the caller need not zero v first (rows outside every segment keep their contents;
  * lorax_sgmv_expand reads no others).  The reference zero-fills v before every shrink (punica.py:176-178).
- * `tiles`: optional row-tile plan (LORAX_TILES_SHRINK) for the call's segment tables, or NULL; it is used by the
- * one-launch path and ignored otherwise.
+ * `tiles`: optional row-tile plan (LORAX_TILES_SHRINK) for the call's segment tables, or NULL; it is used in batches of
+ * more than 512 rows that run as one launch (a single projection of such a shape among them) and ignored otherwise.
  * Order of the sums: a row tile walks the hidden dimension from a starting point that depends on the tile (its
  * adapter's stack address, its number inside the segment, the XCD it runs on), and launches with few tiles cut
  * the hidden dimension into parts whose fp32 sums are added afterwards.  A call is deterministic, but the last

@@ -375,15 +375,14 @@ def bgmv(y, x, w_ptr, indicies, layer_idx, scale, y_offset=0, y_slice_size=None)
 PLAN_RECORD_WORDS = 8
 
 
-def bgmv_multi(problems, layer_idx, scale=1.0, accumulate=True, plans=None, stacks=None) -> None:
+def bgmv_multi(problems, layer_idx, scale=1.0, accumulate=True, plans=None) -> None:
     """lorax_bgmv_multi: `problems` is a list of up to 16 tuples (y, x, w_ptr, indicies, y_offset, y_slice_size)
     that share the token count and the direction; shrink problems share x.shape and may differ in rank
     (y's width), expand problems may differ in rank (x's width) and output width.  y_slice_size None means
     the whole width of y.
     `plans`, if given, holds one routing plan per problem: an int64 device tensor [num_groups, 8]; w_ptr and
-    indicies of a planned problem may then be None (the kernels read the plan only).
-    `stacks` (with plans): per problem the stacked weight tensor [num_adapters, rows, cols] whose entry numbers the
-    plan's address words hold - lora_a stacks for a shrink launch, lora_b stacks for an expand launch."""
+    indicies of a planned problem may then be None (the kernels read the plan only).  Plans over stacked weights:
+    bgmv_stacked."""
     if not 1 <= len(problems) <= MAX_BGMV_PROBLEMS:
         raise RuntimeError(f"between 1 and {MAX_BGMV_PROBLEMS} problems per launch, got {len(problems)}")
     arr = (BgmvProblem * len(problems))()
@@ -417,13 +416,9 @@ def bgmv_multi(problems, layer_idx, scale=1.0, accumulate=True, plans=None, stac
             plan_ptr, num_groups = plan.data_ptr(), plan.size(0)
             if num_groups == 0:
                 plan_ptr = x.data_ptr()  # an empty plan has no storage; any non-null address will do
-        stack = None
-        if stacks is not None and plans is not None:
-            _check_stack(stacks[i], x)
-            stack = stacks[i].data_ptr()
         arr[i] = BgmvProblem(y.data_ptr(), x.data_ptr(), None if planned_only else w_ptr.data_ptr(),
                              None if planned_only else indicies.data_ptr(), int(y_offset),
-                             y.size(1), h_out, plan_ptr, num_groups, x.size(1), stack, stack)
+                             y.size(1), h_out, plan_ptr, num_groups, x.size(1), None, None)
     with _on_device(x0):
         rc = lib().lorax_bgmv_multi(arr, len(problems), x0.size(0), x0.size(1), int(layer_idx), float(scale),
                                     1 if accumulate else 0, _dtype_code(x0), _stream(x0))
