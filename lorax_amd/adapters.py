@@ -540,21 +540,24 @@ class BatchLoraWeights(BatchAdapterWeights):
 
 
 class _AdapterDict(dict):
-    """A dict that counts its changes, so that what is derived from it is rebuilt after any of them."""
+    """A dict that drops what LayerAdapterWeights has derived from it with every change."""
 
-    version = 0
+    lora_entries = None
+    unwrapped = None
 
 
-def _counting(method):
+def _dropping(method):
     def change(self, *args, **kwargs):
-        self.version += 1
-        return method(self, *args, **kwargs)
+        try:
+            return method(self, *args, **kwargs)
+        finally:
+            self.lora_entries = self.unwrapped = None
 
     return change
 
 
 for _name in ("__setitem__", "__delitem__", "__ior__", "clear", "pop", "popitem", "setdefault", "update"):
-    setattr(_AdapterDict, _name, _counting(getattr(dict, _name)))
+    setattr(_AdapterDict, _name, _dropping(getattr(dict, _name)))
 
 
 class LayerAdapterWeights:
@@ -570,7 +573,6 @@ class LayerAdapterWeights:
     @adapter_weights.setter
     def adapter_weights(self, weights: Dict[int, AdapterWeights]) -> None:
         self._adapter_weights = _AdapterDict(weights)
-        self._derived_from = None
 
     def add_adapter(self, adapter_idx: int, weights: AdapterWeights):
         self._adapter_weights[adapter_idx] = weights
@@ -578,46 +580,40 @@ class LayerAdapterWeights:
     def remove_adapter(self, adapter_idx: int):
         self._adapter_weights.pop(adapter_idx, None)
 
-    def _drop_stale(self) -> None:
-        if self._derived_from != self._adapter_weights.version:
-            self._derived_from = self._adapter_weights.version
-            self._lora_entries = None  # cached argument of the native table builder
-            self._unwrapped = None
-
     def unwrapped(self) -> Dict[int, "AdapterWeights"]:
         """adapter index -> the adapter's weights without their wrapper; rebuilt only when adapters come or go."""
-        self._drop_stale()
-        if self._unwrapped is None:
-            self._unwrapped = {idx: _unwrap(w) for idx, w in self.adapter_weights.items()}
-        return self._unwrapped
+        adapters = self._adapter_weights
+        if adapters.unwrapped is None:
+            adapters.unwrapped = {idx: _unwrap(w) for idx, w in adapters.items()}
+        return adapters.unwrapped
 
     def lora_entries(self):
         """(adapter, address of the [L, r, h_in] stack, address of the [L, h_out, r] stack, rank) of every LoRA
         adapter of the layer type, sorted by adapter, as a numpy array of _native.ENTRY_DTYPE; None if an adapter
         of another kind, or of a rank above the kernels' 128, is loaded.  Rebuilt only when adapters come or go."""
-        self._drop_stale()
-        if self._lora_entries is None:
+        adapters = self._adapter_weights
+        if adapters.lora_entries is None:
             import numpy as np
 
             from lorax_amd import _native
 
             rows = []
-            for idx in sorted(self.adapter_weights):
-                w = _unwrap(self.adapter_weights[idx])
+            for idx in sorted(adapters):
+                w = _unwrap(adapters[idx])
                 if not isinstance(w, LoraWeights) or w.get_batch_types() != [BatchLoraWeights]:
                     return None
                 if w.lora_a_r > MAX_RANK_CUSTOM:
                     return None  # served in rank chunks, which the per-layer-type Python path builds
                 rows.append((idx, w.weights_a_t.data_ptr(), w.weights_b_t.data_ptr(), w.lora_a_r, 0))
-            self._lora_entries = np.array(rows, dtype=_native.ENTRY_DTYPE)
-        return self._lora_entries
+            adapters.lora_entries = np.array(rows, dtype=_native.ENTRY_DTYPE)
+        return adapters.lora_entries
 
     @property
     def max_speculative_tokens(self) -> int:
         return max(w.speculative_tokens for w in self.adapter_weights.values())
 
     def is_empty(self) -> bool:
-        return not self.adapter_weights
+        return not self._adapter_weights
 
     def get_data(
         self,

@@ -152,6 +152,12 @@ def test_single_launch_rules_for_one_projection():
         assert _native.sgmv_lora_fits(rank, 4096, rows, 16384) and not _native.sgmv_lora_fits(rank, 4096, rows + 1)
         assert not _native.sgmv_lora_fits(rank, 4096, 1, 16392) and not _native.sgmv_lora_fits(rank, 65536 // rank + 8, 1)
     assert not _native.sgmv_lora_fits(32, 1024, 1)
+    # the short batches that the Python paths know are the C rule's
+    from lorax_amd.sgmv import resident_shrink_applies
+
+    short = _native.SGMV_LORA_MAX_TOKENS
+    assert _native.sgmv_lora_fits(8, 1024, short) and not _native.sgmv_lora_fits(8, 1024, short + 1)
+    assert resident_shrink_applies(24, 200, short) and not resident_shrink_applies(24, 200, short + 1)
 
 
 @pytest.mark.parametrize("ranks,problems,tile_rows,rows,h_in,one_launch", [
