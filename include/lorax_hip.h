@@ -259,7 +259,7 @@ int lorax_sgmv_plan_tiles(const int32_t* s_start, const int32_t* s_end, int32_t 
  *   - in a batch of up to 512 rows, whatever their summed rank (a streaming kernel; h_in a multiple of 8),
  *   - in a larger one when num_problems * r <= 128 and h_in is a multiple of 128: it reads x once (their A matrices are
  *     stacked into one rank-(num_problems * r) tile) and may be followed by one that adds the parts of a split h_in.
- * Otherwise the call issues one launch per projection.
+ * Otherwise, and where two projections name the same v, the call issues one launch per projection.
  * `tmp`/`tmp_bytes`: at least LORAX_SHRINK_TMP_BYTES of scratch, as for lorax_sgmv_shrink
  * with LORAX_A_RH; a larger buffer is accepted and changes nothing (a launch that splits the hidden dimension
  * across workgroups keeps its fp32 partial sums in the first 8 MiB, so that the result does not depend on the
@@ -292,8 +292,8 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
  * lorax_sgmv_shrink_multi for up to 16 groups of projections over the same x - the rank groups of a batch whose
  * adapters differ in rank, projections whose summed rank exceeds 128 - in one launch (and one that adds the parts of a
  * split hidden dimension) where every group brings a row-tile plan of tiles of at most 32 rows, has a summed rank of at most
- * 128 over an h_in that is a multiple of 128, and the batch has more than 512 rows; else one call per group.  The groups'
- * elements of v must be disjoint.
+ * 128 over an h_in that is a multiple of 128, and the batch has more than 512 rows; else one call per group.  The
+ * elements of v of all projections must be disjoint.
  */
 typedef struct lorax_sgmv_shrink_group {
   const lorax_sgmv_shrink_problem_t* problems; /* host */

@@ -530,12 +530,23 @@ int lorax_sgmv_shrink_multi(const lorax_sgmv_shrink_problem_t* problems, int32_t
     a.group.v[i] = problems[i].v;
     a.group.w[i] = problems[i].w_ptrs;
   }
+  if (!streamed)
+    if (int rc = take_tiles(tiles, a)) return rc;
+  // projections that add into one v do so one after the other
+  for (int i = 0; i < num_problems; ++i)
+    for (int k = 0; k < i; ++k)
+      if (problems[i].v == problems[k].v) {
+        for (int p = 0; p < num_problems; ++p)
+          if (int rc = lorax_sgmv_shrink_multi(&problems[p], 1, x, s_start, s_end, num_segments, num_tokens, h_in, r, layer_idx,
+                                               scale, accumulate, tmp, tmp_bytes, tiles, dtype, stream))
+            return rc;
+        return LORAX_OK;
+      }
   if (streamed) {
     const hipError_t e = launch_sgmv_shrink_rows(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_shrink launch failed: %s", hipGetErrorString(e));
     return LORAX_OK;
   }
-  if (int rc = take_tiles(tiles, a)) return rc;
   if (a.tiles != nullptr && a.num_tiles == 0) return LORAX_OK;  // a plan without tiles: no segment has rows
   const hipError_t e = launch_sgmv_shrink_lds(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(LORAX_ELAUNCH, "sgmv_shrink launch failed: %s", hipGetErrorString(e));

@@ -44,3 +44,22 @@ def test_one_launch_for_several_projections(rank, count, lens, h_in, dtype, accu
     # two roundings of the storage type (update, sum), each at most half an ulp, and fp32 sums
     eps = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
     assert torch.linalg.norm(together.double() - want) <= 2 * eps * torch.linalg.norm(want)
+
+
+@pytest.mark.parametrize("rows,h_in", [(100, 256), (900, 256)])
+def test_projections_that_share_their_output_add_up(rows, h_in):
+    """Two projections may add into one v: they then go out one after the other, in short and in long batches."""
+    gen = torch.Generator().manual_seed(rows)
+    dtype, rank = torch.bfloat16, 16
+    x = torch.randn((rows, h_in), generator=gen).to(dtype).cuda()
+    s, e = (torch.tensor([t], dtype=torch.int32, device="cuda") for t in (0, rows))
+    stacks = [torch.randn((1, rank, h_in), generator=gen).mul_(0.02).to(dtype).cuda() for _ in range(3)]
+    tables = [torch.tensor([w.data_ptr()], dtype=torch.int64, device="cuda") for w in stacks]
+    v0 = torch.randn((2, rows, rank), generator=gen).to(dtype).cuda()
+    together, apart = v0.clone(), v0.clone()
+    tmp = get_shrink_scratch(x.device)
+    _native.sgmv_shrink_multi([together[0], together[1], together[0]], x, tables, s, e, tmp, 0)
+    for i, table in zip((0, 1, 0), tables):
+        _native.sgmv_shrink_multi([apart[i]], x, [table], s, e, tmp, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(together, apart)
