@@ -216,9 +216,10 @@ int lorax_sgmv_shrink_static(void* v, const void* x, const int64_t* w_ptrs, cons
  * number inside its segment.  Every row of every non-empty segment must be in exactly one tile, and no tile may
  * be higher than tile_rows.  lorax_sgmv_plan_tiles builds such a list from host copies of the tables (and
  * lorax_build_batch_tables emits one per rank group).  A launch that is captured keeps its num_tiles and tile_rows, so
- * records written for a later replay must stay within both; the expands take tiles of up to 304 rows, the highest
- * that lorax_sgmv_plan_tiles cuts, whatever tile_rows was, and a record of zeros is padding.  Records are clamped on the device to the call's
- * num_segments, num_tokens and tile_rows (expands: 304 if that is more), and a tile whose segment has a null table entry is skipped, so a wrong
+ * records written for a later replay must stay within both (a record of zeros is padding); the expands take tiles of up
+ * to 304 rows, the highest that lorax_sgmv_plan_tiles cuts, whatever tile_rows was, for rows of y of up to 14 million
+ * elements.  Records are clamped on the device to the call's num_segments, num_tokens and tile_rows (expands: 304 if that
+ * is more), and a tile whose segment has a null table entry is skipped, so a wrong
  * plan gives wrong results but reads and writes x, v and y inside the call's bounds only (a tile may not name a
  * segment whose table entry dangles: the entry is dereferenced, as it would be for a non-empty segment).  The results do not depend on how a batch is cut into tiles, except that the shrink's last
  * rounding can (its sums over the hidden dimension are added in an order that depends on the tile, see
