@@ -153,3 +153,34 @@ def test_one_launch_for_unequal_projections(rank, h_in, widths, records, dtype):
     assert torch.equal(together, apart)
     assert not torch.equal(together, y0)
     assert torch.equal(together[:, :8], y0[:, :8]) and torch.equal(together[:, off:], y0[:, off:])
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_prefill_layers_on_two_streams(native):
+    """Layers of two prefill batches whose shrinks cut the hidden dimension, issued on two streams at once: every call has a
+    scratch of its own, so the outputs are the bits of one after the other."""
+    gen = torch.Generator().manual_seed(3)
+    h_in, width, lens = 4096, 512, [300, 410, 90]
+    jobs = []
+    for _ in range(2):
+        weights = {"q_proj": _layer([64, 32, 16], h_in, width, torch.bfloat16, gen)}
+        meta = make_meta([a for a, n in zip((1, 2, 3), lens) for _ in range(n)], torch.device("cuda", 0))
+        data = AdapterBatchData.from_meta(meta, weights, prefill=True)
+        if not native:
+            assert data.data["q_proj"][LORA].rank_data
+        x = torch.randn((sum(lens), h_in), generator=gen).to(torch.bfloat16).cuda()
+        jobs.append((data, x, torch.randn((sum(lens), width), generator=gen).to(torch.bfloat16).cuda(), weights))
+
+    def run(streams):
+        ys = [y0.clone() for _, _, y0, _ in jobs]
+        torch.cuda.synchronize()
+        for _ in range(10):
+            for (data, x, _, _), y, stream in zip(jobs, ys, streams):
+                with torch.cuda.stream(stream):
+                    TensorParallelMultiAdapterLinear.load(lambda _, y=y: y, 0, ["q_proj"], [width])(x, data)
+        torch.cuda.synchronize()
+        return ys
+
+    here = torch.cuda.current_stream()
+    for a, b in zip(run([here, here]), run([torch.cuda.Stream(), torch.cuda.Stream()])):
+        assert torch.equal(a, b)
