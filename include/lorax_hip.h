@@ -239,7 +239,7 @@ typedef struct lorax_sgmv_tiles {
 } lorax_sgmv_tiles_t;
 
 #define LORAX_TILES_SHRINK 0 /* for lorax_sgmv_shrink_multi: tiles of at most 64 rows                    */
-#define LORAX_TILES_EXPAND 1 /* for lorax_sgmv_expand_planned: tiles of about 256 rows                   */
+#define LORAX_TILES_EXPAND 1 /* for lorax_sgmv_expand_planned: tiles of about 1/16 of the rows, 64 to 256  */
 
 /*
  * Builds a tile plan on the HOST: s_start / s_end are host copies of the segment tables of the launch (empty and

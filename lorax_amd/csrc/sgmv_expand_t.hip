@@ -190,10 +190,14 @@ __global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const Expan
   constexpr int kCols = 16 * NJ;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform, in a scalar register
-  // Workgroup numbering: problem by problem; inside one, row tiles fastest, then panel groups, and consecutive
-  // numbers on one XCD.  The row tiles of a long segment read the same panels of B^T; as neighbours on one XCD
-  // they find them in its L2 instead of fetching them once per tile.
-  int vid = static_cast<int>(xcd_virtual_id());
+  // Workgroup numbering: problem by problem, inside one piece by piece, panel groups fastest, and the numbers go round
+  // robin over the XCDs as the hardware deals them: every XCD gets the same share of every problem and of every segment,
+  // and the long segments, which the table builder lists first, start first.  (Numbered so that each XCD owned a run of
+  // one problem's panel groups, a batch whose segments differ waited for the XCD with the most rows: 28672 columns x
+  // 2062 rows of ranks 8 to 64 111 us, dealt out 68; 786 rows of rank 64 42 and 32 us.)  A panel group has one XCD,
+  // where all pieces of a segment find its panel of B^T in the L2, wherever the number of groups is a multiple of the
+  // XCDs; an XCD then takes adjacent groups (15136 rows: 624 -> 615 us for a step of the large prefill).
+  int vid = static_cast<int>(blockIdx.x);
   int prob = 0;
   if (count > 1) {  // lane i looks at problem i's range: one trip to the kernel arguments
     const int end = batch.wg_end[lane < kMaxExpandProblems ? lane : kMaxExpandProblems - 1];
@@ -202,9 +206,12 @@ __global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const Expan
   }
   const ExpandSlot& P = batch.p[prob];
   const bool acc_y = accumulate_into_y != 0;
-  const int pieces = P.tile_slots * P.subs;
-  const int panel = (vid / pieces) * kExpTWaves + wave;
-  const int piece = vid % pieces;
+  const int groups = (P.h_out + kCols * kExpTWaves - 1) / (kCols * kExpTWaves);
+  const int piece = vid / groups;
+  int group = vid - piece * groups;
+  constexpr int kXcdCount = static_cast<int>(kXcds);
+  if (groups % kXcdCount == 0) group = group % kXcdCount * (groups / kXcdCount) + group / kXcdCount;
+  const int panel = group * kExpTWaves + wave;
   const int sub = piece % P.subs;
   const TileList plan{P.tiles, P.num_tiles, P.tile_rows};
   const int64_t pre_w = preload_segment_entry(P.w_ptrs, P.num_segments);

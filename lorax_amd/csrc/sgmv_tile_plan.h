@@ -18,7 +18,7 @@
 namespace lorax {
 
 constexpr int kShrinkTileRowsMax = 64;   // the LDS-staged shrink's buffers hold up to four 16-row blocks
-constexpr int kExpandTileRows = 256;     // nominal height of an expand tile
+constexpr int kExpandTileRows = 256;     // nominal height of an expand tile, at most
 constexpr int kExpandTileRowsMax = kExpandTileRows + kExpandTileRows / 8 + 16;  // with a merged remainder
 
 struct SegmentSpan {
@@ -84,17 +84,29 @@ inline int plan_shrink_tiles(const std::vector<SegmentSpan>& segs, std::vector<l
   return rows;
 }
 
-// Expand tiles: nominally 256 rows; a remainder of at most an eighth of the segment's full tiles is shared out
+// Nominal height of the expand's tiles: a sixteenth of the rows, between 64 and 256.  A workgroup walks its tile's rows
+// one block after the other, so a launch of a few segments of different lengths is as long as its tallest tile: ten
+// segments of 33 to 256 rows (rank 64, four Mistral-7B layers) take 571 / 543 / 528 us of GPU time in tiles of up to
+// 256 / 128 / 64 rows, segments of 24 to 900 rows of four ranks 514 / 480 / 482 us.  Lower tiles fetch their panels of
+// B^T more often: a 4096-row run at rank 128 1873 / 1885 / 1922 us, 15136 rows at rank 64 624 / 623 / 643 us.
+inline int expand_tile_rows(int64_t rows_total) {
+  return static_cast<int>(std::min<int64_t>(std::max<int64_t>((rows_total + 255) / 256 * 16, 64), kExpandTileRows));
+}
+
+// Expand tiles: nominally expand_tile_rows high; a remainder of at most an eighth of the segment's full tiles is shared out
 // among them instead of becoming a tile of its own (a tile's prologue costs as much as a hundred rows), and the
 // segment's tiles get equal heights in 16-row blocks - the rule of the device-side search (merged_tile_count).
 // Returns the height of the tallest tile (the launcher cuts tiles into pieces by it); none is above kExpandTileRowsMax.
 inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<lorax_sgmv_tile_t>& out) {
+  int64_t rows_total = 0;
+  for (const SegmentSpan& s : segs) rows_total += s.end - s.start;
+  const int rows = expand_tile_rows(rows_total);
   int tallest = 1;
   for (const SegmentSpan& s : segs) {
     const int len = s.end - s.start;
-    const int full = len / kExpandTileRows;
-    const int rem = len - full * kExpandTileRows;
-    const int nt = (full >= 1 && rem * 8 <= full * kExpandTileRows) ? full : full + (rem > 0 ? 1 : 0);
+    const int full = len / rows;
+    const int rem = len - full * rows;
+    const int nt = (full >= 1 && rem * 8 <= full * rows) ? full : full + (rem > 0 ? 1 : 0);
     const int blocks = (len + 15) / 16;
     for (int i = 0; i < nt; ++i) {
       lorax_sgmv_tile_t t;

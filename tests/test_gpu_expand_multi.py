@@ -97,3 +97,32 @@ def test_expand_multi_checks_its_problems():
         _native.sgmv_expand_multi([(y, v, w, s, s, 8, 64, None)], 0)
     with pytest.raises(RuntimeError, match="between 1 and 16 problems"):
         _native.sgmv_expand_multi([(y, v, w, s, s, 0, 64, None)] * 17, 0)
+
+
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("h_out", [2048, 2304, 264, 4096])  # 8, 9, 2 and 16 panel groups: dealt out with and without runs
+@pytest.mark.parametrize("lens", [[1], [64, 65, 0, 300, 7], [1100, 3], [4400]])  # tile heights of 64, 80 and 256 rows
+def test_every_element_of_the_expand_is_written_once(h_out, lens, planned):
+    """y += 1 everywhere inside the segments and nowhere else: v and B are such that every update is exactly one."""
+    print(f"case h_out={h_out} lens={lens} planned={planned}", flush=True)
+    r, off = 16, 8
+    starts = [sum(lens[:i]) + i + 1 for i in range(len(lens))]
+    ends = [s + n for s, n in zip(starts, lens)]
+    T = ends[-1] + 2
+    v = torch.zeros((T, r), dtype=torch.bfloat16, device=DEV)
+    v[:, 3] = 1.0
+    bt = torch.zeros((1, h_out, r), dtype=torch.bfloat16, device=DEV)
+    bt[:, :, 3] = 1.0
+    tiles = None
+    if planned:
+        records, rows = _native.plan_tiles(starts, ends, T, _native.TILES_EXPAND)
+        tiles = _native.TilePlan(torch.from_numpy(records.copy()).to(DEV), rows)
+    y = torch.zeros((T, h_out + 2 * off), dtype=torch.bfloat16, device=DEV)
+    s, e = (torch.tensor(b, dtype=torch.int32, device=DEV) for b in (starts, ends))
+    _native.sgmv_expand(y, v, ptr_table([bt] * len(lens), DEV), s, e, sgmv.get_tmp_tensor_for_size(len(lens), torch.device(DEV)),
+                        0, off, h_out, True, True, tiles)
+    want = torch.zeros((T, h_out + 2 * off))
+    for a, b in zip(starts, ends):
+        want[a:b, off:off + h_out] = 1.0
+    torch.cuda.synchronize()
+    assert torch.equal(y.float().cpu(), want)
