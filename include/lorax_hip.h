@@ -513,6 +513,28 @@ int lorax_layer_update(const lorax_table_group_t* groups, int32_t num_groups, co
                        int64_t tmp_bytes, int32_t dtype, int32_t device, void* stream);
 
 /*
+ * The decode update of up to 16 projections that share their input over stacked weights (one [num_adapters, r, h_in] and
+ * one [num_adapters, width, r] tensor per projection): picks the launches as lorax_layer_update does and issues them.
+ *   slices     host: the stacks, rank, width and first column in y of each projection
+ *   plan       device: `records` routing records that name entries of the stacks (lorax_bgmv_multi)
+ *   v, v_bytes device workspace, num_tokens * (sum of the ranks) elements
+ *   device     the GPU the pointers live on; made current for the call
+ * Every row named by a record has to be below num_tokens.  Returns LORAX_EROUTE, with nothing launched, for ranks that are
+ * no multiple of 8 or above 128.
+ */
+typedef struct lorax_stacked_slice {
+  const void* a_stack;
+  const void* b_stack;
+  int64_t y_offset;
+  int32_t rank;
+  int32_t width;
+} lorax_stacked_slice_t;
+
+int lorax_stacked_update(const lorax_stacked_slice_t* slices, int32_t num_slices, const int64_t* plan, int32_t records,
+                         void* y, int64_t y_stride, const void* x, int64_t num_tokens, int32_t h_in, void* v, int64_t v_bytes,
+                         int32_t dtype, int32_t device, void* stream);
+
+/*
  * Per-device set-up: looks up the address of the static scratch of lorax_sgmv_shrink_static on `device`.
  * Nothing is allocated (every other entry point takes its scratch from the caller, as the reference does,
  * punica.py:145-167).  Optional: lorax_sgmv_shrink_static does the same on its first call on a device.

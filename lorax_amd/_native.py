@@ -219,6 +219,11 @@ _SIGNATURES = {
         [_c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64,
          _c.c_int32, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_void_p],
     ),
+    "lorax_stacked_update": (
+        _c.c_int,
+        [_c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_int32,
+         _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_void_p],
+    ),
     "lorax_init": (_c.c_int, [_c.c_int32]),
     "lorax_workspace_bytes": (_c.c_size_t, []),
     "lorax_last_error": (_c.c_char_p, []),
@@ -829,15 +834,18 @@ class BatchTables:
         self.rows = rows
         self.prefill = prefill
         self.device_index = packed.get_device()
-        self.rank_sum = {}  # layer type -> sum of the ranks of its groups
-        for g in groups[:num_groups]:
-            self.rank_sum[g.layer_type] = self.rank_sum.get(g.layer_type, 0) + g.rank
+        self.rank_sum = None  # layer type -> sum of the ranks of its groups, from the first call on
         self._calls = {}  # slices of a call -> (LayerSlice array, columns of v)
 
     def call(self, slices):
         """(LayerSlice array, sum of ranks) of `slices`, a tuple of (layer type, first column, end column)."""
         made = self._calls.get(slices)
         if made is None:
+            if self.rank_sum is None:
+                sums = {}
+                for g in self.groups[: self.num_groups]:
+                    sums[g.layer_type] = sums.get(g.layer_type, 0) + g.rank
+                self.rank_sum = sums
             arr = (LayerSlice * len(slices))(*[LayerSlice(t, end - start, start) for t, start, end in slices])
             made = self._calls[slices] = (arr, sum(self.rank_sum[t] for t, _, _ in slices))
         return made
@@ -876,9 +884,52 @@ def layer_update(y, x, tables: BatchTables, slices, layer_idx: int) -> bool:
     return True
 
 
+_STACKED_SLICE = "2Qq2i"  # lorax_stacked_slice_t
+_STACKED_SLICES = [struct.Struct(_STACKED_SLICE * n) for n in range(MAX_BGMV_PROBLEMS + 1)]
+
+
+def stacked_update(y, x, slices, plan: torch.Tensor, records: int) -> bool:
+    """lorax_stacked_update: y[:, first:first + width] += the update of x over stacked weights for every slice (lora_a
+    [n, r, h_in], lora_b [n, width, r], first, width), all launches from one call; `plan` holds `records` routing records over
+    stack entries.  False, with nothing launched, where the single operators have to be used: operands they would refuse
+    or that need another path."""
+    dtype = x.dtype
+    code = _DTYPE_CODES.get(dtype)
+    if (code is None or y.dtype != dtype or x.dim() != 2 or y.dim() != 2 or not x.is_cuda or not y.is_cuda
+            or not x.is_contiguous() or not y.is_contiguous() or len(slices) > MAX_BGMV_PROBLEMS):
+        return False
+    rows, h_in = x.shape
+    y_rows, y_stride = y.shape
+    index = x.get_device()
+    if (y.get_device() != index or plan.get_device() != index or y_rows != rows or rows == 0 or plan.dtype != torch.int64
+            or not plan.is_contiguous()):
+        return False
+    fields, columns = [], 0
+    for a, b, first, width in slices:
+        if a.dim() != 3 or b.dim() != 3:
+            return False
+        r = a.size(1)
+        if (a.size(2) != h_in or b.size(2) != r or b.size(1) != width or a.dtype != dtype or b.dtype != dtype
+                or a.get_device() != index or b.get_device() != index or not a.is_contiguous() or not b.is_contiguous()):
+            return False
+        fields += (a.data_ptr(), b.data_ptr(), first, r, width)
+        columns += r
+    v_bytes = rows * columns * 2
+    v = torch.empty((v_bytes,), dtype=torch.uint8, device=x.device)  # the call's own, on its stream
+    rc = lib().lorax_stacked_update(_STACKED_SLICES[len(slices)].pack(*fields), len(slices), plan.data_ptr(), records,
+                                    y.data_ptr(), y_stride, x.data_ptr(), rows, h_in, v.data_ptr(), v_bytes, code, index,
+                                    _stream(x))
+    if rc == EROUTE:
+        return False
+    if rc != 0:
+        _raise_last(rc)
+    return True
+
+
 ENTRY_DTYPE = [("adapter", "<i8"), ("a_addr", "<i8"), ("b_addr", "<i8"), ("rank", "<i4"), ("reserved", "<i4")]
 
 
+_entry_dtype = None
 _table_capacity = [64 * 1024, 64]  # bytes of packed tables, number of group records
 
 
@@ -894,8 +945,11 @@ def batch_tables(adapter_indices, entries, entry_counts, prefill: bool):
     """build_batch_tables with the group records as the ctypes array the builder filled and their number."""
     import numpy as np
 
+    global _entry_dtype
+    if _entry_dtype is None:
+        _entry_dtype = np.dtype(ENTRY_DTYPE)  # made once: numpy takes longer to make it than the builder takes for a few rows
     adapter_indices = np.ascontiguousarray(adapter_indices, dtype=np.int64)
-    entries = np.ascontiguousarray(entries, dtype=ENTRY_DTYPE)
+    entries = np.ascontiguousarray(entries, dtype=_entry_dtype)
     entry_counts = np.ascontiguousarray(entry_counts, dtype=np.int32)
     T = adapter_indices.shape[0]
     bounds = np.zeros(T + 1, dtype=np.int32)

@@ -753,8 +753,8 @@ def _native_batch_tables(meta: AdapterBatchMetadata, weights: Dict[str, LayerAda
     device = meta.adapter_indices.device
     indices = meta.adapter_indices.detach().cpu().numpy()
     bounds, owners, packed, groups, num_groups = _native.batch_tables(
-        indices, np.concatenate(tables), np.array([len(t) for t in tables], dtype=np.int32), prefill
-    )
+        indices, np.concatenate([t.view(np.uint8) for t in tables]).view(tables[0].dtype),  # (by bytes: numpy promotes
+        np.array([len(t) for t in tables], dtype=np.int32), prefill)                        # field by field otherwise)
     dev = torch.from_numpy(packed).to(device)
     build = _TableViews(dev, packed, bounds, owners, int(indices.shape[0]), device)
     # a layer's launches can go out in one native call as long as nobody holds (and may have changed) the tables

@@ -22,6 +22,8 @@ struct Job {
   int64_t y_offset;
   int32_t width;
   char* v;  // [num_tokens, rank] piece of the workspace
+  const void* a_stack;  // stacked weights: the plan's records name entries of these tensors; else null
+  const void* b_stack;
 };
 
 // What every launch of the call shares.
@@ -44,9 +46,9 @@ bool fused_rank(int r, int64_t h_in) { return (r == 8 || r == 16) && r * h_in * 
 const void* at(const Call& c, int64_t off) { return c.tables + off; }
 
 lorax_bgmv_problem_t plan_problem(const Call& c, const Job& j, void* y, const void* x, int64_t y_offset, int64_t y_stride,
-                                  int32_t h_out, int32_t h_in) {
+                                  int32_t h_out, int32_t h_in, const void* a_stack, const void* b_stack) {
   return {y, x, nullptr, nullptr, y_offset, y_stride, h_out, static_cast<const int64_t*>(at(c, j.g->plan_off)),
-          j.g->num_chunks, h_in, nullptr, nullptr};
+          j.g->num_chunks, h_in, a_stack, b_stack};
 }
 
 // One planned launch for up to 16 jobs: x -> v (shrink) or v -> y (expand).
@@ -55,8 +57,8 @@ int bgmv_jobs(const Call& c, const Job* const* jobs, int count, bool shrink) {
   for (int i = 0; i < count; ++i) {
     const Job& j = *jobs[i];
     const int r = j.g->rank;
-    p[i] = shrink ? plan_problem(c, j, j.v, c.x, 0, r, r, c.h_in)
-                  : plan_problem(c, j, c.y, j.v, j.y_offset, c.y_stride, j.width, r);
+    p[i] = shrink ? plan_problem(c, j, j.v, c.x, 0, r, r, c.h_in, j.a_stack, nullptr)
+                  : plan_problem(c, j, c.y, j.v, j.y_offset, c.y_stride, j.width, r, nullptr, j.b_stack);
   }
   return lorax_bgmv_multi(p, count, c.rows, shrink ? c.h_in : p[0].h_in, c.layer_idx, 1.0f, shrink ? 0 : 1, c.dtype, c.stream);
 }
@@ -74,7 +76,8 @@ int decode(const Call& c, Job* const* jobs, int count) {
           n = 0;
         }
         if (i < count && jobs[i]->g->rank == r)
-          p[n++] = plan_problem(c, *jobs[i], c.y, c.x, jobs[i]->y_offset, c.y_stride, jobs[i]->width, 0);
+          p[n++] = plan_problem(c, *jobs[i], c.y, c.x, jobs[i]->y_offset, c.y_stride, jobs[i]->width, 0, jobs[i]->a_stack,
+                                jobs[i]->b_stack);
       }
     }
     return LORAX_OK;
@@ -194,7 +197,7 @@ int update(const Call& c, const lorax_table_group_t* groups, int32_t num_groups,
       if (g.use_sgmv != 0 && g.rank % 16 != 0 && c.h_in % 128 != 0 && c.rows > kShortBatchRows) return LORAX_EROUTE;
       if (g.use_sgmv != 0 && (g.segments_id < 0 || g.shrink_tiles_off < 0 || g.expand_tiles_off < 0)) return LORAX_EROUTE;
       if (g.use_sgmv == 0 && g.plan_off < 0) return LORAX_EROUTE;
-      jobs[count++] = {&g, slices[s].y_offset, slices[s].width, nullptr};
+      jobs[count++] = {&g, slices[s].y_offset, slices[s].width, nullptr, nullptr, nullptr};
     }
   if (count == 0) return LORAX_OK;
   const bool by_segments = jobs[0].g->use_sgmv != 0;
@@ -220,6 +223,18 @@ int update(const Call& c, const lorax_table_group_t* groups, int32_t num_groups,
   }
   if (used > v_bytes) return lorax::report_error(LORAX_ESPACE, "layer update: the workspace is smaller than num_tokens * ranks");
   return by_segments ? prefill(c, order, count) : decode(c, order, count);
+}
+
+// Runs `launch` with `device` current.
+template <typename Launch>
+int on_device(int device, const Launch& launch) {
+  int current = 0;
+  if (hipError_t e = hipGetDevice(&current)) return lorax::report_error(LORAX_ELAUNCH, hipGetErrorString(e));
+  if (current != device)
+    if (hipError_t e = hipSetDevice(device)) return lorax::report_error(LORAX_ELAUNCH, hipGetErrorString(e));
+  const int rc = launch();
+  if (current != device) (void)hipSetDevice(current);
+  return rc;
 }
 
 }  // namespace
@@ -278,11 +293,32 @@ extern "C" int lorax_layer_update(const lorax_table_group_t* groups, int32_t num
         return lorax::report_error(LORAX_EINVAL, "layer update: x and y have fewer rows than the batch of the routing tables");
     }
   const Call c{static_cast<const char*>(tables), y, y_stride, x, num_tokens, h_in, layer_idx, tmp, tmp_bytes, dtype, stream};
-  int current = 0;
-  if (hipError_t e = hipGetDevice(&current)) return lorax::report_error(LORAX_ELAUNCH, hipGetErrorString(e));
-  if (current != device)
-    if (hipError_t e = hipSetDevice(device)) return lorax::report_error(LORAX_ELAUNCH, hipGetErrorString(e));
-  const int rc = update(c, groups, num_groups, slices, num_slices, static_cast<char*>(v), v_bytes);
-  if (current != device) (void)hipSetDevice(current);
-  return rc;
+  return on_device(device, [&] { return update(c, groups, num_groups, slices, num_slices, static_cast<char*>(v), v_bytes); });
+}
+
+extern "C" int lorax_stacked_update(const lorax_stacked_slice_t* slices, int32_t num_slices, const int64_t* plan, int32_t records,
+                                    void* y, int64_t y_stride, const void* x, int64_t num_tokens, int32_t h_in, void* v,
+                                    int64_t v_bytes, int32_t dtype, int32_t device, void* stream) {
+  if (num_slices < 0 || num_slices > lorax::kMaxBgmvProblems || num_tokens < 0 || records < 0)
+    return lorax::report_error(LORAX_EINVAL, "stacked update: number of slices (at most 16), rows or plan records out of range");
+  if (num_slices == 0 || num_tokens == 0 || records == 0) return LORAX_OK;
+  if (slices == nullptr || plan == nullptr || y == nullptr || x == nullptr || v == nullptr)
+    return lorax::report_error(LORAX_EINVAL, "null pointer argument (slices, plan, y, x or v)");
+  lorax_table_group_t groups[lorax::kMaxBgmvProblems];
+  Job jobs[lorax::kMaxBgmvProblems];
+  Job* order[lorax::kMaxBgmvProblems];
+  int64_t used = 0;
+  for (int i = 0; i < num_slices; ++i) {
+    const lorax_stacked_slice_t& s = slices[i];
+    if (s.rank < 8 || s.rank % 8 != 0 || s.rank > kMaxKernelRank || s.a_stack == nullptr || s.b_stack == nullptr) return LORAX_EROUTE;
+    groups[i] = lorax_table_group_t{};
+    groups[i].rank = s.rank;
+    groups[i].num_chunks = records;
+    jobs[i] = {&groups[i], s.y_offset, s.width, static_cast<char*>(v) + used, s.a_stack, s.b_stack};
+    order[i] = &jobs[i];
+    used += num_tokens * s.rank * 2;
+  }
+  if (used > v_bytes) return lorax::report_error(LORAX_ESPACE, "stacked update: the workspace is smaller than num_tokens * ranks");
+  const Call c{reinterpret_cast<const char*>(plan), y, y_stride, x, num_tokens, h_in, 0, nullptr, 0, dtype, stream};
+  return on_device(device, [&] { return decode(c, order, num_slices); });
 }

@@ -32,6 +32,7 @@ from torch import nn
 from lorax_amd import _native
 from lorax_amd.adapters import LORA, AdapterBatchData, BatchLoraWeights
 from lorax_amd._native import MAX_SGMV_SHRINK_PROBLEMS
+from lorax_amd.punica_wrapper import PunicaWrapper
 from lorax_amd.sgmv import (
     MAX_RANK_CUSTOM,
     get_shrink_scratch,
@@ -87,10 +88,10 @@ class LoraLinear(nn.Module):
     def _native_update(self, result, input, adapter_data: AdapterBatchData, slices) -> bool:
         """All launches of the call from one native call (lorax_layer_update), where every projection's tables are
         the untouched packed ones of the batch; False, with nothing launched, where the general path has to run."""
-        if adapter_data.layer_to_lora_weights and adapter_data.punica_wrapper is not None:
-            return False
         if not has_sgmv() or self.process_group.size() > 1:
             return False
+        if adapter_data.layer_to_lora_weights and adapter_data.punica_wrapper is not None:
+            return self._stacked_update(result, input, adapter_data, slices)
         tables, targets = None, []
         for name, start, end in slices:
             layer_data = adapter_data.data.get(name)
@@ -105,6 +106,23 @@ class LoraLinear(nn.Module):
         if tables is None:
             return False
         return _native.layer_update(result, input, tables, tuple(targets), self.layer_id)
+
+    def _stacked_update(self, result, input, adapter_data: AdapterBatchData, slices) -> bool:
+        """The same where every projection of a decode call is served by stacked weights."""
+        wrapper = adapter_data.punica_wrapper
+        if type(wrapper) is not PunicaWrapper or not wrapper.enabled or input.shape[0] > wrapper.max_batch_size:
+            return False
+        jobs = []
+        for name, start, end in slices:
+            layer_data = adapter_data.data.get(name)
+            data = layer_data.get(LORA) if layer_data is not None else None
+            if data is None:
+                continue  # no adapter in the batch targets this projection
+            stacks = adapter_data.layer_to_lora_weights.get((name, self.layer_id))
+            if stacks is None or not data.can_vectorize(self.process_group):
+                return False
+            jobs.append((stacks[0], stacks[1], start, end - start))
+        return bool(jobs) and wrapper.add_lora_update(result, input, jobs)
 
     def forward_layer_types(
         self,
@@ -377,7 +395,7 @@ class TensorParallelMultiAdapterLinear(LoraLinear):
                 end = result.shape[1]
             slices.append((name, start, end))
         result = self.forward_layer_types(result, input, adapter_data, slices)
-        return result.reshape(out_shape)
+        return result if result.shape == out_shape else result.reshape(out_shape)
 
 
 class TensorParallelAdapterRowLinear(LoraLinear):

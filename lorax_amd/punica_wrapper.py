@@ -20,7 +20,7 @@ from typing import Callable, List, Optional, Sequence, Tuple
 
 import torch
 
-from lorax_amd import ops
+from lorax_amd import _native, ops
 
 Slice = Tuple[torch.Tensor, torch.Tensor, int, int]  # (lora_a stack, lora_b stack, first column, width)
 
@@ -259,6 +259,13 @@ class PunicaWrapper:
                 mid = callback(mid)  # e.g. all-gather / all-reduce of the intermediate across ranks
             whole = first == 0 and width == rows_y.shape[1]
             self._run("expand", rows_y, mid, lora_b, add_input=True, window=None if whole else (first, width))
+
+    def add_lora_update(self, y: torch.Tensor, x: torch.Tensor, slices: Sequence[Slice]) -> bool:
+        """add_lora_slices at scale 1 in decode from one native call (the same launches, so the same bits).  False, with
+        nothing launched, for batches and operands that need add_lora_slices, which also says what is wrong with them."""
+        if self.is_prefill or self._plan_records is None or self.indices_len[0] > x.shape[0]:
+            return False
+        return _native.stacked_update(y, x, slices, self._plan, self._plan_records)
 
     def add_lora(self, y: torch.Tensor, x: torch.Tensor, wa_t_all: torch.Tensor, wb_t_all: torch.Tensor, scale: float,
                  y_offset: Optional[int] = None, y_slice_size: Optional[int] = None, *,

@@ -232,6 +232,20 @@ def test_sgmv_expand_planned_validation():
     assert f(P, P, P, P, P, 2, 16, 16, 4096, 0, 4096, 0, 1, ctypes.byref(empty), 1, None) == OK
 
 
+def test_stacked_update_validation():
+    f = _native.lib().lorax_stacked_update
+    pack = lambda *slices: b"".join(_native._STACKED_SLICES[1].pack(*s) for s in slices)
+    one = pack((P, P, 0, 16, 256))
+    call = lambda s, n, rows=4, records=2, v_bytes=1 << 20, plan=P: f(s, n, plan, records, P, 256, P, rows, 512, P, v_bytes, 1, 0, None)
+    assert call(one, 0) == call(one, 1, rows=0) == call(one, 1, records=0) == OK  # nothing to do
+    assert call(one, 17) == call(one, -1) == call(one, 1, rows=-1) == call(one, 1, records=-1) == EINVAL and "out of range" in _err()
+    assert call(one, 1, plan=None) == EINVAL and "null" in _err()
+    for rank in (4, 12, 136):
+        assert call(pack((P, P, 0, rank, 256)), 1) == _native.EROUTE
+    assert call(pack((0, P, 0, 16, 256)), 1) == _native.EROUTE
+    assert call(pack((P, P, 0, 16, 256), (P, P, 256, 8, 256)), 2, v_bytes=4 * 24 * 2 - 1) == 5 and "workspace" in _err()
+
+
 def test_plan_tiles_cuts_every_row_once():
     """lorax_sgmv_plan_tiles (host only): every row of every non-empty segment in exactly one tile, tiles inside
     their segment and no higher than the bound, numbered inside the segment; empty and negative segments get none."""

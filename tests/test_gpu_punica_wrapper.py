@@ -277,3 +277,44 @@ def test_slot_plan_buffer_is_padded_with_skipped_records():
     ops.bgmv_lora_slices(x, [(a, b, 0, w)], y_ref, small.to(DEV), 1.0)
     torch.cuda.synchronize()
     assert torch.equal(y_fixed, y_ref) and torch.count_nonzero(y_ref) > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ranks,widths,tokens", [
+    ((8, 8, 8), (4096, 1024, 1024), 40),     # one launch
+    ((16, 8), (1024, 512), 5),               # one launch per rank
+    ((32, 64, 8), (1024, 1024, 264), 1),     # two launches, a single token
+    ((16,) * 2 + (128,) * 15, (264,) * 17, 9),  # more projections than one call takes: slice by slice of 16
+])
+def test_stacked_update_from_one_call_equals_the_operators(ranks, widths, tokens, dtype):
+    """PunicaWrapper.add_lora_update (lorax_stacked_update) against add_lora_slices: the same launches, so the same bits; what
+    it does not take it leaves untouched."""
+    print(f"case ranks={ranks} tokens={tokens} dtype={dtype}", flush=True)
+    gen = torch.Generator().manual_seed(tokens)
+    h_in, n = 1024, 3
+    slots = [(i * 7) % (n + 1) - 1 for i in range(tokens)] if tokens > 1 else [1]
+    x = randn((tokens, h_in), 1.0, gen, dtype, DEV)
+    y0 = randn((tokens, sum(widths) + 8), 0.5, gen, dtype, DEV)
+    slices, off = [], 8
+    for r, width in zip(ranks, widths):
+        a, b = _stacks(n, r, h_in, width, gen, dtype)
+        slices.append((a.view(n, r, h_in), b.view(n, width, r), off, width))
+        off += width
+    wrapper = PunicaWrapper(64, 64, DEV, True)
+    wrapper.update_metadata(make_meta([s + 1 for s in slots], torch.device(DEV)), False)
+    want, got = y0.clone(), y0.clone()
+    wrapper.add_lora_slices(want, x, slices, 1.0)
+    assert wrapper.add_lora_update(got, x, slices) == (len(slices) <= 16)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want if len(slices) <= 16 else y0) and not torch.equal(want, y0)
+
+    a, b, first, width = slices[0]
+    left = y0.clone()
+    for bad in [(a.float(), b), (a, b.transpose(1, 2)), (a[:, :, :-8], b), (a, b[:, :-8]), (a[:, None], b), (a.cpu(), b)]:
+        assert not wrapper.add_lora_update(left, x, [(*bad, first, width)])
+    assert not wrapper.add_lora_update(left[:-1], x[:-1], slices[:1])  # fewer rows than the routing plan's batch
+    assert not wrapper.add_lora_update(left, x.float(), slices[:1]) and not wrapper.add_lora_update(left.t(), x, slices[:1])
+    wrapper.update_metadata(make_meta([s + 1 for s in slots], torch.device(DEV)), True)
+    assert not wrapper.add_lora_update(left, x, slices[:1])  # prefill
+    torch.cuda.synchronize()
+    assert torch.equal(left, y0)
