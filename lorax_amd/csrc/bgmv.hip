@@ -117,7 +117,8 @@ __device__ __forceinline__ void bgmv_shrink_body(typename D::E* __restrict__ Y,
 struct BatchSlot {
   int problem, chunk, sub;
 };
-__device__ __forceinline__ BatchSlot batch_slot(const BgmvBatch& batch, int count) {
+template <int P>
+__device__ __forceinline__ BatchSlot batch_slot(const BgmvBatchOf<P>& batch, int count) {
   const int v = static_cast<int>(xcd_virtual_id());
   if (count == 1) {  // the drop-in single-problem call: no table walk in front of the first useful load
     const int subs = batch.run_subs[0];
@@ -126,10 +127,10 @@ __device__ __forceinline__ BatchSlot batch_slot(const BgmvBatch& batch, int coun
   // Lane i looks at problem i: the five table entries of all problems arrive in one trip to the kernel arguments
   // (a walk with the scalar unit asks for them one after the other, each answer deciding the next question - a
   // handful of dependent cache misses in front of the first useful load of every CU's first workgroup).
-  const int i = lane_id() < kMaxBgmvProblems ? lane_id() : kMaxBgmvProblems - 1;
+  const int i = lane_id() < P ? lane_id() : P - 1;
   const int run_end = batch.run_end[i], base = batch.base[i], subs = batch.run_subs[i];
   const int sub_lo = batch.sub_lo[i], sub_hi = batch.sub_hi[i];
-  const bool mine = lane_id() < kMaxBgmvProblems && i + 1 < count;
+  const bool mine = lane_id() < P && i + 1 < count;
   // first problem of the run that holds v: run_end does not decrease with the problem number
   const int first = __popcll(__ballot(mine && v >= run_end));
   const int rem = v - read_lane(base, first);
@@ -137,8 +138,8 @@ __device__ __forceinline__ BatchSlot batch_slot(const BgmvBatch& batch, int coun
   const int chunk = rem / run_subs, s = rem % run_subs;
   // inside the run, sub_hi increases and the run's last problem has sub_hi = run_subs > s
   const int run_stop = read_lane(run_end, first);
-  const int p = first + __popcll(__ballot(mine && i >= first && run_end == run_stop && s >= sub_hi));
-  return BatchSlot{p, chunk, s - read_lane(sub_lo, p)};
+  const int problem = first + __popcll(__ballot(mine && i >= first && run_end == run_stop && s >= sub_hi));
+  return BatchSlot{problem, chunk, s - read_lane(sub_lo, problem)};
 }
 
 // Problem `p` of a batch, fetched the same way: lane i asks for the fields of problem i before anybody knows p,
@@ -152,12 +153,13 @@ __device__ __forceinline__ int64_t read_lane64(int64_t v, int src) {
   const uint32_t hi = static_cast<uint32_t>(read_lane(static_cast<int>(static_cast<uint64_t>(v) >> 32), src));
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
-struct ProblemFields {  // one lane's copy of problem min(lane, 15)
+struct ProblemFields {  // one lane's copy of problem min(lane, P - 1)
   int64_t y, x, w_ptrs, indices, y_offset, y_stride, plan;
   int width, narrow, num_groups;
 };
-__device__ __forceinline__ ProblemFields preload_problems(const BgmvBatch& batch) {
-  const BgmvProblem& q = batch.p[lane_id() < kMaxBgmvProblems ? lane_id() : kMaxBgmvProblems - 1];
+template <int P>
+__device__ __forceinline__ ProblemFields preload_problems(const BgmvBatchOf<P>& batch) {
+  const BgmvProblem& q = batch.p[lane_id() < P ? lane_id() : P - 1];
   return ProblemFields{reinterpret_cast<int64_t>(q.y), reinterpret_cast<int64_t>(q.x),
                        reinterpret_cast<int64_t>(q.w_ptrs), reinterpret_cast<int64_t>(q.indices), q.y_offset,
                        q.y_stride, reinterpret_cast<int64_t>(q.plan), q.width, q.narrow, q.num_groups};
@@ -185,8 +187,9 @@ struct PlanOfLane {
   int64_t plan;
   int num_groups;
 };
-__device__ __forceinline__ PlanOfLane preload_plans(const BgmvBatch& batch) {
-  const BgmvProblem& q = batch.p[lane_id() < kMaxBgmvProblems ? lane_id() : kMaxBgmvProblems - 1];
+template <int P>
+__device__ __forceinline__ PlanOfLane preload_plans(const BgmvBatchOf<P>& batch) {
+  const BgmvProblem& q = batch.p[lane_id() < P ? lane_id() : P - 1];
   return PlanOfLane{reinterpret_cast<int64_t>(q.plan), q.num_groups};
 }
 
@@ -220,39 +223,39 @@ __device__ __forceinline__ int resolve_chunk(const BgmvProblem& P, const int64_t
   return n;
 }
 
-template <typename D, int RS>
+template <typename D, int RS, int P>
 __global__ __launch_bounds__(kBgmvThreads) void bgmv_shrink_kernel(
-    const BgmvBatch batch, int count, int num_tokens, int h_in, int64_t layer_idx, float scale,
+    const BgmvBatchOf<P> batch, int count, int num_tokens, int h_in, int64_t layer_idx, float scale,
     int accumulate_into_y) {
   __shared__ float red[(kBgmvThreads / kWave) * Pow2Ceil<RS * kGroup>::value];
   using E = typename D::E;
   const PlanOfLane plans = preload_plans(batch);
   const BatchSlot slot = batch_slot(batch, count);
-  const BgmvProblem& P = batch.p[slot.problem];
-  const int r = P.narrow;
+  const BgmvProblem& prob = batch.p[slot.problem];
+  const int r = prob.narrow;
   const int row0 = slot.sub * RS;
   int toks[kGroup];
   int64_t stack_addr;
-  const int n = resolve_chunk(P, reinterpret_cast<const int64_t*>(read_lane64(plans.plan, slot.problem)),
+  const int n = resolve_chunk(prob, reinterpret_cast<const int64_t*>(read_lane64(plans.plan, slot.problem)),
                               read_lane(plans.num_groups, slot.problem), num_tokens, false, slot.chunk, toks,
                               stack_addr);
   if (n == 0) return;
   const E* A = reinterpret_cast<const E*>(stack_addr) + (layer_idx * r + row0) * static_cast<int64_t>(h_in);
-  E* Y = static_cast<E*>(P.y);
-  const E* X = static_cast<const E*>(P.x);
+  E* Y = static_cast<E*>(prob.y);
+  const E* X = static_cast<const E*>(prob.x);
   const bool acc_y = accumulate_into_y != 0;
   switch (n) {
     case 1:
-      bgmv_shrink_body<D, RS, 1>(Y, X, A, toks, h_in, row0, P.y_offset, P.y_stride, scale, acc_y, red);
+      bgmv_shrink_body<D, RS, 1>(Y, X, A, toks, h_in, row0, prob.y_offset, prob.y_stride, scale, acc_y, red);
       break;
     case 2:
-      bgmv_shrink_body<D, RS, 2>(Y, X, A, toks, h_in, row0, P.y_offset, P.y_stride, scale, acc_y, red);
+      bgmv_shrink_body<D, RS, 2>(Y, X, A, toks, h_in, row0, prob.y_offset, prob.y_stride, scale, acc_y, red);
       break;
     case 3:
-      bgmv_shrink_body<D, RS, 3>(Y, X, A, toks, h_in, row0, P.y_offset, P.y_stride, scale, acc_y, red);
+      bgmv_shrink_body<D, RS, 3>(Y, X, A, toks, h_in, row0, prob.y_offset, prob.y_stride, scale, acc_y, red);
       break;
     default:
-      bgmv_shrink_body<D, RS, 4>(Y, X, A, toks, h_in, row0, P.y_offset, P.y_stride, scale, acc_y, red);
+      bgmv_shrink_body<D, RS, 4>(Y, X, A, toks, h_in, row0, prob.y_offset, prob.y_stride, scale, acc_y, red);
       break;
   }
 }
@@ -562,8 +565,8 @@ __host__ __device__ __forceinline__ int expand_lanes_per_column(int r) {
 // VY: y moves in 16-byte pieces (bgmv_expand_body_vec); each wave has kGroup * U * 64 floats of LDS for its sums
 // (one lane per column, the widest case; with 4 and more lanes per column the steps double and the columns per
 // step shrink by more).
-template <typename D, int U, bool VY>
-__global__ __launch_bounds__(kBgmvThreads) void bgmv_expand_kernel(const BgmvBatch batch, int count,
+template <typename D, int U, bool VY, int P>
+__global__ __launch_bounds__(kBgmvThreads) void bgmv_expand_kernel(const BgmvBatchOf<P> batch, int count,
                                                                    int num_tokens, int64_t layer_idx, float scale,
                                                                    int accumulate_into_y) {
   constexpr int kWaveSums = kGroup * U * kWave;
@@ -572,28 +575,28 @@ __global__ __launch_bounds__(kBgmvThreads) void bgmv_expand_kernel(const BgmvBat
   const bool acc_y = accumulate_into_y != 0;
   const PlanOfLane plans = preload_plans(batch);
   const BatchSlot vb = batch_slot(batch, count);
-  const BgmvProblem& P = batch.p[vb.problem];
+  const BgmvProblem& prob = batch.p[vb.problem];
   // the routing record is asked for before the problem's rank is looked at: it travels with the problem's fields
   int toks[kGroup];
   int64_t stack;
-  const int n = resolve_chunk(P, reinterpret_cast<const int64_t*>(read_lane64(plans.plan, vb.problem)),
+  const int n = resolve_chunk(prob, reinterpret_cast<const int64_t*>(read_lane64(plans.plan, vb.problem)),
                               read_lane(plans.num_groups, vb.problem), num_tokens, true, vb.chunk, toks, stack);
   if (n == 0) return;
-  switch (expand_lanes_per_column(P.narrow)) {
+  switch (expand_lanes_per_column(prob.narrow)) {
     case 1:
-      bgmv_expand_problem<D, 1, U, VY>(P, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
+      bgmv_expand_problem<D, 1, U, VY>(prob, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
       break;
     case 2:
-      bgmv_expand_problem<D, 2, U, VY>(P, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
+      bgmv_expand_problem<D, 2, U, VY>(prob, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
       break;
     case 4:
-      bgmv_expand_problem<D, 4, expand_steps(4, U), VY>(P, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
+      bgmv_expand_problem<D, 4, expand_steps(4, U), VY>(prob, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
       break;
     case 8:
-      bgmv_expand_problem<D, 8, expand_steps(8, U), VY>(P, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
+      bgmv_expand_problem<D, 8, expand_steps(8, U), VY>(prob, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
       break;
     default:
-      bgmv_expand_problem<D, 16, expand_steps(16, U), VY>(P, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
+      bgmv_expand_problem<D, 16, expand_steps(16, U), VY>(prob, vb, n, toks, stack, layer_idx, scale, acc_y, wave_sums);
       break;
   }
 }
@@ -859,7 +862,7 @@ __device__ __forceinline__ bool balanced_slot(int count, int chunks, int chunks_
 // NUMBERED: problems of several column slices, numbered without gaps (launch_lora_blk).  An instantiation of its own: the
 // table walk in the same one cost the others 1 %.
 template <typename D, int R, int U, int NBLK, bool VEC4, bool NUMBERED>
-__global__ __launch_bounds__(kBgmvThreads) void bgmv_lora_kernel(const BgmvBatch batch, int h_in,
+__global__ __launch_bounds__(kBgmvThreads) void bgmv_lora_kernel(const BgmvBatchOf<kFewProblems> batch, int h_in,
                                                                  int64_t layer_idx, float scale, int count,
                                                                  int balanced_chunks, int chunks_per_xcd) {
   using E = typename D::E;
@@ -1030,9 +1033,12 @@ static hipError_t launch_shrink_rs(BgmvArgs a, hipStream_t stream) {
   const int64_t total = number_workgroups(a, [](const BgmvProblem& p) { return p.narrow / RS; });
   if (total == 0) return hipSuccess;
   if (total >= INT32_MAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((bgmv_shrink_kernel<D, RS>), dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0, stream,
-                     a.batch, a.count, static_cast<int>(a.num_tokens), a.wide_max, a.layer_idx, a.scale,
-                     a.accumulate);
+  auto launch = [&](auto kernel, const auto& batch) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0, stream, batch, a.count,
+                       static_cast<int>(a.num_tokens), a.wide_max, a.layer_idx, a.scale, a.accumulate);
+  };
+  if (a.count <= kFewProblems) launch(bgmv_shrink_kernel<D, RS, kFewProblems>, first_problems<kFewProblems>(a.batch));
+  else launch(bgmv_shrink_kernel<D, RS, kMaxBgmvProblems>, a.batch);
   return hipGetLastError();
 }
 
@@ -1068,12 +1074,17 @@ static hipError_t launch_expand_u(BgmvArgs a, hipStream_t stream) {
     const BgmvProblem& p = a.batch.p[i];
     vec_y = vec_y && p.y_stride % 8 == 0 && p.y_offset % 8 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
   }
-  if (vec_y)
-    hipLaunchKernelGGL((bgmv_expand_kernel<D, U, true>), dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0,
-                       stream, a.batch, a.count, static_cast<int>(a.num_tokens), a.layer_idx, a.scale, a.accumulate);
-  else
-    hipLaunchKernelGGL((bgmv_expand_kernel<D, U, false>), dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0,
-                       stream, a.batch, a.count, static_cast<int>(a.num_tokens), a.layer_idx, a.scale, a.accumulate);
+  auto launch = [&](auto kernel, const auto& batch) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0, stream, batch, a.count,
+                       static_cast<int>(a.num_tokens), a.layer_idx, a.scale, a.accumulate);
+  };
+  if (a.count <= kFewProblems) {
+    const auto few = first_problems<kFewProblems>(a.batch);
+    vec_y ? launch(bgmv_expand_kernel<D, U, true, kFewProblems>, few) : launch(bgmv_expand_kernel<D, U, false, kFewProblems>, few);
+  } else {
+    vec_y ? launch(bgmv_expand_kernel<D, U, true, kMaxBgmvProblems>, a.batch)
+          : launch(bgmv_expand_kernel<D, U, false, kMaxBgmvProblems>, a.batch);
+  }
   return hipGetLastError();
 }
 
@@ -1150,8 +1161,8 @@ static hipError_t launch_lora_blk(const BgmvArgs& a, hipStream_t stream) {
            reinterpret_cast<uintptr_t>(p.y) % 8 == 0;
   }
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kBgmvThreads), 0, stream, batch, a.h_in, a.layer_idx, a.scale, a.count,
-                       balanced_chunks, chunks_per_xcd);
+    hipLaunchKernelGGL(kernel, grid, dim3(kBgmvThreads), 0, stream, first_problems<kFewProblems>(batch), a.h_in, a.layer_idx,
+                       a.scale, a.count, balanced_chunks, chunks_per_xcd);
   };
   if (numbered_launch)
     vec4 ? launch(bgmv_lora_kernel<D, R, U, NBLK, true, true>) : launch(bgmv_lora_kernel<D, R, U, NBLK, false, true>);

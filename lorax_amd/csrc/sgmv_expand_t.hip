@@ -56,9 +56,10 @@ struct ExpandSlot {
   int tile_slots;  // row tiles counted for the grid
   int subs;        // pieces of sub_rows rows a tile is cut into; the last one takes what is left
 };
+template <int MAX>
 struct ExpandLaunch {
-  ExpandSlot p[kMaxExpandProblems];
-  int wg_end[kMaxExpandProblems];  // problem i owns the workgroups [wg_end[i - 1], wg_end[i])
+  ExpandSlot p[MAX];
+  int wg_end[MAX];  // problem i owns the workgroups [wg_end[i - 1], wg_end[i])
 };
 
 // NJ accumulators per wave, a panel of 16 * NJ output columns.  Accumulator j stands for the columns
@@ -182,8 +183,9 @@ __device__ __forceinline__ void expand_tile(const ExpandSlot& P, const typename 
 }
 
 // KS: 32-wide k steps of the largest rank in the launch; MIXED: the problems' ranks differ in it.
-template <typename D, int KS, int NJ, bool MIXED>
-__global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const ExpandLaunch batch, int count, int num_tokens,
+// MAX: problems the arguments hold (kFewProblems or all).
+template <typename D, int KS, int NJ, bool MIXED, int MAX>
+__global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const ExpandLaunch<MAX> batch, int count, int num_tokens,
                                                                     int64_t layer_idx, int accumulate_into_y,
                                                                     int sub_rows) {
   using E = typename D::E;
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const Expan
   int vid = static_cast<int>(blockIdx.x);
   int prob = 0;
   if (count > 1) {  // lane i looks at problem i's range: one trip to the kernel arguments
-    const int end = batch.wg_end[lane < kMaxExpandProblems ? lane : kMaxExpandProblems - 1];
+    const int end = batch.wg_end[lane < MAX ? lane : MAX - 1];
     prob = __popcll(__ballot(lane + 1 < count && vid >= end));
     if (prob > 0) vid -= read_lane(end, prob - 1);
   }
@@ -239,10 +241,10 @@ __global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const Expan
   }
 }
 
-template <typename D, int KS, bool MIXED>
-static hipError_t launch_expand_t_ks(const ExpandArgs& a, hipStream_t stream) {
+template <typename D, int KS, bool MIXED, int MAX>
+static hipError_t launch_expand_t_max(const ExpandArgs& a, hipStream_t stream) {
   constexpr int kCols = 16 * kExpTLaneCols;
-  ExpandLaunch b{};
+  ExpandLaunch<MAX> b{};
   // The kernel addresses a tile with 32-bit element offsets, and without a plan a tile is up to 9/8 of the searched
   // height + 15 rows high (merged remainders): rows of more than 2^23 elements get lower tiles.
   auto fits = [](int64_t rows, int64_t stride) { return stride * rows < (1ll << 32); };
@@ -297,10 +299,16 @@ static hipError_t launch_expand_t_ks(const ExpandArgs& a, hipStream_t stream) {
     b.wg_end[i] = static_cast<int>(total);
   }
   if (total == 0) return hipSuccess;
-  hipLaunchKernelGGL((sgmv_expand_t_kernel<D, KS, kExpTLaneCols, MIXED>), dim3(static_cast<unsigned>(total)),
+  hipLaunchKernelGGL((sgmv_expand_t_kernel<D, KS, kExpTLaneCols, MIXED, MAX>), dim3(static_cast<unsigned>(total)),
                      dim3(kExpTThreads), 0, stream, b, a.count, static_cast<int>(a.num_tokens), a.layer_idx, a.accumulate,
                      sub_rows);
   return hipGetLastError();
+}
+
+template <typename D, int KS, bool MIXED>
+static hipError_t launch_expand_t_ks(const ExpandArgs& a, hipStream_t stream) {
+  return a.count <= kFewProblems ? launch_expand_t_max<D, KS, MIXED, kFewProblems>(a, stream)
+                                 : launch_expand_t_max<D, KS, MIXED, kMaxExpandProblems>(a, stream);
 }
 
 template <typename D>
