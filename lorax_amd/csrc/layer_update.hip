@@ -16,6 +16,14 @@ constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 
 constexpr int kFusedSlab = 128 * 1024;      // bytes of A that the single-launch updates read again per slice or row chunk
 constexpr int kFusedWidthMax = 16384;       // columns up to which repeating the shrink per slice can pay (an LM head: no)
 constexpr int kNumCus = 256;
+// Summed rank of the projections that lorax_sgmv_shrink_groups is handed as one group, where it takes all of several groups
+// in one launch (tiles of up to 32 rows).  A workgroup holds its group's A tile next to its rows of x: at a summed rank of 128 two
+// stages of 36 KB fit where two workgroups share a CU, at 64 three of 20 KB, and the tiles of the high ranks are no longer
+// the ones the launch waits for.  GPU time of four Mistral-7B layers of 786 rows at rank 64 529 -> 510 us, of two of 2062
+// rows at ranks 8 to 64 484 -> 464 us; summed ranks of 32: 510 and 477 us.  Projections that one group of up to 128 holds
+// stay together (q, k and v of 2009 rows at rank 32 in one group 56 us a layer, in two 64).
+constexpr int kGroupedRank = 64;
+constexpr int kGroupedTileRows = 32;
 
 struct Job {
   const lorax_table_group_t* g;
@@ -134,9 +142,13 @@ int prefill(const Call& c, Job* const* jobs, int count) {
     for (int k = i; k < end; ++k) split = split && jobs[k]->g->plan_off >= 0 && jobs[k]->g->num_chunks <= kMaxBgmvRows;
     const int32_t n_long = split ? g.num_long_segments : g.num_segments;
     const bool planned = n_long == g.num_long_segments;  // the tables' row-tile plans cover these segments
-    // one shrink launch for up to four projections: of a short batch at any rank, else of a summed rank of 128
-    const int step = c.rows <= kShortBatchRows || kMaxKernelRank / g.rank >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup
-                                                                                                   : kMaxKernelRank / g.rank;
+    // one shrink of up to four projections: of a short batch at any rank, else of a summed rank of 128 - of 64 where that
+    // makes several groups anyway and their tiles are low enough for all to be one launch (see kGroupedRank)
+    const bool alone = end - i == count && count * g.rank <= kMaxKernelRank;
+    const int stacked = planned && !alone && g.shrink_tile_rows <= kGroupedTileRows && g.rank <= kGroupedRank ? kGroupedRank
+                                                                                                           : kMaxKernelRank;
+    const int step = c.rows <= kShortBatchRows || stacked / g.rank >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup
+                                                                                            : stacked / g.rank;
     for (int k = i; k < end && n_long > 0; k += step) {
       lorax_sgmv_shrink_problem_t* p = problems[num_shrinks];
       int n = 0;

@@ -540,7 +540,7 @@ static hipError_t launch_lds_m(const SgmvArgs& a, const LdsLaunch& l, hipStream_
   // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU; a third of it when the
   // workgroups make one to three rounds over the CUs (more resident workgroups even out the last round);
   // half of it for long launches.  2 to 8 stages.
-  int budget = wgs <= 256 ? 150 * 1024 : (wgs <= 768 ? 50 * 1024 : 76 * 1024);
+  int budget = wgs <= 256 ? 150 * 1024 : 76 * 1024;
   if (tuning().shrink_lds_kb > 0) budget = tuning().shrink_lds_kb * 1024;
   int stages = budget / kStageBytes;
   stages = stages < 2 ? 2 : (stages > kLdsMaxStages ? kLdsMaxStages : stages);
@@ -682,8 +682,10 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
   }
   const int kparts = sgmv_shrink_groups_kparts(groups, count);
   const int64_t wgs = tiles * kparts;
-  // stage buffers as in launch_lds_m, but never less than two stages of the largest group
-  int budget = wgs <= 256 ? 150 * 1024 : (wgs <= 768 ? 50 * 1024 : 76 * 1024);
+  // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU, else half of it (a third for the launches
+  // of one to three rounds, as in launch_lds_m: 484 against 476 us on the 2062-row batch above), and never less than two
+  // stages of the largest group.
+  int budget = wgs <= 256 ? 150 * 1024 : 76 * 1024;
   if (tuning().shrink_lds_kb > 0) budget = tuning().shrink_lds_kb * 1024;
   if (budget < 2 * stage_max) budget = 2 * stage_max;
   int lds_bytes = 0;

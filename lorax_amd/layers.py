@@ -230,7 +230,7 @@ class LoraLinear(nn.Module):
     def _prefill(self, result, input, groups):
         """The segment launches of forward_layer_types for jobs that touch disjoint elements of `result`: a group is
         [(rank_segments, start, width)] of the projections of one rank with the same segment tables.  Those shrink
-        together, as many per launch as fit a summed rank of 128 - x is read once per launch; the expands of all
+        together, as many per group as fit a summed rank of 128 or, in tiles of up to 32 rows, 64; the expands of all
         projections and ranks are one launch.  (The reference issues a shrink and an expand per projection and rank,
         utils/layers.py:121-143.)"""
         rows = input.size(0)
@@ -265,7 +265,11 @@ class LoraLinear(nn.Module):
             planned = n_long == first.num_long_segments
             # v needs no zero-fill: the shrinks overwrite the rows of their segments and the expands read no others
             vs = list(torch.empty((len(group), rows, r), dtype=input.dtype, device=input.device).unbind(0))
-            step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, MAX_RANK_CUSTOM // r))
+            # (several groups of tiles of up to 32 rows are one launch, which evens out better at summed ranks of 64)
+            alone = len(groups) == 1 and len(group) * r <= MAX_RANK_CUSTOM
+            grouped = (planned and not alone and first.shrink_tiles is not None and first.shrink_tiles.tile_rows <= 32
+                       and r <= 64)
+            step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, (64 if grouped else MAX_RANK_CUSTOM) // r))
             if rows <= _native.SGMV_LORA_MAX_TOKENS:
                 step = MAX_SGMV_SHRINK_PROBLEMS  # the streaming shrink of a short batch takes any ranks
             # (no long segment at all: the per-token launches do the whole update)
