@@ -302,12 +302,13 @@ struct ShrinkSlot {
   int nb;      // 16-column rank blocks of the stacked A tile
   int mblk;    // 16-row blocks of the stage buffers, 1 or 2
   int stages;
+  int kparts;  // parts its hidden dimension is cut into
 };
 constexpr int kMaxShrinkSlots = 16;
 struct ShrinkLaunch {
   ShrinkSlot p[kMaxShrinkSlots];
   int wg_end[kMaxShrinkSlots];    // slot i owns the workgroups [wg_end[i - 1], wg_end[i])
-  int tile_end[kMaxShrinkSlots];  // the same in row tiles (the launch that adds the parts)
+  int tile_end[kMaxShrinkSlots];  // the same in row tiles of the slots cut into parts (the launch that adds them)
 };
 
 // Slot of workgroup `id`; turns id into its number inside the slot.
@@ -323,7 +324,7 @@ template <typename D>
 __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_kernel(const ShrinkLaunch batch, int count,
                                                                          const typename D::E* __restrict__ X, int num_tokens,
                                                                          int h_in, int64_t layer_idx, float scale,
-                                                                         int accumulate_into_v, int kparts, int rotate) {
+                                                                         int accumulate_into_v, int rotate) {
   int id = static_cast<int>(xcd_virtual_id());
   const ShrinkSlot& S = batch.p[shrink_slot_of(batch.wg_end, count, id)];
   const int kpart = id / S.num_tiles;
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_kernel(const S
     constexpr int NB = decltype(nb)::value, MBLK = decltype(mblk)::value;
     const TileList plan{S.tiles, S.num_tiles, MBLK * 16};
     shrink_walk<D, NB, MBLK, true>(S.grp, X, S.s_start, S.s_end, S.num_segments, num_tokens, h_in, layer_idx, S.stages, scale,
-                                   accumulate_into_v, MBLK * 16, kparts, kpart, tile, S.num_tiles, S.num_tiles, S.partials, true,
+                                   accumulate_into_v, MBLK * 16, S.kparts, kpart, tile, S.num_tiles, S.num_tiles, S.partials, true,
                                    rotate, plan);
   };
   auto pick = [&](auto mblk) {
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_parts_kernel(
 // The same for a launch of several groups, whose sums are numbered tile by tile.
 template <typename D>
 __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_parts_kernel(const ShrinkLaunch batch, int count,
-                                                                               int num_tokens, int kparts, float scale,
+                                                                               int num_tokens, float scale,
                                                                                int accumulate_into_v) {
   using E = typename D::E;
   int tile = static_cast<int>(blockIdx.x);
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(kLdsThreads) void sgmv_shrink_groups_parts_kernel(c
     const int row = i / n4;
     const int col = (i - row * n4) * 4;
     f32x4 sum{0.f, 0.f, 0.f, 0.f};
-    for (int p = 0; p < kparts; ++p) {
+    for (int p = 0; p < S.kparts; ++p) {
       const f32x4 part = *reinterpret_cast<const f32x4*>(
           S.partials + ((static_cast<int64_t>(p) * S.num_tiles + tile) * rows + row) * R + col);
       sum[0] += part[0]; sum[1] += part[1]; sum[2] += part[2]; sum[3] += part[3];
@@ -659,6 +660,37 @@ int sgmv_shrink_groups_kparts(const SgmvArgs* groups, int count) {
   return kparts;
 }
 
+// The parts of every group where an average tile is cut into `kparts`: as many more as its tiles stage more bytes than the
+// average, so that the launch does not wait for the workgroups of the high ranks (o_proj, 2062 rows of ranks 8 to 64: a
+// workgroup streams 256 KB at rank 8 and 640 KB at rank 64).  Not into more rounds of workgroups over the CUs than equal
+// parts make.  GPU time of two Mistral-7B layers of 2062 rows at ranks 8 to 64 464 -> 442 us, of a 70B layer of 2741 rows at
+// ranks 32 and 128 577 -> 543.  Returns false, for equal parts, where the sums do not fit the scratch and where every workgroup has a CU to
+// itself: a step of its walk then takes about as long whatever it stages.
+static bool group_kparts(const SgmvArgs* groups, int count, int kparts, int* parts) {
+  const int nst = groups[0].d_in / kLdsKc;
+  const int most = nst / 8 < 8 ? nst / 8 : 8;
+  int64_t tiles = 0, staged = 0;
+  for (int i = 0; i < count; ++i) {
+    tiles += groups[i].num_tiles;
+    staged += static_cast<int64_t>(groups[i].num_tiles) * group_stage_bytes(groups[i]);
+  }
+  const int64_t rounds = (tiles * kparts + 255) / 256;
+  if (rounds < 2) return false;
+  for (double target = kparts; target >= 0.7 * kparts; target -= 0.1 * kparts) {
+    size_t bytes = 0;
+    int64_t wgs = 0;
+    for (int i = 0; i < count; ++i) {
+      const SgmvArgs& g = groups[i];
+      const int k = static_cast<int>(target * group_stage_bytes(g) * tiles / staged + 0.5);
+      parts[i] = k < 1 ? 1 : (k > most ? most : k);
+      wgs += static_cast<int64_t>(parts[i]) * g.num_tiles;
+      if (parts[i] > 1) bytes += static_cast<size_t>(parts[i]) * g.num_tiles * group_mblk(g) * 16 * group_nb(g) * 16 * sizeof(float);
+    }
+    if (wgs <= rounds * 256 && bytes <= kPartialBytes) return true;
+  }
+  return false;
+}
+
 template <typename D>
 static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStream_t stream) {
   const SgmvArgs& a = groups[0];
@@ -681,7 +713,13 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
     stage_max = stage > stage_max ? stage : stage_max;
   }
   const int kparts = sgmv_shrink_groups_kparts(groups, count);
-  const int64_t wgs = tiles * kparts;
+  int parts[kMaxShrinkSlots];
+  const bool uneven = kparts > 1 && tuning().shrink_ksplit == 0 && group_kparts(groups, count, kparts, parts);
+  int64_t wgs = 0;
+  for (int i = 0; i < count; ++i) {
+    b.p[i].kparts = uneven ? parts[i] : kparts;
+    wgs += static_cast<int64_t>(b.p[i].num_tiles) * b.p[i].kparts;
+  }
   // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU, else half of it (a third for the launches
   // of one to three rounds, as in launch_lds_m: 484 against 476 us on the 2062-row batch above), and never less than two
   // stages of the largest group.
@@ -699,9 +737,11 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
     if (s.stages * stage > lds_bytes) lds_bytes = s.stages * stage;
     if (red > lds_bytes) lds_bytes = red;
     s.partials = sums;
-    sums += static_cast<int64_t>(kparts) * s.num_tiles * s.mblk * 16 * s.nb * 16;
-    wg += static_cast<int64_t>(s.num_tiles) * kparts;
-    tile += s.num_tiles;
+    if (s.kparts > 1) {
+      sums += static_cast<int64_t>(s.kparts) * s.num_tiles * s.mblk * 16 * s.nb * 16;
+      tile += s.num_tiles;
+    }
+    wg += static_cast<int64_t>(s.num_tiles) * s.kparts;
     b.wg_end[i] = static_cast<int>(wg);
     b.tile_end[i] = static_cast<int>(tile);
   }
@@ -710,11 +750,11 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
   const int rotate = (tuning().shrink_no_rotate || fixed_order_shrink()) ? 0 : 1;
   hipLaunchKernelGGL(sgmv_shrink_groups_kernel<D>, dim3(static_cast<unsigned>(wgs)), dim3(kLdsThreads), lds_bytes, stream, b,
                      count, static_cast<const typename D::E*>(a.x), static_cast<int>(a.num_tokens), a.d_in, a.layer_idx,
-                     a.scale, a.accumulate, kparts, rotate);
+                     a.scale, a.accumulate, rotate);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || kparts == 1) return e;
-  hipLaunchKernelGGL(sgmv_shrink_groups_parts_kernel<D>, dim3(static_cast<unsigned>(tiles)), dim3(kLdsThreads), 0, stream, b,
-                     count, static_cast<int>(a.num_tokens), kparts, a.scale, a.accumulate);
+  if (e != hipSuccess || tile == 0) return e;
+  hipLaunchKernelGGL(sgmv_shrink_groups_parts_kernel<D>, dim3(static_cast<unsigned>(tile)), dim3(kLdsThreads), 0, stream, b,
+                     count, static_cast<int>(a.num_tokens), a.scale, a.accumulate);
   return hipGetLastError();
 }
 
