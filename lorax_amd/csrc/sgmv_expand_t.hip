@@ -184,8 +184,13 @@ __device__ __forceinline__ void expand_tile(const ExpandSlot& P, const typename 
 
 // KS: 32-wide k steps of the largest rank in the launch; MIXED: the problems' ranks differ in it.
 // MAX: problems the arguments hold (kFewProblems or all).
+// Registers: launches of several ranks are held to 128 (ranks up to 64: four waves per SIMD) and 168 (rank 128: three).  The
+// bodies take a few more by themselves, and the short tiles of such batches, mostly waiting for their first loads, gain from
+// the wave: GPU time of two Mistral-7B layers of 2062 rows at ranks 8 to 64 444 -> 425 us, of a gate/up and down block of
+// 2741 rows at ranks 32 and 128 207 -> 199.  One rank alone is left as it is: at rank 64 four waves gain 1-3 % in attention
+// projections and lose 1 % in large launches (a 70B layer of 4573 rows 591 -> 598 us), at rank 128 three spill (748 -> 782).
 template <typename D, int KS, int NJ, bool MIXED, int MAX>
-__global__ __launch_bounds__(kExpTThreads) void sgmv_expand_t_kernel(const ExpandLaunch<MAX> batch, int count, int num_tokens,
+__global__ __launch_bounds__(kExpTThreads, MIXED ? (KS == 2 ? 4 : 3) : 1) void sgmv_expand_t_kernel(const ExpandLaunch<MAX> batch, int count, int num_tokens,
                                                                     int64_t layer_idx, int accumulate_into_y,
                                                                     int sub_rows) {
   using E = typename D::E;
