@@ -1028,6 +1028,27 @@ static int64_t number_workgroups(BgmvArgs& a, SubsOf subs_of) {
   return total;
 }
 
+// Whether a launch passes a batch of kFewProblems.  That its problems are no more than four is not enough: the instantiations
+// are copies of the code (90 KB of it for the expand), and the launches of a step that takes both keep fetching it.  The
+// projections of one rank are at most three a launch, so a step of one rank takes only the small one: 2 to 5 % less at 8
+// rows, 0.5 % at 512.  A step of several ranks takes both (four ranks: launches of 12, 4, 8 and 4 problems), which pays while
+// the launches are short.  Replayed steps, us a layer, the small one wherever it fits against the full one everywhere, by
+// routing records of all problems: Mistral-7B, four ranks 34.2 and 34.9 at 8, 50.0 and 51.0 at 24, 62.9 and 63.5 at 36,
+// 67.7 and 67.3 at 45, 280.3 and 277.9 at 512; two ranks 78.7 and 80.0 at 36, 87.7 and 88.8 at 45, 109.9 and 108.8 at 64;
+// a 70B layer of four ranks 73.0 and 73.8 at 24, 95.7 and 96.2 at 36, 107.1 and 105.7 at 45.
+constexpr int64_t kFewRecords = 40;
+static bool pass_few_problems(const BgmvArgs& a) {
+  if (a.count > kFewProblems) return false;
+  bool one_rank = true;
+  int64_t records = 0;
+  for (int i = 0; i < a.count; ++i) {
+    const BgmvProblem& p = a.batch.p[i];
+    one_rank = one_rank && p.narrow == a.batch.p[0].narrow;
+    records += p.plan != nullptr ? p.num_groups : a.num_tokens;
+  }
+  return one_rank || records <= kFewRecords;
+}
+
 template <typename D, int RS>
 static hipError_t launch_shrink_rs(BgmvArgs a, hipStream_t stream) {
   const int64_t total = number_workgroups(a, [](const BgmvProblem& p) { return p.narrow / RS; });
@@ -1037,7 +1058,7 @@ static hipError_t launch_shrink_rs(BgmvArgs a, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0, stream, batch, a.count,
                        static_cast<int>(a.num_tokens), a.wide_max, a.layer_idx, a.scale, a.accumulate);
   };
-  if (a.count <= kFewProblems) launch(bgmv_shrink_kernel<D, RS, kFewProblems>, first_problems<kFewProblems>(a.batch));
+  if (pass_few_problems(a)) launch(bgmv_shrink_kernel<D, RS, kFewProblems>, first_problems<kFewProblems>(a.batch));
   else launch(bgmv_shrink_kernel<D, RS, kMaxBgmvProblems>, a.batch);
   return hipGetLastError();
 }
@@ -1078,7 +1099,7 @@ static hipError_t launch_expand_u(BgmvArgs a, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total)), dim3(kBgmvThreads), 0, stream, batch, a.count,
                        static_cast<int>(a.num_tokens), a.layer_idx, a.scale, a.accumulate);
   };
-  if (a.count <= kFewProblems) {
+  if (pass_few_problems(a)) {
     const auto few = first_problems<kFewProblems>(a.batch);
     vec_y ? launch(bgmv_expand_kernel<D, U, true, kFewProblems>, few) : launch(bgmv_expand_kernel<D, U, false, kFewProblems>, few);
   } else {

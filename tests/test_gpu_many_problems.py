@@ -1,5 +1,6 @@
-"""Launches of up to four problems pass their arguments in a smaller struct than launches of up to sixteen: at and beside
-that edge, several problems in one launch against one launch each, bit for bit."""
+"""Launches of up to four problems pass their arguments in a smaller struct than launches of up to sixteen - decode launches
+of several ranks only with few routing records: at and beside those edges, several problems in one launch against one
+launch each, bit for bit."""
 
 import pytest
 import torch
@@ -33,14 +34,15 @@ def test_expands(count):
     assert torch.equal(together, apart) and not torch.equal(together, y0)
 
 
+@pytest.mark.parametrize("times", [1, 4, 5, 9])  # 3, 8, 11 and 19 routing records a problem: 32 and 44 in launches of four
 @pytest.mark.parametrize("planned", [True, False])
 @pytest.mark.parametrize("count", [1, 4, 5, 16])
-def test_decode_shrinks_and_expands(count, planned):
+def test_decode_shrinks_and_expands(count, planned, times):
     gen = torch.Generator().manual_seed(count)
-    T, h_in, width = 9, 512, 264
+    T, h_in, width = 9 * times, 512, 264
     x = randn((T, h_in), 1.0, gen, torch.bfloat16, DEV)
     y0 = randn((T, width * count), 0.5, gen, torch.bfloat16, DEV)
-    slots = [0, 1, -1, 1, 0, 1, 1, 1, 1]
+    slots = [0, 1, -1, 1, 0, 1, 1, 1, 1] * times
     idx = torch.tensor(slots, device=DEV)
     shrinks, expands, plans, keep = [], [], [], []
     for i in range(count):
