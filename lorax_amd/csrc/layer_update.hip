@@ -313,7 +313,7 @@ extern "C" int lorax_stacked_update(const lorax_stacked_slice_t* slices, int32_t
                                     int64_t v_bytes, int32_t dtype, int32_t device, void* stream) {
   if (num_slices < 0 || num_slices > lorax::kMaxBgmvProblems || num_tokens < 0 || records < 0)
     return lorax::report_error(LORAX_EINVAL, "stacked update: number of slices (at most 16), rows or plan records out of range");
-  if (num_slices == 0 || num_tokens == 0 || records == 0) return LORAX_OK;
+  if (num_slices == 0 || num_tokens == 0) return LORAX_OK;
   if (slices == nullptr || plan == nullptr || y == nullptr || x == nullptr || v == nullptr)
     return lorax::report_error(LORAX_EINVAL, "null pointer argument (slices, plan, y, x or v)");
   lorax_table_group_t groups[lorax::kMaxBgmvProblems];
@@ -332,5 +332,7 @@ extern "C" int lorax_stacked_update(const lorax_stacked_slice_t* slices, int32_t
   }
   if (used > v_bytes) return lorax::report_error(LORAX_ESPACE, "stacked update: the workspace is smaller than num_tokens * ranks");
   const Call c{reinterpret_cast<const char*>(plan), y, y_stride, x, num_tokens, h_in, 0, nullptr, 0, dtype, stream};
+  // (a batch of base-model tokens only: nothing is launched, but its operands are checked like any other's)
+  if (records == 0) return decode(c, order, num_slices);
   return on_device(device, [&] { return decode(c, order, num_slices); });
 }

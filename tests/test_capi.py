@@ -238,6 +238,10 @@ def test_stacked_update_validation():
     one = pack((P, P, 0, 16, 256))
     call = lambda s, n, rows=4, records=2, v_bytes=1 << 20, plan=P: f(s, n, plan, records, P, 256, P, rows, 512, P, v_bytes, 1, 0, None)
     assert call(one, 0) == call(one, 1, rows=0) == call(one, 1, records=0) == OK  # nothing to do
+    # no row to route: nothing is launched, but a window beyond y, a width the kernels do not take and a misaligned stack are refused
+    assert call(pack((P, P, 8, 16, 256)), 1, records=0) == EINVAL and "do not hold" in _err()
+    assert call(pack((P, P, 0, 16, 252)), 1, records=0) == ENOKERNEL
+    assert call(pack((P, P + 2, 0, 16, 256)), 1, records=0) == EINVAL and "aligned" in _err()
     assert call(one, 17) == call(one, -1) == call(one, 1, rows=-1) == call(one, 1, records=-1) == EINVAL and "out of range" in _err()
     assert call(one, 1, plan=None) == EINVAL and "null" in _err()
     for rank in (4, 12, 136):

@@ -316,5 +316,11 @@ def test_stacked_update_from_one_call_equals_the_operators(ranks, widths, tokens
     assert not wrapper.add_lora_update(left, x.float(), slices[:1]) and not wrapper.add_lora_update(left.t(), x, slices[:1])
     wrapper.update_metadata(make_meta([s + 1 for s in slots], torch.device(DEV)), True)
     assert not wrapper.add_lora_update(left, x, slices[:1])  # prefill
+    wrapper.update_metadata(make_meta([0] * tokens, torch.device(DEV)), False)  # base model only: no routing records
+    beyond = [(a, b, y0.shape[1] - width + 8, width)]
+    for update in (wrapper.add_lora_update, lambda *args: wrapper.add_lora_slices(*args, 1.0)):
+        with pytest.raises(RuntimeError, match="do not hold"):
+            update(left, x, beyond)
+    assert wrapper.add_lora_update(left, x, slices[:1])
     torch.cuda.synchronize()
     assert torch.equal(left, y0)
