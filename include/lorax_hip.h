@@ -216,7 +216,8 @@ int lorax_sgmv_shrink_static(void* v, const void* x, const int64_t* w_ptrs, cons
  * number inside its segment.  Every row of every non-empty segment must be in exactly one tile, and no tile may
  * be higher than tile_rows.  lorax_sgmv_plan_tiles builds such a list from host copies of the tables (and
  * lorax_build_batch_tables emits one per rank group).  A launch that is captured keeps its num_tiles and tile_rows, so
- * records written for a later replay must stay within both (a record of zeros is padding); the expands take tiles of up
+ * records written for a later replay must stay within both (a record of zeros is padding; LORAX_TILES_EXPAND and
+ * LORAX_TILES_EXPAND_BATCH say how many a smaller batch can have); the expands take tiles of up
  * to 304 rows, the highest that lorax_sgmv_plan_tiles cuts, whatever tile_rows was, for rows of y of up to 14 million
  * elements.  Records are clamped on the device to the call's num_segments, num_tokens and tile_rows (expands: 304 if that
  * is more), and a tile whose segment has a null table entry is skipped, so a wrong
@@ -239,7 +240,11 @@ typedef struct lorax_sgmv_tiles {
 } lorax_sgmv_tiles_t;
 
 #define LORAX_TILES_SHRINK 0 /* for lorax_sgmv_shrink_multi: tiles of at most 64 rows                    */
-#define LORAX_TILES_EXPAND 1 /* for lorax_sgmv_expand_planned: tiles of about 1/16 of the rows, 64 to 256  */
+#define LORAX_TILES_EXPAND 1 /* for lorax_sgmv_expand_planned: tiles of about 256 rows                   */
+/* The same, for one batch: tiles of about 1/16 of the rows, 64 to 256, as lorax_build_batch_tables cuts them.  Faster below
+   4096 rows.  The cut of a segment depends on the others: unlike a plan of LORAX_TILES_EXPAND, whose records become no more
+   when segments become shorter, this one's are bounded only by max(16, rows / 256) + the number of segments with rows. */
+#define LORAX_TILES_EXPAND_BATCH 2
 
 /*
  * Builds a tile plan on the HOST: s_start / s_end are host copies of the segment tables of the launch (empty and
@@ -367,7 +372,7 @@ int lorax_sgmv_expand(void* y, const void* v, const int64_t* w_ptrs, const int32
                       int32_t dtype, void* stream);
 
 /*
- * lorax_sgmv_expand over B^T stacks (LORAX_B_HR) with a row-tile plan (LORAX_TILES_EXPAND) and without the tmp
+ * lorax_sgmv_expand over B^T stacks (LORAX_B_HR) with a row-tile plan (LORAX_TILES_EXPAND or _BATCH) and without the tmp
  * argument, which that kernel has no use for.  No counterpart in the reference.  Same result as lorax_sgmv_expand,
  * bit for bit (every element of the update is one dot product over r whatever the tiling); `tiles` may be NULL.
  */
@@ -394,7 +399,7 @@ typedef struct lorax_sgmv_expand_problem {
   int32_t h_out;
   int64_t y_offset;
   int64_t y_stride;
-  const lorax_sgmv_tiles_t* tiles; /* row-tile plan (LORAX_TILES_EXPAND) or NULL; host struct, read during the call */
+  const lorax_sgmv_tiles_t* tiles; /* row-tile plan (LORAX_TILES_EXPAND or _BATCH) or NULL; host struct, read during the call */
 } lorax_sgmv_expand_problem_t;
 
 int lorax_sgmv_expand_multi(const lorax_sgmv_expand_problem_t* problems, int32_t num_problems, int64_t num_tokens,
@@ -427,7 +432,7 @@ size_t lorax_sgmv_tmp_size(int32_t num_problems);
  *   kernels over the whole table.  The reference routes every row of such a batch through its segment kernels
  *   (lorax_server/adapters/lora.py:279, server/lorax_server/models/flash_causal_lm.py:1594).
  * Every segment-table group also carries the row-tile plans of its first num_long_segments segments for
- *   lorax_sgmv_shrink_multi and lorax_sgmv_expand_planned (the builder has the segment lengths anyway).
+ *   lorax_sgmv_shrink_multi (LORAX_TILES_SHRINK) and lorax_sgmv_expand_planned (LORAX_TILES_EXPAND_BATCH; the builder has the segment lengths anyway).
  */
 typedef struct lorax_adapter_entry {
   int64_t adapter; /* adapter index as it appears in adapter_indices            */

@@ -108,7 +108,7 @@ class SgmvExpandProblem(ctypes.Structure):
                 ("y_offset", _c.c_int64), ("y_stride", _c.c_int64), ("tiles", _c.POINTER(SgmvTiles))]
 
 
-TILES_SHRINK, TILES_EXPAND = 0, 1
+TILES_SHRINK, TILES_EXPAND, TILES_EXPAND_BATCH = 0, 1, 2
 
 
 class TilePlan:

@@ -322,7 +322,7 @@ def _tile_plans(starts: List[int], ends: List[int], num_long: int, device, rank:
         return None, None
     rows = max(ends[:num_long], default=0)
     plans = []
-    for kind in (_native.TILES_SHRINK, _native.TILES_EXPAND):
+    for kind in (_native.TILES_SHRINK, _native.TILES_EXPAND_BATCH):
         records, tile_rows = _native.plan_tiles(starts[:num_long], ends[:num_long], rows, kind, rank)
         plans.append(_native.TilePlan(torch.from_numpy(records.copy()).to(device), tile_rows))
     return plans[0], plans[1]

@@ -84,23 +84,24 @@ inline int plan_shrink_tiles(const std::vector<SegmentSpan>& segs, std::vector<l
   return rows;
 }
 
-// Nominal height of the expand's tiles: a sixteenth of the rows, between 64 and 256.  A workgroup walks its tile's rows
+// Nominal height of the expand's tiles in a plan made for one batch (LORAX_TILES_EXPAND_BATCH): a sixteenth of the rows, between
+// 64 and 256.  It depends on all segments: a batch of shorter ones can have more tiles (1025 rows 12, 1024 rows 16), never more
+// than max(16, rows / 256) and one a segment.  A workgroup walks its tile's rows
 // one block after the other, so a launch of a few segments of different lengths is as long as its tallest tile: ten
 // segments of 33 to 256 rows (rank 64, four Mistral-7B layers) take 571 / 543 / 528 us of GPU time in tiles of up to
 // 256 / 128 / 64 rows, segments of 24 to 900 rows of four ranks 514 / 480 / 482 us.  Lower tiles fetch their panels of
 // B^T more often: a 4096-row run at rank 128 1873 / 1885 / 1922 us, 15136 rows at rank 64 624 / 623 / 643 us.
-inline int expand_tile_rows(int64_t rows_total) {
+inline int expand_tile_rows(const std::vector<SegmentSpan>& segs) {
+  int64_t rows_total = 0;
+  for (const SegmentSpan& s : segs) rows_total += s.end - s.start;
   return static_cast<int>(std::min<int64_t>(std::max<int64_t>((rows_total + 255) / 256 * 16, 64), kExpandTileRows));
 }
 
-// Expand tiles: nominally expand_tile_rows high; a remainder of at most an eighth of the segment's full tiles is shared out
+// Expand tiles: nominally `rows` high; a remainder of at most an eighth of the segment's full tiles is shared out
 // among them instead of becoming a tile of its own (a tile's prologue costs as much as a hundred rows), and the
 // segment's tiles get equal heights in 16-row blocks - the rule of the device-side search (merged_tile_count).
 // Returns the height of the tallest tile (the launcher cuts tiles into pieces by it); none is above kExpandTileRowsMax.
-inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<lorax_sgmv_tile_t>& out) {
-  int64_t rows_total = 0;
-  for (const SegmentSpan& s : segs) rows_total += s.end - s.start;
-  const int rows = expand_tile_rows(rows_total);
+inline int plan_expand_tiles(const std::vector<SegmentSpan>& segs, std::vector<lorax_sgmv_tile_t>& out, int rows) {
   int tallest = 1;
   for (const SegmentSpan& s : segs) {
     const int len = s.end - s.start;

@@ -256,7 +256,7 @@ def test_plan_tiles_cuts_every_row_once():
     starts = [5, 100, 100, -1, 400, 2000]
     ends = [47, 100, 90, -1, 1500, 2003]
     T = 2500
-    for kind, limit in ((_native.TILES_SHRINK, 64), (_native.TILES_EXPAND, 256 + 32 + 16)):
+    for kind, limit in ((_native.TILES_SHRINK, 64), (_native.TILES_EXPAND, 256 + 32 + 16), (_native.TILES_EXPAND_BATCH, 256 + 32 + 16)):
         records, tile_rows = _native.plan_tiles(starts, ends, T, kind)
         assert tile_rows <= limit
         covered = {}
@@ -284,6 +284,31 @@ def test_plan_tiles_cuts_every_row_once():
     # 64 they go down to 16 (256 tiles, one per CU)
     assert _native.plan_tiles([0], [4096], 4096, _native.TILES_SHRINK, 128)[1] == 32
     assert _native.plan_tiles([0], [4096], 4096, _native.TILES_SHRINK, 64)[1] == 16
+
+
+def test_expand_tile_counts_of_smaller_batches():
+    """What a caller that sized its records, or captured a launch, for its largest batch relies on: with LORAX_TILES_EXPAND
+    shorter segments never make more records; plans for one batch stay below the bound that the header names."""
+    import random
+
+    def count(lens, kind):
+        bounds = [sum(lens[:i]) for i in range(len(lens) + 1)]
+        return len(_native.plan_tiles(bounds[:-1], bounds[1:], bounds[-1], kind)[0])
+
+    most = 0
+    for n in range(4500):
+        now = count([n], _native.TILES_EXPAND)
+        assert most <= now <= n // 256 + 1
+        most = now
+    rng = random.Random(3)
+    for _ in range(400):
+        lens = [rng.choice([0, 1, 15, 64, 65, 200, 256, 289, 700, 1025, 2100]) for _ in range(rng.randrange(1, 12))]
+        shorter = [rng.randint(0, n) for n in lens]
+        assert count(shorter, _native.TILES_EXPAND) <= count(lens, _native.TILES_EXPAND) <= sum(lens) // 256 + len(lens)
+        for batch in (lens, shorter):
+            bound = max(16, sum(batch) // 256) + sum(n > 0 for n in batch)
+            assert count(batch, _native.TILES_EXPAND_BATCH) <= bound
+    assert count([1024], _native.TILES_EXPAND_BATCH) == 16 and count([1025], _native.TILES_EXPAND_BATCH) == 12
 
 
 def test_python_binding_rejects_cpu_tensors():

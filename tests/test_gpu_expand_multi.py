@@ -115,7 +115,7 @@ def test_every_element_of_the_expand_is_written_once(h_out, lens, planned):
     bt[:, :, 3] = 1.0
     tiles = None
     if planned:
-        records, rows = _native.plan_tiles(starts, ends, T, _native.TILES_EXPAND)
+        records, rows = _native.plan_tiles(starts, ends, T, _native.TILES_EXPAND_BATCH)
         tiles = _native.TilePlan(torch.from_numpy(records.copy()).to(DEV), rows)
     y = torch.zeros((T, h_out + 2 * off), dtype=torch.bfloat16, device=DEV)
     s, e = (torch.tensor(b, dtype=torch.int32, device=DEV) for b in (starts, ends))
