@@ -493,7 +493,7 @@ int lorax_build_batch_tables(const int64_t* adapter_indices, int64_t num_tokens,
  * that of a table with a routing plan, whose records may name rows that x and y do not have.
  */
 /*
- * The two routing rules of lorax_layer_update, for callers that issue the single entry points themselves (host only, no
+ * The routing rules of lorax_layer_update, for callers that issue the single entry points themselves (host only, no
  * GPU state): whether the update of these projections of a decode batch goes out as single-launch updates
  * (lorax_bgmv_lora_multi, one per rank) rather than as a shrink and an expand launch, and whether that of a rank's
  * projections (the widest of `widest` columns) in a prefill batch does (lorax_sgmv_lora_multi).  1 = yes.
@@ -506,6 +506,18 @@ typedef struct lorax_decode_job {
 
 int lorax_decode_in_one_launch(const lorax_decode_job_t* jobs, int32_t num_jobs, int64_t num_tokens, int32_t h_in);
 int lorax_prefill_in_one_launch(int32_t rank, int32_t h_in, int64_t num_tokens, int32_t widest);
+
+/* The third rule: the summed rank, 64 or 128, up to which the projections of each of these groups are handed to
+ * lorax_sgmv_shrink_groups as one of its groups (at most 4, at least one).  A group: the projections of one rank over the same
+ * segments that have rows for the segment kernels. */
+typedef struct lorax_shrink_plan {
+  int32_t rank;
+  int32_t num_problems; /* projections                                  */
+  int32_t num_tiles;    /* of their row-tile plan (shrink); 0 = no plan */
+  int32_t tile_rows;
+} lorax_shrink_plan_t;
+
+int lorax_shrink_summed_rank(const lorax_shrink_plan_t* groups, int32_t num_groups, int64_t num_tokens, int32_t h_in);
 
 typedef struct lorax_layer_slice {
   int32_t layer_type;

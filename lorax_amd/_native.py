@@ -213,6 +213,7 @@ _SIGNATURES = {
          _c.POINTER(_c.c_int32)],
     ),
     "lorax_decode_in_one_launch": (_c.c_int, [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32]),
+    "lorax_shrink_summed_rank": (_c.c_int, [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32]),
     "lorax_prefill_in_one_launch": (_c.c_int, [_c.c_int32, _c.c_int32, _c.c_int64, _c.c_int32]),
     "lorax_layer_update": (
         _c.c_int,
@@ -484,6 +485,17 @@ def decode_in_one_launch(jobs, num_tokens: int, h_in: int) -> bool:
     per rank) rather than as a shrink and an expand launch.  `jobs`: (rank, columns, routing records) per projection."""
     packed = b"".join([_DECODE_JOB.pack(*job) for job in jobs])
     return lib().lorax_decode_in_one_launch(packed, len(jobs), num_tokens, h_in) != 0
+
+
+_SHRINK_PLAN = struct.Struct("4i")  # lorax_shrink_plan_t
+
+
+def shrink_summed_rank(groups, num_tokens: int, h_in: int) -> int:
+    """lorax_shrink_summed_rank: the summed rank up to which projections go to sgmv_shrink_groups as one group.  `groups`:
+    (rank, projections, TilePlan or None) per rank group of the call that has rows for the segment kernels."""
+    packed = b"".join([_SHRINK_PLAN.pack(r, n, tiles.num_tiles if tiles is not None else 0, tiles.tile_rows if tiles is not None else 0)
+                       for r, n, tiles in groups])
+    return lib().lorax_shrink_summed_rank(packed, len(groups), num_tokens, h_in)
 
 
 def bgmv_lora_fits(rank: int, h_in: int, h_out: int) -> bool:

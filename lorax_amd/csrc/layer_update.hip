@@ -16,14 +16,9 @@ constexpr int64_t kShortBatchRows16 = 128;  // ... and of the latter at rank 16 
 constexpr int kFusedSlab = 128 * 1024;      // bytes of A that the single-launch updates read again per slice or row chunk
 constexpr int kFusedWidthMax = 16384;       // columns up to which repeating the shrink per slice can pay (an LM head: no)
 constexpr int kNumCus = 256;
-// Summed rank of the projections that lorax_sgmv_shrink_groups is handed as one group, where it takes all of several groups
-// in one launch (tiles of up to 32 rows).  A workgroup holds its group's A tile next to its rows of x: at a summed rank of 128 two
-// stages of 36 KB fit where two workgroups share a CU, at 64 three of 20 KB, and the tiles of the high ranks are no longer
-// the ones the launch waits for.  GPU time of four Mistral-7B layers of 786 rows at rank 64 529 -> 510 us, of two of 2062
-// rows at ranks 8 to 64 484 -> 464 us; summed ranks of 32: 510 and 477 us.  Projections that one group of up to 128 holds
-// stay together (q, k and v of 2009 rows at rank 32 in one group 56 us a layer, in two 64).
-constexpr int kGroupedRank = 64;
-constexpr int kGroupedTileRows = 32;
+constexpr int kGroupedRank = 64;      // lorax_shrink_summed_rank
+constexpr int kGroupedTileRows = 32;  // highest row tiles that lorax_sgmv_shrink_groups takes several groups of in one launch
+constexpr int kShrinkBatch = 16;      // groups of one call of lorax_sgmv_shrink_groups
 
 struct Job {
   const lorax_table_group_t* g;
@@ -103,7 +98,6 @@ int prefill(const Call& c, Job* const* jobs, int count) {
   const Job* shorts[kMaxJobs];
   int32_t expand_segments[kMaxJobs];
   int num_expand = 0, num_shorts = 0;
-  constexpr int kShrinkBatch = 16;
   lorax_sgmv_shrink_problem_t problems[kShrinkBatch][lorax::kMaxShrinkGroup];
   lorax_sgmv_tiles_t tiles[kShrinkBatch];
   lorax_sgmv_shrink_group_t shrinks[kShrinkBatch];
@@ -114,15 +108,39 @@ int prefill(const Call& c, Job* const* jobs, int count) {
     return lorax_sgmv_shrink_groups(shrinks, n, c.x, c.rows, c.h_in, c.layer_idx, 1.0f, 0, c.tmp, c.tmp_bytes, c.dtype,
                                     c.stream);
   };
-  // `jobs` is ordered by group of equal rank and segment tables
-  for (int i = 0, end = 0; i < count; i = end) {
+  // `jobs` is ordered by group of equal rank and segment tables: [first, end) of each
+  struct Group {
+    int first, end;
+    bool fused;      // shrink and expand in one launch
+    bool split;      // segments of a few rows go to the per-token kernels, where every projection has a plan over them
+    int32_t n_long;  // segments for the segment kernels
+    bool planned;    // the tables' row-tile plans cover these
+  } group_of[kMaxJobs];
+  lorax_shrink_plan_t plans[kMaxJobs];
+  int num_groups = 0, num_plans = 0;
+  for (int i = 0; i < count; i = group_of[num_groups++].end) {
     const lorax_table_group_t& g = *jobs[i]->g;
+    Group& q = group_of[num_groups];
+    q = {i, i, false, c.rows <= kMaxBgmvRows, 0, false};
     int widest = 0;
-    for (end = i; end < count && jobs[end]->g->rank == g.rank && jobs[end]->g->segments_id == g.segments_id; ++end)
-      widest = jobs[end]->width > widest ? jobs[end]->width : widest;
+    for (; q.end < count && jobs[q.end]->g->rank == g.rank && jobs[q.end]->g->segments_id == g.segments_id; ++q.end) {
+      const Job& j = *jobs[q.end];
+      widest = j.width > widest ? j.width : widest;
+      q.split = q.split && j.g->plan_off >= 0 && j.g->num_chunks <= kMaxBgmvRows;
+    }
+    q.fused = lorax_prefill_in_one_launch(g.rank, c.h_in, c.rows, widest) != 0;
+    q.n_long = q.split ? g.num_long_segments : g.num_segments;
+    q.planned = q.n_long == g.num_long_segments;
+    if (!q.fused && q.n_long > 0)
+      plans[num_plans++] = {g.rank, q.end - i, q.planned ? g.num_shrink_tiles : 0, q.planned ? g.shrink_tile_rows : 0};
+  }
+  const int stacked = lorax_shrink_summed_rank(plans, num_plans, c.rows, c.h_in);
+  for (int q = 0; q < num_groups; ++q) {
+    const auto [i, end, fused, split, n_long, planned] = group_of[q];
+    const lorax_table_group_t& g = *jobs[i]->g;
     const int32_t* starts = static_cast<const int32_t*>(at(c, g.starts_off));
     const int32_t* ends = static_cast<const int32_t*>(at(c, g.ends_off));
-    if (lorax_prefill_in_one_launch(g.rank, c.h_in, c.rows, widest)) {
+    if (fused) {
       for (int k = i; k < end; k += lorax::kMaxSgmvLoraProblems) {
         lorax_sgmv_lora_problem_t p[lorax::kMaxSgmvLoraProblems];
         int n = 0;
@@ -137,18 +155,9 @@ int prefill(const Call& c, Job* const* jobs, int count) {
       }
       continue;
     }
-    // segments of a few rows go to the per-token kernels where every projection has a plan over them
-    bool split = c.rows <= kMaxBgmvRows;
-    for (int k = i; k < end; ++k) split = split && jobs[k]->g->plan_off >= 0 && jobs[k]->g->num_chunks <= kMaxBgmvRows;
-    const int32_t n_long = split ? g.num_long_segments : g.num_segments;
-    const bool planned = n_long == g.num_long_segments;  // the tables' row-tile plans cover these segments
-    // one shrink of up to four projections: of a short batch at any rank, else of a summed rank of 128 - of 64 where that
-    // makes several groups anyway and their tiles are low enough for all to be one launch (see kGroupedRank)
-    const bool alone = end - i == count && count * g.rank <= kMaxKernelRank;
-    const int stacked = planned && !alone && g.shrink_tile_rows <= kGroupedTileRows && g.rank <= kGroupedRank ? kGroupedRank
-                                                                                                           : kMaxKernelRank;
-    const int step = c.rows <= kShortBatchRows || stacked / g.rank >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup
-                                                                                            : stacked / g.rank;
+    // one shrink of up to four projections: of a short batch at any rank, else of a summed rank
+    const int fit = stacked / g.rank > 0 ? stacked / g.rank : 1;
+    const int step = c.rows <= kShortBatchRows || fit >= lorax::kMaxShrinkGroup ? lorax::kMaxShrinkGroup : fit;
     for (int k = i; k < end && n_long > 0; k += step) {
       lorax_sgmv_shrink_problem_t* p = problems[num_shrinks];
       int n = 0;
@@ -283,6 +292,28 @@ extern "C" int lorax_decode_in_one_launch(const lorax_decode_job_t* jobs, int32_
 // 54 at 192, 116 and 72 at 512; at rank 8 56 and 65 at 512.
 extern "C" int lorax_prefill_in_one_launch(int32_t rank, int32_t h_in, int64_t num_tokens, int32_t widest) {
   return fused_rank(rank, h_in) && num_tokens <= (rank == 8 ? kShortBatchRows : kShortBatchRows16) && widest <= kFusedWidthMax;
+}
+
+// lorax_sgmv_shrink_groups takes several groups in one launch only if all of them come in tiles of up to 32 rows.  There a
+// workgroup holds its group's A tile next to its rows of x: at a summed rank of 128 two stages of 36 KB fit where two
+// workgroups share a CU, at 64 three of 20 KB, and the tiles of the high ranks are no longer the ones the launch waits for -
+// unless one projection's rank is above 64, for which the launch waits as before.  Whole layers in one process, 514 to 7321
+// rows in 8 to 300 runs, attention projections of hidden size 4096, gate/up and down, a 70B layer (time at 64 over that at
+// 128, geometric mean and range): ranks 8 to 64 0.93, 0.96 and 0.97 (0.86 to 1.00), 32 and 64 0.95, 0.97 and 0.97 (0.88 to
+// 1.02), 16 and 32 0.98, 1.00 and 1.00 (0.91 to 1.05), 64 alone 0.95 and 0.99 (0.87 to 1.07: 3017 rows in tiles of 16 make
+// a third round where two groups of 128 end with the second), 32 and 128 1.04, 1.00 and 1.01 (0.94 to 1.19).
+// One group of up to 128 stays whole (q, k and v of 2009 rows at rank 32 in one group 56 us a layer, in two 64).
+extern "C" int lorax_shrink_summed_rank(const lorax_shrink_plan_t* groups, int32_t num_groups, int64_t num_tokens, int32_t h_in) {
+  if (num_groups < 1 || groups == nullptr || num_tokens <= kShortBatchRows || h_in % 128 != 0) return kMaxKernelRank;
+  int calls = 0;
+  for (int i = 0; i < num_groups; ++i) {
+    const lorax_shrink_plan_t& g = groups[i];
+    if (g.rank < 1 || g.rank > kGroupedRank || g.num_tiles < 1 || g.tile_rows > kGroupedTileRows) return kMaxKernelRank;
+    const int fit = kGroupedRank / g.rank < lorax::kMaxShrinkGroup ? kGroupedRank / g.rank : lorax::kMaxShrinkGroup;
+    calls += (g.num_problems + fit - 1) / fit;
+  }
+  const bool alone = num_groups == 1 && groups[0].num_problems * groups[0].rank <= kMaxKernelRank;
+  return alone || calls > kShrinkBatch ? kMaxKernelRank : kGroupedRank;
 }
 
 extern "C" int lorax_layer_update(const lorax_table_group_t* groups, int32_t num_groups, const void* tables,

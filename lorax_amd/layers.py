@@ -34,7 +34,6 @@ from lorax_amd.adapters import LORA, AdapterBatchData, BatchLoraWeights
 from lorax_amd._native import MAX_SGMV_SHRINK_PROBLEMS
 from lorax_amd.punica_wrapper import PunicaWrapper
 from lorax_amd.sgmv import (
-    MAX_RANK_CUSTOM,
     get_shrink_scratch,
     get_tmp_expand_size,
     has_sgmv,
@@ -230,11 +229,12 @@ class LoraLinear(nn.Module):
     def _prefill(self, result, input, groups):
         """The segment launches of forward_layer_types for jobs that touch disjoint elements of `result`: a group is
         [(rank_segments, start, width)] of the projections of one rank with the same segment tables.  Those shrink
-        together, as many per group as fit a summed rank of 128 or, in tiles of up to 32 rows, 64; the expands of all
+        together, as many per group as fit the summed rank of _native.shrink_summed_rank; the expands of all
         projections and ranks are one launch.  (The reference issues a shrink and an expand per projection and rank,
         utils/layers.py:121-143.)"""
         rows = input.size(0)
-        shrinks, expands, short_shrinks, short_expands = [], [], [], []
+        expands, short_shrinks, short_expands = [], [], []
+        shrink_jobs = []  # (rank, [v], [table], starts, ends, tiles) per group with rows for the segment kernels
         for group in groups:
             r = group[0][0].rank
             if _native.sgmv_lora_fits(r, input.size(1), rows, max(width for _, _, width in group)):
@@ -265,17 +265,10 @@ class LoraLinear(nn.Module):
             planned = n_long == first.num_long_segments
             # v needs no zero-fill: the shrinks overwrite the rows of their segments and the expands read no others
             vs = list(torch.empty((len(group), rows, r), dtype=input.dtype, device=input.device).unbind(0))
-            # (several groups of tiles of up to 32 rows are one launch, which evens out better at summed ranks of 64)
-            alone = len(groups) == 1 and len(group) * r <= MAX_RANK_CUSTOM
-            grouped = (planned and not alone and first.shrink_tiles is not None and first.shrink_tiles.tile_rows <= 32
-                       and r <= 64)
-            step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, (64 if grouped else MAX_RANK_CUSTOM) // r))
-            if rows <= _native.SGMV_LORA_MAX_TOKENS:
-                step = MAX_SGMV_SHRINK_PROBLEMS  # the streaming shrink of a short batch takes any ranks
             # (no long segment at all: the per-token launches do the whole update)
-            for i in range(0, len(group) if n_long > 0 else 0, step):
-                shrinks.append((vs[i : i + step], [rs.lora_a_t_ptr[:n_long] for rs, _, _ in group[i : i + step]], starts, ends,
-                                first.shrink_tiles if planned else None))
+            if n_long > 0:
+                shrink_jobs.append((r, vs, [rs.lora_a_t_ptr[:n_long] for rs, _, _ in group], starts, ends,
+                                    first.shrink_tiles if planned else None))
             for v, plan, (rs, start, width) in zip(vs, plans, group):
                 if n_long > 0:
                     expands.append((result, v, rs.lora_b_t_ptr[:n_long], starts, ends, start, width,
@@ -284,6 +277,13 @@ class LoraLinear(nn.Module):
                 if split:
                     short_shrinks.append(((v, input, None, None, 0, None), plan))
                     short_expands.append(((result, v, None, None, start, width), plan))
+        shrinks = []
+        summed_rank = _native.shrink_summed_rank([(r, len(vs), tiles) for r, vs, _, _, _, tiles in shrink_jobs], rows, input.size(1))
+        for r, vs, tables, starts, ends, tiles in shrink_jobs:
+            step = max(1, min(MAX_SGMV_SHRINK_PROBLEMS, summed_rank // r))
+            if rows <= _native.SGMV_LORA_MAX_TOKENS:
+                step = MAX_SGMV_SHRINK_PROBLEMS  # the streaming shrink of a short batch takes any ranks
+            shrinks += [(vs[i : i + step], tables[i : i + step], starts, ends, tiles) for i in range(0, len(vs), step)]
         if len(shrinks) == 1:
             (v, tables, starts, ends, tiles), = shrinks
             _native.sgmv_shrink_multi(v, input, tables, starts, ends, get_shrink_scratch(input.device), self.layer_id, 1.0, False,

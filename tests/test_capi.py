@@ -286,6 +286,24 @@ def test_plan_tiles_cuts_every_row_once():
     assert _native.plan_tiles([0], [4096], 4096, _native.TILES_SHRINK, 64)[1] == 16
 
 
+def test_shrink_summed_rank_looks_at_the_whole_call():
+    """lorax_shrink_summed_rank: 64 only where every group of the call can be in one launch, several are, and none is higher."""
+    from types import SimpleNamespace
+
+    def rule(*groups, rows=2000, h_in=4096):
+        return _native.shrink_summed_rank([(r, n, SimpleNamespace(num_tiles=t, tile_rows=h) if t else None) for r, n, t, h in groups],
+                                          rows, h_in)
+
+    assert rule((64, 3, 120, 16)) == rule((32, 3, 60, 16), (64, 3, 60, 32)) == rule((8, 3, 9, 16), (16, 3, 9, 16)) == 64
+    assert rule((32, 3, 60, 16)) == rule((64, 2, 100, 16)) == 128            # one group of up to 128
+    assert rule((32, 3, 60, 16), (64, 3, 60, 48)) == 128                     # another group's tiles are too high ...
+    assert rule((32, 3, 60, 16), (64, 3, 0, 0)) == 128                       # ... or it has no plan
+    assert rule((32, 3, 60, 16), (128, 3, 60, 32)) == rule((64, 3, 60, 16), (72, 3, 60, 32)) == 128
+    assert rule((64, 3, 120, 16), rows=512) == rule((64, 3, 120, 16), h_in=2752) == rule() == 128
+    assert rule(*[(40 + 8 * (i % 4), 4, 20, 16) for i in range(4)]) == 64    # 16 groups ...
+    assert rule(*[(40 + 8 * (i % 4), 4, 20, 16) for i in range(5)]) == 128   # ... and more than one call takes
+
+
 def test_expand_tile_counts_of_smaller_batches():
     """What a caller that sized its records, or captured a launch, for its largest batch relies on: with LORAX_TILES_EXPAND
     shorter segments never make more records; plans for one batch stay below the bound that the header names."""

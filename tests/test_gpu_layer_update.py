@@ -192,6 +192,8 @@ def test_prefill_layers_on_two_streams(native):
     ([32], [700]),                   # one group of all three projections
     ([128, 64], [400, 200]),         # a rank that fills a group by itself
     ([64], [9000]),                  # tiles of 48 rows and more: launches of their own
+    ([64, 32], [9000, 300, 280]),    # ... next to a rank that is then alone
+    ([128, 32], [700, 300]),         # a rank above 64
 ])
 def test_prefill_shrinks_of_several_groups(ranks, lens):
     """The groups that a layer's shrinks are cut into, natively and on the general path: the same bits, and the update of

@@ -756,3 +756,35 @@ def test_decode_paths_follow_the_one_rule(monkeypatch, records, together):
     ops.bgmv_lora_slices(x, [(a, torch.zeros(2, 4096, 16, dtype=torch.bfloat16), 0, 4096)], y, torch.zeros(20, dtype=torch.int64),
                          1.0, plan=torch.zeros((records[0], 8), dtype=torch.int64))
     assert calls == (["bgmv_lora_multi"] if records[0] <= 16 else ["bgmv_stacked"])
+
+
+@pytest.mark.parametrize("spec,want", [
+    ([(32, 16, 60), (64, 16, 60)], [2, 1, 1, 1, 1]),        # all in one launch: summed ranks of 64
+    ([(32, 16, 60), (64, 48, 200)], [3, 2, 1]),             # the tall tiles of rank 64 need a call of their own
+    ([(32, 16, 60), (64, 16, 0)], [3]),                     # rank 64 has only short segments: rank 32 is alone
+])
+def test_prefill_shrinks_are_grouped_by_the_whole_call(monkeypatch, spec, want):
+    """Projections a group of LoraLinear._prefill's shrinks for q/k/v of two ranks: (rank, tile rows, tiles), none = no
+    long segment."""
+    from types import SimpleNamespace
+
+    from lorax_amd import _native, layers
+
+    calls, rows = [], 2000
+    monkeypatch.setattr(layers, "get_shrink_scratch", lambda device: None)
+    monkeypatch.setattr(_native, "sgmv_shrink_groups", lambda groups, *a: calls.extend(len(g[0]) for g in groups))
+    monkeypatch.setattr(_native, "sgmv_shrink_multi", lambda vs, *a: calls.append(len(vs)))
+    for launch in ("sgmv_expand_multi", "bgmv_multi"):
+        monkeypatch.setattr(_native, launch, lambda *a, **k: None)
+    table = torch.zeros(40, dtype=torch.int32)
+
+    def segments(rank, tile_rows, tiles):
+        plan = lambda n, height: _native.TilePlan(torch.zeros((n, 4), dtype=torch.int32), height)
+        return SimpleNamespace(rank=rank, lora_a_t_ptr=table, lora_b_t_ptr=table, segment_starts=table, segment_ends=table,
+                               num_long_segments=4 if tiles else 0, short_plan=torch.zeros((9, 8), dtype=torch.int64), num_rows=rows,
+                               shrink_tiles=plan(tiles, tile_rows), expand_tiles=plan(8, 64), tmp_expand=None)
+
+    x, y = torch.zeros((rows, 1024), dtype=torch.bfloat16), torch.zeros((rows, 6144), dtype=torch.bfloat16)
+    layers.LoraLinear(None, 0)._prefill(y, x, [[(segments(*s), start, width) for start, width in ((0, 4096), (4096, 1024), (5120, 1024))]
+                                               for s in spec])
+    assert calls == want
