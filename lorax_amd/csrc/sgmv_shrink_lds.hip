@@ -540,8 +540,13 @@ static hipError_t launch_lds_m(const SgmvArgs& a, const LdsLaunch& l, hipStream_
   const int64_t wgs = tiles * kparts;
   // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU; a third of it when the
   // workgroups make one to three rounds over the CUs (more resident workgroups even out the last round);
-  // half of it for long launches.  2 to 8 stages.
-  int budget = wgs <= 256 ? 150 * 1024 : 76 * 1024;
+  // half of it for long launches.  2 to 8 stages.  Half of it for one to three rounds: 600 segments of 16 rows over 8192
+  // columns at ranks 16 / 32 / 64 56 / 76 / 123 us, a third 48 / 62 / 81; 2160 rows at ranks 8 to 32 in K parts 2 to 5 % more.
+  // Only where a third holds no more than two stages do K parts gain from the third one: 2160 rows over 8192 and 28672 columns
+  // at rank 64 23.5 and 62.7 us in two stages, 21.0 and 55.5 in three; a Mistral-7B step of 2741 rows in the reference's
+  // layouts 389 and 374.
+  int budget = wgs <= 256 ? 150 * 1024 : (wgs <= 768 ? 50 * 1024 : 76 * 1024);
+  if (kparts > 1 && budget < 3 * kStageBytes && 3 * kStageBytes <= 76 * 1024) budget = 3 * kStageBytes;
   if (tuning().shrink_lds_kb > 0) budget = tuning().shrink_lds_kb * 1024;
   int stages = budget / kStageBytes;
   stages = stages < 2 ? 2 : (stages > kLdsMaxStages ? kLdsMaxStages : stages);
@@ -720,9 +725,10 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
     b.p[i].kparts = uneven ? parts[i] : kparts;
     wgs += static_cast<int64_t>(b.p[i].num_tiles) * b.p[i].kparts;
   }
-  // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU, else half of it (a third for the launches
-  // of one to three rounds, as in launch_lds_m: 484 against 476 us on the 2062-row batch above), and never less than two
-  // stages of the largest group.
+  // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU, else half of it, and never less than two
+  // stages of the largest group.  (A third for one to three rounds, as for a single group above: two Mistral-7B layers of
+  // 2062 rows at ranks 8 to 64 484 us, half 476; over segments of 12 to 1900 rows, where the largest group's stage is 20 KB,
+  // half takes 0.90 times as long on average - up to 1.4 where every segment is one tile -, at other sizes 0.97 to 1.07.)
   int budget = wgs <= 256 ? 150 * 1024 : 76 * 1024;
   if (tuning().shrink_lds_kb > 0) budget = tuning().shrink_lds_kb * 1024;
   if (budget < 2 * stage_max) budget = 2 * stage_max;

@@ -76,6 +76,8 @@ def test_expand_with_a_plan_is_bit_identical(dtype, r, h_out, lens):
     (1, 40, 1536, [33] * 30),                      # a rank that is not a multiple of 16
     (3, 16, 512, [9000]),                          # many tiles: more than one round over the CUs
     (2, 32, 1024, [70, 7] * 50),                   # a hundred segments: table entries past the first 64
+    (1, 64, 4096, [270] * 8),                      # 136 tiles in three parts: three stages of 20 KB
+    (1, 32, 512, [16] * 600),                      # 600 tiles: a third of the LDS each
 ])
 def test_shrink_with_a_plan(count, r, h_in, lens):
     print(f"case count={count} r={r} h_in={h_in} lens={lens}", flush=True)
