@@ -315,12 +315,17 @@ int lorax_sgmv_shrink_groups(const lorax_sgmv_shrink_group_t* groups, int32_t nu
                              int64_t num_tokens, int32_t h_in, int64_t layer_idx, float scale, int32_t accumulate,
                              void* tmp, int64_t tmp_bytes, int32_t dtype, void* stream);
 
-/* What lorax_sgmv_shrink_groups does with these groups: the parts it cuts the hidden dimension into where they go out as
- * one launch (1 = not cut; more: and a second launch that adds them; a group whose tiles stage more bytes than the others'
- * may be cut further, and one that stages fewer less far), 0 where it issues one call per group.  Host only. */
+/* What lorax_sgmv_shrink_groups does with these groups: the parts it cuts the hidden dimension of an average tile into where
+ * they go out as one launch (1 = not cut; more: and a second launch that adds them), 0 where it issues one call per group.
+ * A group whose tiles stage more bytes than the others' may be cut further, and one that stages fewer less far or not at all:
+ * _parts_of also leaves the parts of every group in `parts` (host, num_groups entries; 0 = a group without tiles) where the
+ * result is not 0.  Host only. */
 int lorax_sgmv_shrink_groups_parts(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x,
                                    int64_t num_tokens, int32_t h_in, int64_t layer_idx, int32_t accumulate, void* tmp,
                                    int64_t tmp_bytes, int32_t dtype);
+int lorax_sgmv_shrink_groups_parts_of(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x,
+                                      int64_t num_tokens, int32_t h_in, int64_t layer_idx, int32_t accumulate, void* tmp,
+                                      int64_t tmp_bytes, int32_t dtype, int32_t* parts);
 
 /* Process-wide switch (default 0): 1 = the SGMV shrinks add their sums over the hidden dimension in one fixed
  * order whatever the batch (see lorax_sgmv_shrink_multi).  Returns the previous value.  Not meant to be flipped

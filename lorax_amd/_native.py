@@ -179,6 +179,11 @@ _SIGNATURES = {
         [_c.POINTER(SgmvShrinkGroup), _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_void_p,
          _c.c_int64, _c.c_int32],
     ),
+    "lorax_sgmv_shrink_groups_parts_of": (
+        _c.c_int,
+        [_c.POINTER(SgmvShrinkGroup), _c.c_int32, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_void_p,
+         _c.c_int64, _c.c_int32, _c.c_void_p],
+    ),
     "lorax_sgmv_expand_planned": (
         _c.c_int,
         [_c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int32,
@@ -758,6 +763,17 @@ def sgmv_shrink_groups_parts(groups, x, tmp, layer_idx, accumulate: bool = True)
     return lib().lorax_sgmv_shrink_groups_parts(arr, len(groups), x.data_ptr(), x.size(0), x.size(1), int(layer_idx),
                                                 1 if accumulate else 0, tmp.data_ptr(), tmp.numel() * tmp.element_size(),
                                                 _dtype_code(x))
+
+
+def sgmv_shrink_groups_parts_of(groups, x, tmp, layer_idx, accumulate: bool = True) -> list:
+    """lorax_sgmv_shrink_groups_parts_of: those parts of every group, 0 = it has no tiles; empty where the call goes out group by
+    group."""
+    arr, _keep = _shrink_groups(groups, x, tmp)
+    parts = (_c.c_int32 * len(groups))()
+    together = lib().lorax_sgmv_shrink_groups_parts_of(arr, len(groups), x.data_ptr(), x.size(0), x.size(1), int(layer_idx),
+                                                       1 if accumulate else 0, tmp.data_ptr(), tmp.numel() * tmp.element_size(),
+                                                       _dtype_code(x), parts)
+    return list(parts) if together > 0 else []
 
 
 def plan_tiles(s_start, s_end, num_tokens: int, kind: int, rank: int = 0):

@@ -586,6 +586,20 @@ int lorax_sgmv_shrink_groups_parts(const lorax_sgmv_shrink_group_t* groups, int3
   return count > 0 ? sgmv_shrink_groups_kparts(args, count) : 0;
 }
 
+int lorax_sgmv_shrink_groups_parts_of(const lorax_sgmv_shrink_group_t* groups, int32_t num_groups, const void* x,
+                                      int64_t num_tokens, int32_t h_in, int64_t layer_idx, int32_t accumulate, void* tmp,
+                                      int64_t tmp_bytes, int32_t dtype, int32_t* parts) {
+  if (num_groups < 0 || num_groups > kMaxShrinkGroups || groups == nullptr || parts == nullptr) return 0;
+  SgmvArgs args[kMaxShrinkGroups];
+  const int count = shrink_groups_together(groups, num_groups, x, num_tokens, h_in, layer_idx, 1.0f, accumulate, tmp, tmp_bytes,
+                                           dtype, args);
+  if (count == 0) return 0;
+  int of_launched[kMaxShrinkGroups];
+  sgmv_shrink_groups_parts_of(args, count, of_launched);
+  for (int i = 0, launched = 0; i < num_groups; ++i) parts[i] = groups[i].tiles->num_tiles > 0 ? of_launched[launched++] : 0;
+  return sgmv_shrink_groups_kparts(args, count);
+}
+
 int lorax_sgmv_expand(void* y, const void* v, const int64_t* w_ptrs, const int32_t* s_start,
                       const int32_t* s_end, int32_t num_segments, int64_t num_tokens, int32_t r,
                       int32_t h_out, int32_t b_layout, int64_t y_offset, int64_t y_stride,

@@ -216,7 +216,8 @@ hipError_t launch_sgmv_shrink_lds(const SgmvArgs& a, hipStream_t stream);
 // Several groups of projections over the same x in one launch: all fields but y, w_ptrs, group, d_out, the segment
 // tables and the tile plan are those of groups[0].
 bool sgmv_shrink_groups_applies(const SgmvArgs* groups, int count);
-int sgmv_shrink_groups_kparts(const SgmvArgs* groups, int count);  // parts the hidden dimension is cut into
+int sgmv_shrink_groups_kparts(const SgmvArgs* groups, int count);  // parts the hidden dimension of an average tile is cut into
+void sgmv_shrink_groups_parts_of(const SgmvArgs* groups, int count, int* parts);  // and that of every group
 hipError_t launch_sgmv_shrink_groups(const SgmvArgs* groups, int count, hipStream_t stream);
 // Per-device set-up of the LDS-staged shrink on the current device (the dynamic LDS limit of every instantiation),
 // so that no launch has first-call state; a launch that finds it missing does it itself.

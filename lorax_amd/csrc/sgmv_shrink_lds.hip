@@ -665,7 +665,7 @@ int sgmv_shrink_groups_kparts(const SgmvArgs* groups, int count) {
   return kparts;
 }
 
-// The parts of every group where an average tile is cut into `kparts`: as many more as its tiles stage more bytes than the
+// The parts of every group where an average tile would be cut into `kparts`: as many more as its tiles stage more bytes than the
 // average, so that the launch does not wait for the workgroups of the high ranks (o_proj, 2062 rows of ranks 8 to 64: a
 // workgroup streams 256 KB at rank 8 and 640 KB at rank 64).  Not into more rounds of workgroups over the CUs than equal
 // parts make.  GPU time of two Mistral-7B layers of 2062 rows at ranks 8 to 64 464 -> 442 us, of a 70B layer of 2741 rows at
@@ -696,6 +696,12 @@ static bool group_kparts(const SgmvArgs* groups, int count, int kparts, int* par
   return false;
 }
 
+void sgmv_shrink_groups_parts_of(const SgmvArgs* groups, int count, int* parts) {
+  const int kparts = sgmv_shrink_groups_kparts(groups, count);
+  if (kparts > 1 && tuning().shrink_ksplit == 0 && group_kparts(groups, count, kparts, parts)) return;
+  for (int i = 0; i < count; ++i) parts[i] = kparts;
+}
+
 template <typename D>
 static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStream_t stream) {
   const SgmvArgs& a = groups[0];
@@ -717,12 +723,11 @@ static hipError_t launch_groups_dtype(const SgmvArgs* groups, int count, hipStre
     const int stage = group_stage_bytes(g);
     stage_max = stage > stage_max ? stage : stage_max;
   }
-  const int kparts = sgmv_shrink_groups_kparts(groups, count);
   int parts[kMaxShrinkSlots];
-  const bool uneven = kparts > 1 && tuning().shrink_ksplit == 0 && group_kparts(groups, count, kparts, parts);
+  sgmv_shrink_groups_parts_of(groups, count, parts);
   int64_t wgs = 0;
   for (int i = 0; i < count; ++i) {
-    b.p[i].kparts = uneven ? parts[i] : kparts;
+    b.p[i].kparts = parts[i];
     wgs += static_cast<int64_t>(b.p[i].num_tiles) * b.p[i].kparts;
   }
   // Stage buffers: all of a CU's LDS when there is at most one workgroup per CU, else half of it, and never less than two

@@ -102,9 +102,9 @@ def test_sgmv_shrink_multi_validation():
     assert f(two, 2, P, P, P, 2, 1000, 4096, 64, 0, 1.0, 1, P, big, ctypes.byref(empty), 1, None) == OK
 
 
-def _shrink_groups(rank, num_problems, num_groups, tile_rows=16):
+def _shrink_groups(rank, num_problems, num_groups, tile_rows=16, num_tiles=40):
     problems = (_native.SgmvShrinkProblem * num_problems)(*[_native.SgmvShrinkProblem(P, P)] * num_problems)
-    tiles = _native.SgmvTiles(P, 40, tile_rows)
+    tiles = _native.SgmvTiles(P, num_tiles, tile_rows)
     group = _native.SgmvShrinkGroup(problems, num_problems, rank, P, P, 2, ctypes.addressof(tiles))
     return (_native.SgmvShrinkGroup * num_groups)(*[group] * num_groups), (problems, tiles)
 
@@ -179,6 +179,35 @@ def test_sgmv_shrink_groups_route(ranks, problems, tile_rows, rows, h_in, one_la
     groups = (_native.SgmvShrinkGroup * 16)(*[g[0] for g, _ in made])
     for count in range(2, 17):
         assert 1 <= f(groups, count, P, 12000, 128 * 67, 0, 0, P, big, 1) <= max(1, (big - 65536) // (count * 40 * 16 * 128 * 4))
+
+
+def test_sgmv_shrink_groups_parts_of_every_group():
+    """lorax_sgmv_shrink_groups_parts_of: at least one part of at least eight stages each, at most eight of them, their fp32 sums
+    in the first 8 MiB (less the counters), and no part for a group without tiles."""
+    import random
+
+    average, each = (getattr(_native.lib(), "lorax_sgmv_shrink_groups_parts" + suffix) for suffix in ("", "_of"))
+    rng, big, seen = random.Random(5), 8 * 1024 * 1024, set()
+    for _ in range(2000):
+        n, h_in = rng.randint(2, 16), 128 * rng.choice([3, 16, 32, 64, 67, 112, 224])
+        shapes = [(rng.choice([8, 16, 24, 32, 64]), rng.randint(1, 2), rng.choice([0, 1, 9, 40, 90, 170]), rng.choice([16, 32]))
+                  for _ in range(n)]
+        made = [_shrink_groups(r, count, 1, height, tiles) for r, count, tiles, height in shapes]
+        groups = (_native.SgmvShrinkGroup * n)(*[g[0] for g, _ in made])
+        parts = (ctypes.c_int32 * n)(*[-1] * n)
+        args = (groups, n, P, 12000, h_in, 0, 0, P, big, 1)
+        k = average(*args)
+        assert each(*args, parts) == k
+        if k == 0:
+            assert list(parts) == [-1] * n
+            continue
+        sums = 0
+        for (r, count, tiles, height), got in zip(shapes, parts):
+            assert got == 0 if tiles == 0 else 1 <= got <= max(1, min(8, h_in // 128 // 8))
+            sums += got * tiles * height * ((r * count + 15) // 16 * 16) * 4 if got > 1 else 0
+        assert sums <= big - 65536 and (k > 1 or max(parts) == 1)
+        seen.add((k > 1, 1 in parts, len(set(parts) - {0}) > 1))
+    assert (True, True, True) in seen and (True, False, True) in seen
 
 
 def test_sgmv_lora_multi_validation():

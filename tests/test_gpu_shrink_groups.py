@@ -1,6 +1,7 @@
 """lorax_sgmv_shrink_groups: the shrinks of several rank groups over one x in one launch, against fp64 and against one
 launch per group.  Sizes at the edges: one-row tiles, 16- and 32-row tiles, every stacked rank, groups without rows, more
-tiles than CUs; and launches that cut the hidden dimension into parts, of stages that do not divide among them.  ROUTES says
+tiles than CUs; and launches that cut the hidden dimension into parts, of stages that do not divide among them, of some
+groups further than of others and of some not at all.  ROUTES says
 what each case has to run as, so that none compares the calls per group with themselves."""
 
 import pytest
@@ -33,18 +34,23 @@ CASES = {
     "a group without rows": (512, [(16, 2, [300]), (8, 1, [0]), (32, 1, [250])]),
     "many tiles": (256, [(64, 2, [1500]), (128, 1, [33] * 60)]),
     "32-row tiles": (256, [(128, 1, [4096]), (64, 1, [64])]),
-    # 67 stages in 6, 7, 5 and 3 parts
+    # 67 stages
     "parts, four ranks": (128 * 67, [(8, 3, [100, 1, 33]), (16, 3, [17, 200]), (32, 3, [90, 16]), (64, 2, [130])]),
     "parts, a group without rows": (128 * 67, [(16, 2, [300]), (8, 1, [0]), (32, 1, [250])]),
     "parts, every stacked rank": (128 * 67, [(8, 1, [700]), (16, 1, [33] * 9), (24, 1, [71]), (40, 2, [9]), (48, 2, [17]),
                                              (56, 2, [31]), (128, 1, [65])]),
     "parts, 32-row tiles": (128 * 67, [(128, 1, [4096]), (64, 1, [64])]),
+    "parts, some groups whole": (128 * 67, [(32, 1, [820]), (16, 1, [190]), (64, 1, [730]), (32, 2, [730]), (8, 2, [190])]),
+    "parts, the first group whole": (128 * 67, [(16, 1, [190]), (8, 1, [0]), (32, 1, [820]), (64, 1, [730]), (32, 2, [730]),
+                                                (8, 2, [190])]),
 }
-# (parts of the hidden dimension, heights of the groups' tiles)
+# (parts of every group's hidden dimension, heights of the groups' tiles)
 ROUTES = {
-    "four ranks": (1, {16}), "every stacked rank": (1, {16}), "an odd number of stages": (1, {16}),
-    "a group without rows": (1, {16}), "many tiles": (1, {16}), "32-row tiles": (1, {16, 32}), "parts, four ranks": (6, {16}),
-    "parts, a group without rows": (7, {16}), "parts, every stacked rank": (5, {16}), "parts, 32-row tiles": (3, {16, 32}),
+    "four ranks": ([1, 1, 1, 1], {16}), "every stacked rank": ([1] * 8, {16}), "an odd number of stages": ([1, 1], {16}),
+    "a group without rows": ([1, 0, 1], {16}), "many tiles": ([1, 1], {16}), "32-row tiles": ([1, 1], {16, 32}),
+    "parts, four ranks": ([6, 6, 6, 6], {16}), "parts, a group without rows": ([7, 0, 7], {16}),
+    "parts, every stacked rank": ([4, 4, 5, 8, 8, 8, 8], {16}), "parts, 32-row tiles": ([3, 2], {16, 32}),
+    "parts, some groups whole": ([2, 1, 3, 3, 1], {16}), "parts, the first group whole": ([1, 0, 2, 3, 3, 1], {16}),
 }
 
 
@@ -68,7 +74,7 @@ def test_groups_in_one_launch(case, accumulate, dtype):
     shrinks = [(list(g[5].unbind(0)), g[1], g[2], g[3], g[4]) for g in groups]
     parts, heights = ROUTES[case]
     assert {g[4].tile_rows for g in groups} == heights
-    assert _native.sgmv_shrink_groups_parts(shrinks, x, tmp, 1, accumulate) == parts
+    assert _native.sgmv_shrink_groups_parts_of(shrinks, x, tmp, 1, accumulate) == parts
 
     def run(apart):
         vs = [g[5].clone() for g in groups]
