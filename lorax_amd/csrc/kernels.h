@@ -45,8 +45,9 @@ struct BgmvBatchOf {
   int sub_hi[P];
 };
 using BgmvBatch = BgmvBatchOf<kMaxBgmvProblems>;
-// A launch of a few problems passes a batch of this many: the runtime writes a launch's arguments into device memory over
-// the bus, 2.75 us a launch at 128 bytes, 2.9 at 500 and 3.7 to 3.9 at the 2 KB of a full batch.
+// A launch of a few problems can pass a batch of this many, 368 instead of 1472 bytes: the runtime writes a launch's arguments
+// into device memory over the bus (a kernel of a few instructions launched back to back, by the bytes of its arguments: 2.75 us a launch at 128,
+// 2.9 at 500, 3.7 to 3.9 at 2 KB).
 constexpr int kFewProblems = 4;
 static_assert(kFewProblems >= kMaxFusedBgmvProblems, "the single-launch kernels only exist for few problems");
 template <int P>
