@@ -203,7 +203,9 @@ __global__ __launch_bounds__(kExpTThreads, MIXED ? (KS == 2 ? 4 : 3) : 1) void s
   // one problem's panel groups, a batch whose segments differ waited for the XCD with the most rows: 28672 columns x
   // 2062 rows of ranks 8 to 64 111 us, dealt out 68; 786 rows of rank 64 42 and 32 us.)  A panel group has one XCD,
   // where all pieces of a segment find its panel of B^T in the L2, wherever the number of groups is a multiple of the
-  // XCDs; an XCD then takes adjacent groups (15136 rows: 624 -> 615 us for a step of the large prefill).
+  // XCDs; an XCD then takes adjacent groups (15136 rows: 624 -> 615 us for a step of the large prefill).  Elsewhere every XCD
+  // fetches every panel, in about the same time: 27 groups x 9126 rows of rank 64 162 -> 185 MB, 61.8 -> 59.1 us, 27 x 4096 of
+  // rank 128 71 -> 91 MB, 31.4 -> 32.4 us; with 56 groups (10658 rows, rank 64) 433 -> 377 MB.
   int vid = static_cast<int>(blockIdx.x);
   int prob = 0;
   if (count > 1) {  // lane i looks at problem i's range: one trip to the kernel arguments
